@@ -51,6 +51,7 @@ MARCH_KINDS = {
     9: "persistent chunked march, 56 columns, 64-byte-aligned stores, loads two rows ahead",
     10: "persistent chunked march, 56 columns, 64-byte-aligned stores",
     11: _ALIGNED + ", loads three rows ahead",
+    12: "band tiles by grid size, metrics by row, Flather faces included",
 }
 # rocprofv3 summaries holding "[label] traffic_bytes_per_launch:" lines
 PROFILE_TRAFFIC = (ROOT / "profiles" / "fused_step_4096_counters.md",

@@ -164,8 +164,11 @@ NEMO_API double nemo_hip_fused_kernel_ms(void);
 /* Kernel shape of the fused form: -1 = 64x4-cell tiles with an LDS ssh
  * tile; 0 .. nemo_hip_fused_variant_count()-1 = row-march shapes (block
  * width x rows per band). All shapes compute bitwise the same result;
- * default 31 (4-row bands of 56 columns with the loads issued two rows
- * ahead, the fastest measured at 4096^2).
+ * default 31, the band form: it evaluates every face once, has the Flather
+ * faces in the same launch, picks the band height by the size of the grid
+ * and, in calls of two or more steps on a grid whose metrics do not vary
+ * along a row, reads them as one record a row (checked on the device arrays
+ * in every such call).
  * Applies to the next launches of every context. */
 NEMO_API int nemo_hip_fused_variant_count(void);
 NEMO_API void nemo_hip_set_fused_variant(int variant);
@@ -179,7 +182,8 @@ NEMO_API int nemo_hip_fused_variant(void);
  * ahead, compiled for at least 2 / 3 waves per SIMD, 9 / 10 = the persistent
  * chunked 56-column march with / without the loads two rows ahead (rows = 0:
  * one chunk of rows per wavefront the GPU holds at once, set at launch),
- * 11 = the 56-column march with its loads issued three rows ahead. */
+ * 11 = the 56-column march with its loads issued three rows ahead, 12 = the
+ * band form (rows = 0: by the size of the grid). */
 NEMO_API void nemo_hip_fused_variant_shape(int variant, int *block_width,
                                            int *rows, int *prefetch);
 /* Name of the kernel a variant launches, as profilers report it. */

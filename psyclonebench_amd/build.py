@@ -41,7 +41,7 @@ HIPCC_FLAGS = [
     "-Wno-unused-command-line-argument",
 ]
 
-HIP_SOURCES = ["nemo_step.hip", "nemo_march.hip", "nemo_psy.cpp", "nemo_mixed.hip",
+HIP_SOURCES = ["nemo_step.hip", "nemo_march.hip", "nemo_band.hip", "nemo_psy.cpp", "nemo_mixed.hip",
                "nemo_mixed_api.cpp", "nemo_ensemble.hip", "nemo_ensemble_api.cpp",
                "nemo_closure.hip", "nemo_closure_api.cpp", "nemo_noalloc.hip"]
 

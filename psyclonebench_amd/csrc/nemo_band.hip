@@ -1,0 +1,201 @@
+// Launcher of the band tile (nemo_band.h) for one FP64 domain, and the table
+// of metrics by row.
+#include <algorithm>
+
+#include "nemo_band.h"
+#include "nemo_hip_common.h"
+
+namespace nemo {
+namespace {
+
+using band::Flather;
+
+template <typename T, bool ROWM, int R, int OW, int PF, bool NEXT, bool STREAM>
+__global__ __launch_bounds__(64) void k_band(typename band::Types<T>::In f,
+                                             const T *__restrict__ tab, StepScalars<T> p,
+                                             typename band::Types<T>::Out o, Flather<T> fl,
+                                             int W, Bounds b, int nstrip,
+                                             const double *__restrict__ tide_tab, int tide_k,
+                                             double tide_val)
+{
+    const int logical = wave::xcd_tile((int)blockIdx.x, (int)gridDim.x);
+    const int bd = logical / nstrip, strip = logical - bd * nstrip;
+    const int jlo = b.ys - 1 + bd * R, jhi = min(jlo + R, b.ye + 2);
+    const double tide = tide_tab ? tide_tab[tide_k] : tide_val;
+    if constexpr (sizeof(T) == 8)
+        band::tile<T, ROWM, R, OW, PF, NEXT, STREAM>(f, tab, p, o, fl, W, 0u, b, strip, jlo, jhi,
+                                                     tide);
+    else
+        band::tile<T, ROWM, R, OW, PF, NEXT, STREAM>(f, tab, p, o, fl, W, 0u, b, strip, jlo, jhi,
+                                                     wave::split(tide));
+}
+
+template <typename T>
+struct Args {
+    hipStream_t s;
+    const typename band::Types<T>::In &f;
+    const T *tab;
+    const StepScalars<T> &p;
+    const typename band::Types<T>::Out &o;
+    const Flather<T> &fl;
+    int W;
+    const Bounds &b;
+    const double *tide_tab;
+    int tide_k;
+    double tide_val;
+};
+
+template <typename T, bool ROWM, int R, int OW, int PF, bool NEXT, bool STREAM>
+void launch(const Args<T> &a)
+{
+    const int nstrip = wave::strips(a.b, OW);
+    const dim3 grid((unsigned)(nstrip * wave::bands(a.b, R)));
+    k_band<T, ROWM, R, OW, PF, NEXT, STREAM><<<grid, dim3(64), 0, a.s>>>(
+        a.f, a.tab, a.p, a.o, a.fl, a.W, a.b, nstrip, a.tide_tab, a.tide_k, a.tide_val);
+    NEMO_LAUNCH_CHECK();
+}
+
+// The 13 arrays of the row table, in this order.
+constexpr int kRowArrays = 13;
+template <typename T>
+struct RowSource {
+    const T *a[kRowArrays];
+};
+template <typename T, typename In>
+RowSource<T> row_source(const In &f)
+{
+    return RowSource<T>{{f.area_t, f.area_u, f.area_v, f.dx_u, f.dx_v, f.dx_t, f.dy_u, f.dy_v,
+                         f.dy_t, f.fcor_u, f.fcor_v, f.ssha_u, f.ssha_v}};
+}
+
+// A divisor that uniform_quotient takes (FP64).
+__device__ bool divisor_ok(double d)
+{
+    return isfinite(d) && d != 0.0 && abs(__builtin_amdgcn_frexp_exp(d)) <= kDivisorExp;
+}
+__device__ double reciprocal(double d) { return band::refined_reciprocal(d); }
+
+// One workgroup per row: writes the row's record from its first column and
+// stores `mark` to *bad when another column of the row holds other bits or a
+// divisor is out of range. Reads 13 arrays once at most; a grid whose metrics
+// vary is recognised in the first 256 columns of each row.
+template <typename T>
+__global__ __launch_bounds__(256) void k_row_metrics(RowSource<T> src, int W, unsigned base,
+                                                     int ncol, T *__restrict__ tab, int *bad,
+                                                     int mark)
+{
+    using B = std::conditional_t<sizeof(T) == 8, unsigned long long, unsigned>;
+    const int j = (int)blockIdx.x, nrow = (int)gridDim.x;
+    const unsigned row = base + (unsigned)(j * W);
+    B first[kRowArrays];
+#pragma unroll
+    for (int q = 0; q < kRowArrays; q++) first[q] = __builtin_bit_cast(B, ld32(src.a[q], row));
+    bool differs = false;
+    for (int x = (int)threadIdx.x; x - (int)threadIdx.x < ncol; x += 256) {
+        const unsigned c = row + (unsigned)min(x, ncol - 1);
+#pragma unroll
+        for (int q = 0; q < kRowArrays; q++)
+            differs |= __builtin_bit_cast(B, ld32(src.a[q], c)) != first[q];
+        differs = __syncthreads_or(differs);  // the workgroup's answer in every thread
+        if (differs) break;
+    }
+    if (threadIdx.x != 0) return;
+    T v[kRowArrays];
+#pragma unroll
+    for (int q = 0; q < kRowArrays; q++) v[q] = __builtin_bit_cast(T, first[q]);
+    const T e2u_n = ld32(src.a[6], base + (unsigned)(min(j + 1, nrow - 1) * W));
+    T *r = tab + (size_t)j * band::ROW_WIDTH;
+    using namespace band;
+    r[M_AT] = v[0];
+    r[M_ARU] = v[1];
+    r[M_ARV] = v[2];
+    r[M_E1U] = v[3];
+    r[M_E1V] = v[4];
+    r[M_E1V2] = v[4] + v[4];
+    r[M_E1T] = v[5];
+    r[M_E2U] = v[6];
+    r[M_E2US] = v[6] + e2u_n;
+    r[M_E2V] = v[7];
+    r[M_E2T] = v[8];
+    r[M_FCU] = v[9];
+    r[M_FCV] = v[10];
+    r[M_SAU] = v[11];
+    r[M_SAV] = v[12];
+    auto divisor = [&](int slot, T d) {
+        differs |= !divisor_ok(d);
+        r[slot] = reciprocal(d);
+    };
+    divisor(R_AT, v[0]);
+    divisor(R_ARU, v[1]);
+    divisor(R_ARV, v[2]);
+    divisor(R_E1V2, v[4] + v[4]);
+    divisor(R_E1T, v[5]);
+    divisor(R_E2US, v[6] + e2u_n);
+    divisor(R_E2T, v[8]);
+    if (differs) *bad = mark;
+}
+
+template <typename T, typename In>
+void row_metrics(hipStream_t s, const In &f, int W, unsigned base, const Bounds &b, T *tab,
+                 int *bad, int mark)
+{
+    k_row_metrics<T><<<dim3((unsigned)(b.ye + 2)), dim3(256), 0, s>>>(
+        row_source<T>(f), W, base, b.xe + 2, tab, bad, mark);
+    NEMO_LAUNCH_CHECK();
+}
+
+// Tiles of a launch with R-row bands of ow columns.
+long tiles(const Bounds &b, int rows, int ow)
+{
+    return (long)wave::strips(b, ow) * wave::bands(b, rows);
+}
+
+// Band height by the number of tiles. A wavefront takes about 2 us a row when
+// it has a SIMD to itself, so a grid that does not fill the chip wants
+// one-row bands, although each also evaluates the faces of the row before it
+// (565 against 390 instructions a row); a large one wants the fewest halo
+// rows, in 56-column strips (64-byte-aligned stores). Measured, us a step
+// with one / two / four or eight rows:
+//   FP64 by row  128^2 4.2 / 5.6 / 10;  384^2 7.1 / 7.5 / 11;  512^2 10.1 /
+//                9.7 / 13.7;  1400^2 46 / 39 / 46;  2048^2 136 / 109 / 106;
+//                4096^2 540 / 430 / 406
+//   FP64         400^2 8.1 / 9.3 / 13.6;  700^2 20.3 / 22 / 23.5;  2048^2 207
+//                / 193 / 195;  4096^2 809 / 751 / 741
+constexpr long kOneRowTilesF64 = 12000, kOneRowTilesByRowF64 = 3500;
+constexpr long kTwoRowTilesF64 = 48000, kTwoRowTilesByRowF64 = 24000;
+
+}  // namespace
+
+size_t row_table_values(const Bounds &b) { return (size_t)(b.ye + 2) * band::ROW_WIDTH; }
+
+void launch_row_metrics(hipStream_t s, const StepIn<double> &f, int W, unsigned base,
+                        const Bounds &b, double *tab, int *bad, int mark)
+{
+    row_metrics<double>(s, f, W, base, b, tab, bad, mark);
+}
+
+void launch_band_f64(hipStream_t s, const StepIn<double> &f, const double *tab,
+                     const StepScalars<double> &p, const StepOut<double> &o,
+                     const double *u_prev, const double *v_prev, int W, const Bounds &b,
+                     const double *tide_tab, int tide_k, double tide_val)
+{
+    const Flather<double> fl{u_prev, v_prev, nullptr, nullptr, 1};
+    const Args<double> a{s, f, tab, p, o, fl, W, b, tide_tab, tide_k, tide_val};
+    if (tab) {
+        if (tiles(b, 1, 61) <= kOneRowTilesByRowF64)
+            launch<double, true, 1, 61, 0, true, false>(a);
+        else if (tiles(b, 2, 61) <= kTwoRowTilesByRowF64)
+            launch<double, true, 2, 61, 0, true, false>(a);
+        else
+            launch<double, true, 8, 56, 0, true, true>(a);
+    } else {
+        if (tiles(b, 1, 61) <= kOneRowTilesF64)
+            launch<double, false, 1, 61, 0, true, false>(a);
+        else if (tiles(b, 2, 61) <= kTwoRowTilesF64)
+            launch<double, false, 2, 61, 0, true, false>(a);
+        else
+            launch<double, false, 4, 56, 1, true, true>(a);
+    }
+}
+
+}  // namespace nemo

@@ -575,7 +575,9 @@ void launch_wave_t(hipStream_t s, const StepIn<double> &f,
 // its loads issued two rows ahead, compiled for >= 2 / 3 wavefronts per SIMD,
 // 9 / 10 the persistent chunked 56-column march with / without the loads two
 // rows ahead (rows 0: the chunk height is set at launch from the occupancy),
-// 11 the 56-column march with its loads issued three rows ahead
+// 11 the 56-column march with its loads issued three rows ahead,
+// 12 the band form (nemo_band.hip, launched by launch_band_f64; rows 0: by
+// the size of the grid)
 struct MarchShape {
     int mx, rows, prefetch;
 };
@@ -603,7 +605,7 @@ static const MarchShape kShapes[] = {
     {64, 64, 2},  {64, 128, 2}, {64, 32, 3},  {64, 64, 3},  {64, 32, 4},
     {64, 64, 4},  {64, 16, 5},  {64, 32, 5},  {64, 8, 5},   {64, 16, 6},
     {64, 32, 6},  {64, 4, 5},   {64, 8, 6},   {64, 4, 6},   {64, 2, 5},
-    {64, 6, 5},   {64, 4, 7},   {64, 6, 7},   {64, 8, 7},   {64, 12, 7},
+    {64, 6, 5},   {64, 0, 12},  {64, 6, 7},   {64, 8, 7},   {64, 12, 7},
     {64, 4, 8},   {64, 8, 8},   {64, 32, 7},  {64, 64, 7},  {64, 0, 9},
     {64, 0, 9},   {64, 0, 10},  {64, 4, 11},  {64, 6, 11},  {64, 8, 11},
 };
@@ -625,7 +627,7 @@ static const char *const kNames[] = {
     "k_fused_wave_a<16, 48>",        "k_fused_wave_a<32, 48>",
     "k_fused_wave_a<4, 56>",         "k_fused_wave_a<8, 48>",
     "k_fused_wave_a<4, 48>",         "k_fused_wave_a<2, 56>",
-    "k_fused_wave_a<6, 56>",         "k_fused_wave_p<4, 56, 2, 1>",
+    "k_fused_wave_a<6, 56>",         "k_band",
     "k_fused_wave_p<6, 56, 2, 1>",      "k_fused_wave_p<8, 56, 2, 1>",
     "k_fused_wave_p<12, 56, 2, 1>",     "k_fused_wave_p<4, 56, 3, 1>",
     "k_fused_wave_p<8, 56, 3, 1>",      "k_fused_wave_p<32, 56, 2, 1>",
@@ -715,9 +717,6 @@ void launch_fused_march(hipStream_t s, int variant, const StepIn<double> &f,
         break;
     case 30:
         launch_wave_aligned_t<6, 56>(s, f, p, o, W, b, tide_tab, tide_k, tide_val);
-        break;
-    case 31:
-        launch_wave_prefetch_t<4, 56, 2>(s, f, p, o, W, b, tide_tab, tide_k, tide_val);
         break;
     case 32:
         launch_wave_prefetch_t<6, 56, 2>(s, f, p, o, W, b, tide_tab, tide_k, tide_val);

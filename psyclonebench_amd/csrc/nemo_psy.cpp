@@ -33,10 +33,10 @@ namespace {
 double g_amp_tide = 0.2;
 double g_omega_tide = 2.0 * 3.14159 / (12.42 * 3600.0);
 int g_mode = 0;
-// -1: tile kernel; >= 0: row-march variant. The default is the fastest
-// measured at 4096^2: 4-row bands of 56-column, 64-byte-aligned strips with
-// the loads issued two rows ahead.
-int g_fused_variant = 31;
+// -1: tile kernel; >= 0: row-march variant; the default runs the band form
+// (nemo_band.hip), which picks its tiles by the grid.
+constexpr int kDefaultVariant = 31;
+int g_fused_variant = kDefaultVariant;
 bool g_kernel_timing = false;
 double g_fused_ms = -1.0;
 
@@ -67,8 +67,14 @@ struct Context {
     double *d_tide = nullptr;
     double *h_tide = nullptr;  // pinned
     int tide_cap = 0;
-    // n, parity, variant, hook key (0: plain steps)
-    std::map<std::tuple<int, int, int, unsigned long long>, hipGraphExec_t> graphs;
+    // fused: the table of metrics by row, rebuilt from the device arrays by
+    // every call that uses it; row_bad (pinned) holds the mark of the last
+    // call whose metrics vary along a row
+    double *row_tab = nullptr;
+    int *row_bad = nullptr;
+    int row_mark = 0;
+    // n, parity, variant, metrics by row, hook key (0: plain steps)
+    std::map<std::tuple<int, int, int, bool, unsigned long long>, hipGraphExec_t> graphs;
     void **slots[A_COUNT] = {};  // the caller's slots of the last call
     std::vector<hipEvent_t> ev;
 
@@ -126,6 +132,8 @@ struct Context {
         if (spare_sv) (void)hipFree(spare_sv);
         if (d_tide) (void)hipFree(d_tide);
         if (h_tide) (void)hipHostFree(h_tide);
+        if (row_tab) (void)hipFree(row_tab);
+        if (row_bad) (void)hipHostFree(row_bad);
         fl_u.release();
         fl_v.release();
     }
@@ -223,26 +231,51 @@ void step_unfused(Context &C, int istep, hipStream_t s)
 }
 
 // ---- one step, fused: state set `par` -> set 1-par -----------------------
+// by_row: the context's table of metrics by row stands for the arrays.
 void launch_fused_pair(Context &C, int par, hipStream_t s, const double *tide_tab,
-                       int tide_k, double tide_val, hipEvent_t e0 = nullptr,
+                       int tide_k, double tide_val, bool by_row, hipEvent_t e0 = nullptr,
                        hipEvent_t e1 = nullptr)
 {
     const int q = 1 - par;
     const StepOut<double> o{C.T(q), C.U(q), C.V(q), C.SU(q), C.SV(q)};
     const Bounds bd{C.G.xs, C.G.xe, C.G.ys, C.G.ye};
+    // the previous step's velocities: set `par` once the sets are paired; on
+    // the first step the after arrays themselves, as the reference has them
+    const int prev = C.paired ? par : q;
     if (e0) NEMO_HIP_CHECK(hipEventRecord(e0, s));
-    if (g_fused_variant < 0)
+    if (g_fused_variant == kDefaultVariant)
+        launch_band_f64(s, C.inputs(par), by_row ? C.row_tab : nullptr, C.scalars(), o,
+                        C.U(prev), C.V(prev), C.G.W, bd, tide_tab, tide_k, tide_val);
+    else if (g_fused_variant < 0)
         launch_fused_step(s, C.inputs(par), C.scalars(), o, C.G.W, bd, tide_tab,
                           tide_k, tide_val);
     else
         launch_fused_march(s, g_fused_variant, C.inputs(par), C.scalars(), o,
                            C.G.W, bd, tide_tab, tide_k, tide_val);
     if (e1) NEMO_HIP_CHECK(hipEventRecord(e1, s));
-    // the previous step's velocities: set `par` once the sets are paired; on
-    // the first step the after arrays themselves, as the reference has them
-    const int prev = C.paired ? par : q;
-    launch_flather(s, C.fl_u.view(), C.fl_v.view(), C.U(q), C.V(q), C.U(prev), C.V(prev),
-                   C.SU(par), C.SV(par));
+    if (g_fused_variant != kDefaultVariant)  // the band form's tiles do these
+        launch_flather(s, C.fl_u.view(), C.fl_v.view(), C.U(q), C.V(q), C.U(prev), C.V(prev),
+                       C.SU(par), C.SV(par));
+}
+
+// Builds the table of metrics by row and says whether the grid has them: the
+// metrics do not vary along a row and every divisor of the step is in the
+// range its kernels take. Nothing is carried over from an earlier call: the
+// caller may have written to the arrays through their handles. Ends with the
+// stream idle.
+bool metrics_by_row(Context &C, hipStream_t s)
+{
+    const Bounds bd{C.G.xs, C.G.xe, C.G.ys, C.G.ye};
+    const int e_fric = std::ilogb(C.scalars().fric);  // INT_MAX / INT_MIN: inf, NaN, 0
+    if (e_fric < -kDivisorExp || e_fric > kDivisorExp) return false;
+    if (!C.row_tab) {
+        C.row_tab = dev_alloc<double>(row_table_values(bd));
+        NEMO_HIP_CHECK(hipHostMalloc((void **)&C.row_bad, sizeof(int), hipHostMallocDefault));
+        *C.row_bad = 0;
+    }
+    launch_row_metrics(s, C.inputs(0), C.G.W, 0u, bd, C.row_tab, C.row_bad, ++C.row_mark);
+    NEMO_HIP_CHECK(hipStreamSynchronize(s));
+    return *static_cast<volatile int *>(C.row_bad) != C.row_mark;
 }
 
 void run_hook(const Context &C, const StepHook *hook, hipStream_t s)
@@ -255,7 +288,7 @@ void run_hook(const Context &C, const StepHook *hook, hipStream_t s)
 
 void step_fused(Context &C, int istep, hipStream_t s, const StepHook *hook = nullptr)
 {
-    launch_fused_pair(C, C.parity, s, nullptr, 0, tide_at(istep, C.P.rdt));
+    launch_fused_pair(C, C.parity, s, nullptr, 0, tide_at(istep, C.P.rdt), false);
     C.parity = 1 - C.parity;
     run_hook(C, hook, s);
     if (!C.paired) {
@@ -286,17 +319,17 @@ void ensure_tide_table(Context &C, int n)
     C.graphs.clear();
 }
 
-hipGraphExec_t fused_graph(Context &C, int n, int par, hipStream_t s,
+hipGraphExec_t fused_graph(Context &C, int n, int par, bool by_row, hipStream_t s,
                            const StepHook *hook)
 {
-    auto key = std::make_tuple(n, par, g_fused_variant, hook ? hook->key : 0ull);
+    auto key = std::make_tuple(n, par, g_fused_variant, by_row, hook ? hook->key : 0ull);
     auto it = C.graphs.find(key);
     if (it != C.graphs.end()) return it->second;
     hipGraph_t graph;
     const int parity = C.parity;
     NEMO_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
     for (int k = 0; k < n; k++) {
-        launch_fused_pair(C, (par + k) & 1, s, C.d_tide, k, 0.0);
+        launch_fused_pair(C, (par + k) & 1, s, C.d_tide, k, 0.0, by_row);
         C.parity = (par + k + 1) & 1;  // the set this step wrote, for the hook
         run_hook(C, hook, s);
     }
@@ -325,6 +358,10 @@ void run_steps(Context &C, int nsteps, int istep, hipStream_t s,
         if (nsteps == 0) return;
     }
     ensure_tide_table(C, nsteps);
+    // The table costs one pass over 13 arrays and saves about that much a
+    // step, so a single step goes without (20 steps at 4096^2: 0.3 of 8.3 ms).
+    bool by_row = false;
+    if (g_fused_variant == kDefaultVariant && nsteps > 1) by_row = metrics_by_row(C, s);
     NEMO_HIP_CHECK(hipStreamSynchronize(s));  // h_tide may still be in flight
     for (int k = 0; k < nsteps; k++) C.h_tide[k] = tide_at(istep + k, C.P.rdt);
     NEMO_HIP_CHECK(hipMemcpyAsync(C.d_tide, C.h_tide, (size_t)nsteps * sizeof(double),
@@ -339,7 +376,7 @@ void run_steps(Context &C, int nsteps, int istep, hipStream_t s,
         }
         const int parity = C.parity;
         for (int k = 0; k < nsteps; k++) {
-            launch_fused_pair(C, (parity + k) & 1, s, C.d_tide, k, 0.0, C.ev[2 * k],
+            launch_fused_pair(C, (parity + k) & 1, s, C.d_tide, k, 0.0, by_row, C.ev[2 * k],
                               C.ev[2 * k + 1]);
             C.parity = (parity + k + 1) & 1;
             run_hook(C, hook, s);
@@ -354,7 +391,7 @@ void run_steps(Context &C, int nsteps, int istep, hipStream_t s,
         }
         g_fused_ms = sum / nsteps;
     } else {
-        NEMO_HIP_CHECK(hipGraphLaunch(fused_graph(C, nsteps, C.parity, s, hook), s));
+        NEMO_HIP_CHECK(hipGraphLaunch(fused_graph(C, nsteps, C.parity, by_row, s, hook), s));
     }
     C.parity = (C.parity + nsteps) & 1;
 }

@@ -96,6 +96,24 @@ int march_variant_count();
 void march_variant_shape(int variant, int *mx, int *rows, int *prefetch);
 const char *march_variant_kernel(int variant);
 
+// --- band form (nemo_band.hip): the library's default ----------------------
+// Metrics by row: on a grid where the 13 metric, area, Coriolis and after-ssh
+// face arrays do not vary along a row, a table of one record a row stands for
+// them. launch_row_metrics builds the table (row_table_values() values) from
+// the arrays whose (0,0) is at element `base` and stores `mark` to *bad
+// (memory that the device can write) when they do vary or a divisor is out of
+// the table's range (2^+-kDivisorExp).
+constexpr int kDivisorExp = 100;
+size_t row_table_values(const Bounds &b);
+void launch_row_metrics(hipStream_t s, const StepIn<double> &f, int W, unsigned base,
+                        const Bounds &b, double *tab, int *bad, int mark);
+// One fused step with its Flather faces in one launch: the same results as
+// launch_fused_march followed by launch_flather. tab: the row table, or null
+// (any metrics). u_prev / v_prev as in launch_flather.
+void launch_band_f64(hipStream_t s, const StepIn<double> &f, const double *tab,
+                     const StepScalars<double> &p, const StepOut<double> &o,
+                     const double *u_prev, const double *v_prev, int W, const Bounds &b,
+                     const double *tide_tab, int tide_k, double tide_val);
 // Small helpers.
 void launch_fill_int(hipStream_t s, int *p, int n, int value);
 
