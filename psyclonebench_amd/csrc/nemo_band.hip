@@ -1,5 +1,5 @@
-// Launcher of the band tile (nemo_band.h) for one FP64 domain, and the table
-// of metrics by row.
+// Launchers of the band tile (nemo_band.h) for one FP64 domain, into the other
+// state set or in place, and the table of metrics by row.
 #include <algorithm>
 
 #include "nemo_band.h"
@@ -144,6 +144,41 @@ void row_metrics(hipStream_t s, const In &f, int W, unsigned base, const Bounds 
     NEMO_LAUNCH_CHECK();
 }
 
+// In-place step, second half: now <- after over the reference's copy region
+// (time_step.cpp:115-122), and the face ssh from the new cell ssh (which the
+// copy region covers, so the after field stands for the now field).
+__global__ __launch_bounds__(256) void k_finish(double *__restrict__ un,
+                                                const double *__restrict__ ua,
+                                                double *__restrict__ vn,
+                                                const double *__restrict__ va,
+                                                double *__restrict__ sshn_t,
+                                                const double *__restrict__ ssha_t,
+                                                double *__restrict__ sshn_u,
+                                                double *__restrict__ sshn_v,
+                                                const int *__restrict__ tm,
+                                                const double *__restrict__ area_t,
+                                                const double *__restrict__ area_u,
+                                                const double *__restrict__ area_v, int W,
+                                                Bounds b)
+{
+    const int i = b.xs - 1 + (int)(blockIdx.x * 64 + threadIdx.x);
+    const int j = b.ys - 1 + (int)(blockIdx.y * 4 + threadIdx.y);
+    if (i > b.xe + 1 || j > b.ye) return;
+    const int c = j * W + i;
+    un[c] = ua[c];
+    vn[c] = va[c];
+    const double s = ssha_t[c];
+    sshn_t[c] = s;
+    if (i < b.xs || j < b.ys || i > b.xe) return;
+    double v;
+    if (i <= b.xe - 1 &&
+        next_ssh_pt(s, ssha_t[c + 1], area_t[c], area_t[c + 1], area_u[c], tm[c], tm[c + 1], &v))
+        sshn_u[c] = v;
+    if (j <= b.ye - 1 &&
+        next_ssh_pt(s, ssha_t[c + W], area_t[c], area_t[c + W], area_v[c], tm[c], tm[c + W], &v))
+        sshn_v[c] = v;
+}
+
 // Tiles of a launch with R-row bands of ow columns.
 long tiles(const Bounds &b, int rows, int ow)
 {
@@ -196,6 +231,30 @@ void launch_band_f64(hipStream_t s, const StepIn<double> &f, const double *tab,
         else
             launch<double, false, 4, 56, 1, true, true>(a);
     }
+}
+
+void launch_band_inplace(hipStream_t s, const StepIn<double> &f, const StepScalars<double> &p,
+                         const StepOut<double> &o, int W, const Bounds &b, double tide)
+{
+    // the after arrays hold the previous step's velocities until their faces
+    // are written
+    const Flather<double> fl{o.u, o.v, nullptr, nullptr, 1};
+    const Args<double> a{s, f, nullptr, p, o, fl, W, b, nullptr, 0, tide};
+    if (tiles(b, 1, 61) <= kOneRowTilesF64)
+        launch<double, false, 1, 61, 0, false, false>(a);
+    else
+        launch<double, false, 2, 61, 0, false, false>(a);
+}
+
+void launch_finish(hipStream_t s, double *un, const double *ua, double *vn, const double *va,
+                   double *sshn_t, const double *ssha_t, double *sshn_u, double *sshn_v,
+                   const int *tmask, const double *area_t, const double *area_u,
+                   const double *area_v, int W, const Bounds &b)
+{
+    const dim3 grid((unsigned)((b.xe - b.xs + 3 + 63) / 64), (unsigned)((b.ye - b.ys + 2 + 3) / 4));
+    k_finish<<<grid, dim3(64, 4), 0, s>>>(un, ua, vn, va, sshn_t, ssha_t, sshn_u, sshn_v, tmask,
+                                          area_t, area_u, area_v, W, b);
+    NEMO_LAUNCH_CHECK();
 }
 
 }  // namespace nemo

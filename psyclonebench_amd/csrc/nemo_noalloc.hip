@@ -4,17 +4,20 @@
 // (manual_versions/psykal_cpp/time_step.cpp:53-136: every sweep in order, in
 // place, now <- after copied over the reference's copy region) on 25 device
 // arrays that the caller owns, for callers that cannot allocate device
-// memory (code under HIP graph capture, tight serving loops). It runs the
-// unfused kernels of nemo_step.hip. Two things the allocating forms keep in
-// buffers of their own are arranged differently:
+// memory (code under HIP graph capture, tight serving loops). Three launches:
+// the Coriolis factors, the band tile of nemo_band.h over the after arrays
+// (every sweep up to bc_flather), and the copies with next_sshu/v. 511 x 383:
+// 18.7 us a step, against 222 us with one kernel per sweep, of which 187 us
+// were a Flather kernel that walked each row and column with one thread. Two
+// things the allocating forms keep in buffers of their own are arranged
+// differently:
 //
 //  * the Coriolis factors (2*omega)*sin(gphi*d2r) are evaluated on the
 //    device into `scratch` at every call (the allocating forms evaluate them
 //    once on the host with libm; the device sin may differ from it in the
 //    last bit, far inside the 1e-12 relative bound of the FP64 step);
-//  * the Flather faces are walked straight from the mask, one thread per U
-//    row and per V column in the reference's serial order, instead of over
-//    host-built segment lists.
+//  * the Flather faces are found from the mask, not from host-built segment
+//    lists.
 //
 // `scratch` is the only device memory beyond the caller's arrays. It is a
 // file-scope array: each GPU holds one copy from the library's load until
@@ -68,57 +71,6 @@ __global__ __launch_bounds__(256) void k_coriolis(const double *__restrict__ gph
     if (k >= n) return;
     fcor_u[k] = 2. * omega * sin(gphiu[k] * d2r);
     fcor_v[k] = 2. * omega * sin(gphiv[k] * d2r);
-}
-
-// bc_flather_u / bc_flather_v (boundary_conditions_kern.c:271-293,
-// :313-333) at face c with neighbours along `stride`; a neighbour outside
-// the allocation reads as 0, as in the segment-list kernel.
-__device__ __forceinline__ void flather_face(int c, int stride, int total,
-                                             const int *__restrict__ tm,
-                                             double *__restrict__ vel,
-                                             const double *__restrict__ h,
-                                             const double *__restrict__ ssh, double g)
-{
-    const int mc = tm[c], mp = tm[c + stride];
-    if (mc + mp <= -1) return;
-    int d;
-    if (mc < 0)
-        d = stride;
-    else if (mp < 0)
-        d = -stride;
-    else
-        return;
-    const int q = c + d;
-    const bool in = q >= 0 && q < total;
-    const double v_nb = in ? vel[q] : 0.0;
-    const double s_nb = in ? ssh[q] : 0.0;
-    vel[c] = v_nb + sqrt(g / h[c]) * (ssh[c] - s_nb);
-}
-
-// Thread t < nu walks U row ys-1+t over ji = xs-1 .. xe; the next nv
-// threads walk V column xs-1+(t-nu) over jj = ys-1 .. ye. Within a row (a
-// column) a face may read the one the sweep wrote just before it, so each
-// walk keeps the reference's order; rows and columns are independent.
-__global__ __launch_bounds__(64) void k_flather_walk(const int *__restrict__ tm,
-                                                     double *__restrict__ ua,
-                                                     double *__restrict__ va,
-                                                     const double *__restrict__ hu,
-                                                     const double *__restrict__ hv,
-                                                     const double *__restrict__ su,
-                                                     const double *__restrict__ sv,
-                                                     int W, int total, Bounds b, double g)
-{
-    const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    const int nu = b.ye - b.ys + 3, nv = b.xe - b.xs + 3;
-    if (t < nu) {
-        const int row = (b.ys - 1 + t) * W;
-        for (int ji = b.xs - 1; ji <= b.xe; ji++)
-            flather_face(row + ji, 1, total, tm, ua, hu, su, g);
-    } else if (t < nu + nv) {
-        const int ji = b.xs - 1 + (t - nu);
-        for (int jj = b.ys - 1; jj <= b.ye; jj++)
-            flather_face(jj * W + ji, W, total, tm, va, hv, sv, g);
-    }
 }
 
 }  // namespace
@@ -176,24 +128,9 @@ extern "C" void c_invoke_time_step_noalloc(NEMO_HOST_ARRAYS, int istep, int inte
     f.fcor_v = fcor_v;
     f.tmask = tmask;
     const StepScalars<double> p{rdt, visc, g, 1.0 + cbfr * rdt};
-    const int W = width;
-    const int xs = G.xs, xe = G.xe, ys = G.ys, ye = G.ye;
-    const Region interior{xs, xe, ys, ye};
-
-    // the sweep order and regions of time_step.cpp:53-136
-    launch_continuity(s, f, ssha_t, W, interior, rdt);
-    launch_momentum_u(s, f, p, ua, W, Region{xs, xe - 1, ys, ye});
-    launch_momentum_v(s, f, p, va, W, Region{xs, xe, ys, ye - 1});
-    launch_bc_ssh(s, tmask, ssha_t, W, interior, tide_at(istep, rdt));
-    launch_bc_solid(s, tmask, ua, W, 1, Region{xs - 1, xe, ys - 1, ye + 1});
-    launch_bc_solid(s, tmask, va, W, W, Region{xs - 1, xe + 1, ys - 1, ye});
-    const int walkers = (ye - ys + 3) + (xe - xs + 3);
-    k_flather_walk<<<dim3((unsigned)((walkers + 63) / 64)), dim3(64), 0, s>>>(
-        tmask, ua, va, hu, hv, sshn_u, sshn_v, W, total_size, Bounds{xs, xe, ys, ye}, g);
-    NEMO_LAUNCH_CHECK();
-    launch_copy3(s, un, ua, vn, va, sshn_t, ssha_t, W, Region{xs - 1, xe + 1, ys - 1, ye});
-    launch_next_ssh(s, tmask, sshn_t, area_t, area_u, sshn_u, W, 1,
-                    Region{xs, xe - 1, ys, ye});
-    launch_next_ssh(s, tmask, sshn_t, area_t, area_v, sshn_v, W, W,
-                    Region{xs, xe, ys, ye - 1});
+    const Bounds b{G.xs, G.xe, G.ys, G.ye};
+    launch_band_inplace(s, f, p, StepOut<double>{ssha_t, ua, va, nullptr, nullptr}, width, b,
+                        tide_at(istep, rdt));
+    launch_finish(s, un, ua, vn, va, sshn_t, ssha_t, sshn_u, sshn_v, tmask, area_t, area_u,
+                  area_v, width, b);
 }

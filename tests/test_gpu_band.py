@@ -124,3 +124,19 @@ def test_metrics_written_between_calls_are_seen():
         done += 3
         st.run(3)
         check(st, oracle_steps(m, host, done, 3), f"dx_v times {factor}")
+
+
+@pytest.mark.parametrize("nx, ny", [(3, 3), (61, 40), (509, 130), (1201, 900)])
+def test_inplace_step_equals_oracle(nx, ny):
+    """The allocation-free step, two in a row: one- and two-row bands on a
+    random mask, latitude 0 (where the device's sine and the host's agree),
+    every in-place array bitwise."""
+    from test_zz_no_alloc import OUT as INPLACE, _run_noalloc
+    m = live_model(nx, ny, "point", seed=7)
+    m.array("gphiu")[:] = 0.0
+    m.array("gphiv")[:] = 0.0
+    _native.hip_lib().nemo_hip_set_tide(m.cfg.tide_amp, m.cfg.tide_omega)
+    ref = oracle_steps(m, [a.copy() for a in m.arrays()], 1, 2)
+    got = _run_noalloc(m.copy(), 1, 2)
+    for n in INPLACE:
+        assert_bitwise(got[n], ref[n], f"in place {nx}x{ny} {n}")
