@@ -209,7 +209,8 @@ NEMO_API void nemo_mp_steps(void *handle, int nsteps, int istep);
  * mean duration in ms of the mixed step kernel. */
 NEMO_API double nemo_mp_kernel_ms(void *handle, int nsteps, int istep);
 /* Rows per band of the kernel: 4, 8, 16, 32 (default), 48, 64, 80, 96 or
- * 128. */
+ * 128. With the other settings at their defaults, 32 leaves the band height
+ * to the library, which picks it by the size of the grid. */
 NEMO_API void nemo_mp_set_rows(void *handle, int rows);
 /* Output columns per wavefront: 61 (default; strips overlap by 3 columns),
  * 56 (every strip's stores start on a 32-byte boundary) or 48 (on a 64-byte

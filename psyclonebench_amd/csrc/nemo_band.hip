@@ -1,5 +1,5 @@
-// Launchers of the band tile (nemo_band.h) for one FP64 domain, into the other
-// state set or in place, and the table of metrics by row.
+// Launchers of the band tile (nemo_band.h) for one domain: FP64 into the other
+// state set or in place, mixed precision, and the table of metrics by row.
 #include <algorithm>
 
 #include "nemo_band.h"
@@ -73,7 +73,9 @@ __device__ bool divisor_ok(double d)
 {
     return isfinite(d) && d != 0.0 && abs(__builtin_amdgcn_frexp_exp(d)) <= kDivisorExp;
 }
+__device__ bool divisor_ok(float) { return true; }
 __device__ double reciprocal(double d) { return band::refined_reciprocal(d); }
+__device__ float reciprocal(float d) { return __builtin_amdgcn_rcpf(d); }
 
 // One workgroup per row: writes the row's record from its first column and
 // stores `mark` to *bad when another column of the row holds other bits or a
@@ -196,8 +198,11 @@ long tiles(const Bounds &b, int rows, int ow)
 //                4096^2 540 / 430 / 406
 //   FP64         400^2 8.1 / 9.3 / 13.6;  700^2 20.3 / 22 / 23.5;  2048^2 207
 //                / 193 / 195;  4096^2 809 / 751 / 741
+//   FP32         512^2 6.2 / 7.1 / 10.3;  1024^2 16.6 / 16.7 / 17.7;  2048^2
+//                65 / 58 / 56;  4096^2 314 / 266 / 242 (by row)
 constexpr long kOneRowTilesF64 = 12000, kOneRowTilesByRowF64 = 3500;
 constexpr long kTwoRowTilesF64 = 48000, kTwoRowTilesByRowF64 = 24000;
+constexpr long kOneRowTilesF32 = 16000, kTwoRowTilesF32 = 20000;
 
 }  // namespace
 
@@ -207,6 +212,12 @@ void launch_row_metrics(hipStream_t s, const StepIn<double> &f, int W, unsigned 
                         const Bounds &b, double *tab, int *bad, int mark)
 {
     row_metrics<double>(s, f, W, base, b, tab, bad, mark);
+}
+
+void launch_row_metrics(hipStream_t s, const MixedIn &f, int W, unsigned base, const Bounds &b,
+                        float *tab, int *bad, int mark)
+{
+    row_metrics<float>(s, f, W, base, b, tab, bad, mark);
 }
 
 void launch_band_f64(hipStream_t s, const StepIn<double> &f, const double *tab,
@@ -231,6 +242,58 @@ void launch_band_f64(hipStream_t s, const StepIn<double> &f, const double *tab,
         else
             launch<double, false, 4, 56, 1, true, true>(a);
     }
+}
+
+bool band_f32_shape(int rows, int cols, int prefetch)
+{
+    return band_f32_auto(rows, cols, prefetch) ||
+           ((rows == 4 || rows == 8) && (cols == 61 || cols == 56) && prefetch >= 0 &&
+            prefetch <= 2);
+}
+
+void launch_band_f32(hipStream_t s, int rows, int cols, int prefetch, const MixedIn &f,
+                     const float *tab, const StepScalars<float> &p, const MixedOut &o,
+                     const float *u_prev, const float *v_prev, const float *cu,
+                     const float *cv, int W, const Bounds &b, const double *tide_tab, int tide_k,
+                     double tide_val)
+{
+    const Flather<float> fl{u_prev, v_prev, cu, cv, cu != nullptr};
+    const Args<float> a{s, f, tab, p, o, fl, W, b, tide_tab, tide_k, tide_val};
+    if (band_f32_auto(rows, cols, prefetch)) {
+        if (tiles(b, 1, 61) <= kOneRowTilesF32) {
+            tab ? launch<float, true, 1, 61, 0, true, false>(a)
+                : launch<float, false, 1, 61, 0, true, false>(a);
+            return;
+        }
+        if (tiles(b, 2, 61) <= kTwoRowTilesF32) {
+            tab ? launch<float, true, 2, 61, 0, true, false>(a)
+                : launch<float, false, 2, 61, 0, true, false>(a);
+            return;
+        }
+        rows = 4;
+        prefetch = tab ? 2 : 0;
+    }
+#define NEMO_BAND_F32(R, OW, PF)                                                     \
+    if (rows == R && cols == OW && prefetch == PF) {                                 \
+        tab ? launch<float, true, R, OW, PF, true, true>(a)                          \
+            : launch<float, false, R, OW, PF, true, true>(a);                        \
+        return;                                                                      \
+    }
+    NEMO_BAND_F32(4, 61, 0)
+    NEMO_BAND_F32(4, 61, 1)
+    NEMO_BAND_F32(4, 61, 2)
+    NEMO_BAND_F32(4, 56, 0)
+    NEMO_BAND_F32(4, 56, 1)
+    NEMO_BAND_F32(4, 56, 2)
+    NEMO_BAND_F32(8, 61, 0)
+    NEMO_BAND_F32(8, 61, 1)
+    NEMO_BAND_F32(8, 61, 2)
+    NEMO_BAND_F32(8, 56, 0)
+    NEMO_BAND_F32(8, 56, 1)
+    NEMO_BAND_F32(8, 56, 2)
+#undef NEMO_BAND_F32
+    NEMO_FATAL("mixed step: no band kernel for %d rows x %d columns, prefetch %d", rows, cols,
+               prefetch);
 }
 
 void launch_band_inplace(hipStream_t s, const StepIn<double> &f, const StepScalars<double> &p,

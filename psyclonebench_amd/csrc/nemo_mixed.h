@@ -43,6 +43,23 @@ struct MixedOut {
 void launch_mixed_step(hipStream_t s, int rows, int cols, int prefetch, const MixedIn &f,
                        const StepScalars<float> &p, const MixedOut &o, int W,
                        Bounds b, const double *tide_tab, int tide_k, double tide_val);
+// The band form (nemo_band.hip): the shapes it has (the others run
+// launch_mixed_step), and one step with its Flather faces. The default shape
+// of a handle (32 rows, 61 columns, no prefetch) stands for the library's
+// choice by grid size. tab: the row table (launch_row_metrics) or null; cu /
+// cv: sqrt(g / h) at the Flather faces, as arrays (null: no Flather face).
+constexpr bool band_f32_auto(int rows, int cols, int prefetch)
+{
+    return rows == 32 && cols == 61 && prefetch == 0;
+}
+bool band_f32_shape(int rows, int cols, int prefetch);
+void launch_row_metrics(hipStream_t s, const MixedIn &f, int W, unsigned base, const Bounds &b,
+                        float *tab, int *bad, int mark);
+void launch_band_f32(hipStream_t s, int rows, int cols, int prefetch, const MixedIn &f,
+                     const float *tab, const StepScalars<float> &p, const MixedOut &o,
+                     const float *u_prev, const float *v_prev, const float *cu,
+                     const float *cv, int W, const Bounds &b, const double *tide_tab, int tide_k,
+                     double tide_val);
 // ua_prev / va_prev: the previous step's velocities (see FlatherList)
 void launch_flather_f32(hipStream_t s, const FlatherList &lu, const FlatherList &lv,
                         float *ua, float *va, const float *ua_prev, const float *va_prev,

@@ -2,6 +2,7 @@
 // opaque handle owns FP32 copies of the 25 arrays (ssh as a compensated
 // hi/lo pair), the Flather segment lists and captured step graphs. The state
 // ping-pongs between two buffer sets like the FP64 fused form.
+#include <algorithm>
 #include <cmath>
 #include <map>
 #include <memory>
@@ -26,6 +27,9 @@ struct MixedContext {
     float *cst[A_COUNT] = {};        // constant arrays (FP32); tmask in tm
     signed char *tm = nullptr;       // T mask, one byte a point
     float *fcor_u = nullptr, *fcor_v = nullptr;
+    // band form: the table of metrics by row (null: they vary along a row) and
+    // the Flather factors at their faces (null: no Flather face)
+    float *row_tab = nullptr, *cu = nullptr, *cv = nullptr;
     float *t_hi[2] = {}, *t_lo[2] = {}, *u[2] = {}, *v[2] = {}, *su[2] = {}, *sv[2] = {};
     DeviceFlather fl_u, fl_v;
     int parity = 0;
@@ -81,7 +85,7 @@ struct MixedContext {
         for (hipEvent_t e : ev) (void)hipEventDestroy(e);
         for (float *p : cst)
             if (p) (void)hipFree(p);
-        float *more[] = {fcor_u, fcor_v, t_hi[0], t_hi[1], t_lo[0], t_lo[1], u[0], u[1],
+        float *more[] = {fcor_u, fcor_v, row_tab, cu, cv, t_hi[0], t_hi[1], t_lo[0], t_lo[1], u[0], u[1],
                          v[0], v[1], su[0], su[1], sv[0], sv[1]};
         for (float *p : more)
             if (p) (void)hipFree(p);
@@ -108,13 +112,50 @@ void launch_pair(MixedContext &C, int par, hipStream_t s, const double *tide_tab
 {
     const int q = 1 - par;
     const MixedOut o{C.t_hi[q], C.t_lo[q], C.u[q], C.v[q], C.su[q], C.sv[q]};
-    if (e0) NEMO_HIP_CHECK(hipEventRecord(e0, s));
-    launch_mixed_step(s, C.rows, C.cols, C.prefetch, C.inputs(par), C.scalars(), o, C.G.W,
-                      Bounds{C.G.xs, C.G.xe, C.G.ys, C.G.ye}, tide_tab, k, tide_val);
-    if (e1) NEMO_HIP_CHECK(hipEventRecord(e1, s));
+    const Bounds b{C.G.xs, C.G.xe, C.G.ys, C.G.ye};
     const int prev = C.paired ? par : q;  // the previous step's velocities
-    launch_flather_f32(s, C.fl_u.view(), C.fl_v.view(), C.u[q], C.v[q], C.u[prev],
-                       C.v[prev], C.su[par], C.sv[par]);
+    const bool band = band_f32_shape(C.rows, C.cols, C.prefetch);
+    if (e0) NEMO_HIP_CHECK(hipEventRecord(e0, s));
+    if (band)
+        launch_band_f32(s, C.rows, C.cols, C.prefetch, C.inputs(par), C.row_tab, C.scalars(), o,
+                        C.u[prev], C.v[prev], C.cu, C.cv, C.G.W, b, tide_tab, k, tide_val);
+    else
+        launch_mixed_step(s, C.rows, C.cols, C.prefetch, C.inputs(par), C.scalars(), o, C.G.W,
+                          b, tide_tab, k, tide_val);
+    if (e1) NEMO_HIP_CHECK(hipEventRecord(e1, s));
+    if (!band)  // the band form's tiles do these
+        launch_flather_f32(s, C.fl_u.view(), C.fl_v.view(), C.u[q], C.v[q], C.u[prev],
+                           C.v[prev], C.su[par], C.sv[par]);
+}
+
+// The Flather factors as arrays (read at the Flather faces only) and the
+// table of metrics by row, if the grid has them. The arrays of a handle are
+// its own, so one look at creation stands.
+void prepare_band(MixedContext &C, const HostFlather &u, const HostFlather &v, hipStream_t s)
+{
+    const size_t n = (size_t)C.G.total;
+    if (!u.idx.empty() || !v.idx.empty()) {
+        std::vector<float> c(n, 0.0f);
+        for (size_t k = 0; k < u.idx.size(); k++) c[u.idx[k]] = (float)u.coef[k];
+        C.cu = dev_alloc<float>(n);
+        NEMO_HIP_CHECK(hipMemcpy(C.cu, c.data(), n * sizeof(float), hipMemcpyHostToDevice));
+        std::fill(c.begin(), c.end(), 0.0f);
+        for (size_t k = 0; k < v.idx.size(); k++) c[v.idx[k]] = (float)v.coef[k];
+        C.cv = dev_alloc<float>(n);
+        NEMO_HIP_CHECK(hipMemcpy(C.cv, c.data(), n * sizeof(float), hipMemcpyHostToDevice));
+    }
+    const Bounds b{C.G.xs, C.G.xe, C.G.ys, C.G.ye};
+    C.row_tab = dev_alloc<float>(row_table_values(b));
+    int *bad = dev_alloc<int>(1), host_bad = 0;
+    NEMO_HIP_CHECK(hipMemcpy(bad, &host_bad, sizeof(int), hipMemcpyHostToDevice));
+    launch_row_metrics(s, C.inputs(0), C.G.W, 0u, b, C.row_tab, bad, 1);
+    NEMO_HIP_CHECK(hipStreamSynchronize(s));
+    NEMO_HIP_CHECK(hipMemcpy(&host_bad, bad, sizeof(int), hipMemcpyDeviceToHost));
+    NEMO_HIP_CHECK(hipFree(bad));
+    if (host_bad) {
+        NEMO_HIP_CHECK(hipFree(C.row_tab));
+        C.row_tab = nullptr;
+    }
 }
 
 void first_step(MixedContext &C, int istep, hipStream_t s)
@@ -210,8 +251,11 @@ void *nemo_mp_create(NEMO_HOST_ARRAYS, int internal_xstart, int internal_xstop,
         C->su[set] = upload_f32(sshn_u, n, s);
         C->sv[set] = upload_f32(sshn_v, n, s);
     }
-    C->fl_u.upload(build_flather(tmask, hu, G, g, true), s);
-    C->fl_v.upload(build_flather(tmask, hv, G, g, false), s);
+    const HostFlather fu_list = build_flather(tmask, hu, G, g, true);
+    const HostFlather fv_list = build_flather(tmask, hv, G, g, false);
+    C->fl_u.upload(fu_list, s);
+    C->fl_v.upload(fv_list, s);
+    prepare_band(*C, fu_list, fv_list, s);
     return C.release();
 }
 

@@ -13,7 +13,7 @@ import oracle
 from helpers import assert_bitwise
 from psyclonebench_amd import _native
 from psyclonebench_amd.model import Model, c1_config
-from psyclonebench_amd.psy import TimeStepper
+from psyclonebench_amd.psy import MixedStepper, TimeStepper
 
 pytestmark = pytest.mark.gpu
 
@@ -140,3 +140,23 @@ def test_inplace_step_equals_oracle(nx, ny):
     got = _run_noalloc(m.copy(), 1, 2)
     for n in INPLACE:
         assert_bitwise(got[n], ref[n], f"in place {nx}x{ny} {n}")
+
+
+@pytest.mark.parametrize("metrics", ["row", "point"])
+@pytest.mark.parametrize("nx, ny", [(3, 3), (61, 64), (130, 33), (1101, 1000), (2003, 1250)])
+def test_mixed_band_equals_the_other_kernels(nx, ny, metrics):
+    """The FP32 band form (automatic: one, two and four rows; and the explicit
+    shapes that run it) has the bits of the 48-column kernel with its separate
+    Flather launch, on a random mask."""
+    print("mixed band", nx, ny, metrics, flush=True)
+    m = live_model(nx, ny, metrics, seed=8)
+    ref = None
+    for rows, cols, pf in ((16, 48, 0), (32, 61, 0), (4, 61, 2), (4, 56, 1), (8, 61, 0),
+                           (8, 56, 2)):
+        st = MixedStepper(m, rows=rows, cols=cols, prefetch=pf)
+        st.run(4)
+        out = {n: st.fetch(n) for n in ("sshn_t", "un", "vn", "sshn_u", "sshn_v")}
+        st.release()
+        ref = ref or out
+        for n in out:
+            assert_bitwise(out[n], ref[n], f"{nx}x{ny} {metrics} {rows}x{cols} p{pf} {n}")
