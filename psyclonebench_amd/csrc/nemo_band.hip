@@ -200,6 +200,11 @@ long tiles(const Bounds &b, int rows, int ow)
 //                / 193 / 195;  4096^2 809 / 751 / 741
 //   FP32         512^2 6.2 / 7.1 / 10.3;  1024^2 16.6 / 16.7 / 17.7;  2048^2
 //                65 / 58 / 56;  4096^2 314 / 266 / 242 (by row)
+// The largest FP64 bands store past the caches (STREAM): by then a step's
+// output is gone from them before the next step reads it (us a step, with and
+// without: 1800^2 82 / 88, 2048^2 102 / 113, 4096^2 404 / 423). Below, and in
+// FP32, the next step finds it there (1024^2 31.1 / 25.4, 1500^2 61 / 54;
+// FP32 1500^2 79 / 69, 2048^2 116 / 110 with the read-back).
 constexpr long kOneRowTilesF64 = 12000, kOneRowTilesByRowF64 = 3500;
 constexpr long kTwoRowTilesF64 = 48000, kTwoRowTilesByRowF64 = 24000;
 constexpr long kOneRowTilesF32 = 16000, kTwoRowTilesF32 = 20000;
@@ -275,8 +280,8 @@ void launch_band_f32(hipStream_t s, int rows, int cols, int prefetch, const Mixe
     }
 #define NEMO_BAND_F32(R, OW, PF)                                                     \
     if (rows == R && cols == OW && prefetch == PF) {                                 \
-        tab ? launch<float, true, R, OW, PF, true, true>(a)                          \
-            : launch<float, false, R, OW, PF, true, true>(a);                        \
+        tab ? launch<float, true, R, OW, PF, true, false>(a)                         \
+            : launch<float, false, R, OW, PF, true, false>(a);                       \
         return;                                                                      \
     }
     NEMO_BAND_F32(4, 61, 0)
