@@ -52,7 +52,7 @@ using wave::Ssh;
 enum RowSlot {
     M_AT, M_ARU, M_ARV, M_E1U, M_E1V, M_E1V2, M_E1T, M_E2U, M_E2US, M_E2V, M_E2T, M_FCU,
     M_FCV, M_SAU, M_SAV,
-    R_AT = 16, R_ARU, R_ARV, R_E1V2, R_E1T, R_E2US, R_E2T, ROW_WIDTH = 32
+    R_AT = 16, R_ARU, R_ARV, R_E1V2, R_E1T, R_E2US, R_E2T, ROW_WIDTH = kRowTableWidth
 };
 
 // Quotient by a divisor that a whole row shares: a multiplication by its
@@ -111,8 +111,9 @@ struct Flather {
     int on;
 };
 
-// First owned lane of a strip of ow columns.
-constexpr int first_lane(int ow) { return (64 - ow) / 2; }
+// First owned lane of a strip of ow columns: one neighbour lane below and two
+// above, so ow <= 61.
+__device__ __forceinline__ constexpr int first_lane(int ow) { return (64 - ow) / 2; }
 
 template <bool STREAM, typename T>
 __device__ __forceinline__ void store(T *__restrict__ base, unsigned off, T v)
@@ -190,17 +191,18 @@ __device__ __forceinline__ void flather_faces(T *vel, const T *ssh, const T *coe
 // The Flather faces next to the points that the lanes of a strip own in rows
 // jlo .. jhi-1, from memory, after the rows are stored (the lane's own stores
 // are visible to it).
-template <typename T, int OW>
+template <typename T>
 __device__ __forceinline__ void flather_rows(const typename Types<T>::In &f,
                                              const StepScalars<T> &p,
                                              const typename Types<T>::Out &o,
                                              const Flather<T> &fl, int W, unsigned base,
-                                             const Bounds &b, int strip, int jlo, int jhi)
+                                             const Bounds &b, int ow, int strip, int jlo,
+                                             int jhi)
 {
-    constexpr int L0 = first_lane(OW);
+    const int l0 = first_lane(ow);
     const int xmax = b.xe + 1, ymax = b.ye + 1;
-    const int lane = (int)(threadIdx.x & 63), i = b.xs - 1 + strip * OW + lane - L0;
-    if (lane < L0 || lane >= L0 + OW || i > xmax) return;
+    const int lane = (int)(threadIdx.x & 63), i = b.xs - 1 + strip * ow + lane - l0;
+    if (lane < l0 || lane >= l0 + ow || i > xmax) return;
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
 #pragma unroll 1
     for (int j = jlo; j < jhi; j++) {
@@ -230,31 +232,31 @@ __device__ __forceinline__ void flather_rows(const typename Types<T>::In &f,
 
 // ---- the tile ---------------------------------------------------------------
 // T: double (the reference's bits) or float (mixed form). ROWM: metrics by
-// row, `tab` the record of row 0. At most R rows (jlo .. jhi-1), PF rows of
+// row, `tab` the record of row 0. ow: owned columns of the strip (a constant
+// of the launch or of the tile). At most R rows (jlo .. jhi-1), PF rows of
 // loads in flight beyond the next (the loop is unrolled, so the window shifts
 // are register renaming). NEXT: write the new face ssh (false where the step
 // updates the caller's arrays in place and a second kernel follows). STREAM:
 // non-temporal stores. QUICK: uniform_quotient for the row's divisors.
 // Returns the first row that is not done: jhi (or jlo + R), or with QUICK a
 // row with a numerator outside its range.
-template <typename T, bool ROWM, int R, int OW, int PF, bool NEXT, bool STREAM, bool QUICK>
+template <typename T, bool ROWM, int R, int PF, bool NEXT, bool STREAM, bool QUICK>
 __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__restrict__ tab,
                                     const StepScalars<T> &p, const typename Types<T>::Out &o,
                                     const Flather<T> &fl, int W, unsigned base,
-                                    const Bounds &b, int strip, int jlo, int jhi,
+                                    const Bounds &b, int ow, int strip, int jlo, int jhi,
                                     typename Types<T>::Tide tide)
 {
     constexpr bool MIXED = sizeof(T) == 4;
-    constexpr int L0 = first_lane(OW);
+    const int l0 = first_lane(ow);
     constexpr bool SHORT = R <= 2;  // Flather faces from the registers
-    static_assert(L0 >= 1 && L0 + OW + 2 <= 64, "one neighbour lane below, two above");
     static_assert(PF >= 0 && PF <= 2 && R >= 1 && R <= 16, "unrolled band");
     using S = typename Types<T>::NewSsh;
     const int xmax = b.xe + 1, ymax = b.ye + 1;
     const int lane = (int)(threadIdx.x & 63);
-    const int i = b.xs - 1 + strip * OW + lane - L0;  // may be < 0 or > xmax
+    const int i = b.xs - 1 + strip * ow + lane - l0;  // may be < 0 or > xmax
     const unsigned ci = (unsigned)min(max(i, 0), xmax);
-    const bool own = lane >= L0 && lane < L0 + OW && i <= xmax;
+    const bool own = lane >= l0 && lane < l0 + ow && i <= xmax;
     auto row = [&](int j) { return min(max(j, 0), ymax); };
     auto at_row = [&](int j) { return base + (unsigned)(row(j) * W) + ci; };
     auto rec = [&](int j) { return tab + row(j) * ROW_WIDTH; };
@@ -613,27 +615,27 @@ __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__r
     }
     // longer bands: the Flather faces afterwards, where the band has open cells
     if (!SHORT && fl.on && __any(open < 0))
-        flather_rows<T, OW>(f, p, o, fl, W, base, b, strip, jlo, done);
+        flather_rows<T>(f, p, o, fl, W, base, b, ow, strip, jlo, done);
     return done;
 }
 
 // Rows jlo .. jhi-1 (at most R) of one strip: the quick form, and plain
 // divisions from a row on whose numerators leave its range (a wave front that
 // runs into a basin at rest).
-template <typename T, bool ROWM, int R, int OW, int PF, bool NEXT, bool STREAM>
+template <typename T, bool ROWM, int R, int PF, bool NEXT, bool STREAM>
 __device__ __forceinline__ void tile(const typename Types<T>::In &f, const T *__restrict__ tab,
                                      const StepScalars<T> &p, const typename Types<T>::Out &o,
                                      const Flather<T> &fl, int W, unsigned base,
-                                     const Bounds &b, int strip, int jlo, int jhi,
+                                     const Bounds &b, int ow, int strip, int jlo, int jhi,
                                      typename Types<T>::Tide tide)
 {
     constexpr bool QUICK = ROWM && sizeof(T) == 8;
-    const int next = rows<T, ROWM, R, OW, PF, NEXT, STREAM, QUICK>(f, tab, p, o, fl, W, base, b,
-                                                                   strip, jlo, jhi, tide);
+    const int next = rows<T, ROWM, R, PF, NEXT, STREAM, QUICK>(f, tab, p, o, fl, W, base, b, ow,
+                                                               strip, jlo, jhi, tide);
     if constexpr (QUICK)
         if (next < jhi)
-            rows<T, ROWM, R, OW, 0, NEXT, STREAM, false>(f, tab, p, o, fl, W, base, b, strip,
-                                                         next, jhi, tide);
+            rows<T, ROWM, R, 0, NEXT, STREAM, false>(f, tab, p, o, fl, W, base, b, ow, strip,
+                                                     next, jhi, tide);
 }
 
 }  // namespace band

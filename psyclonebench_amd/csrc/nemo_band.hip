@@ -18,16 +18,17 @@ __global__ __launch_bounds__(64) void k_band(typename band::Types<T>::In f,
                                              const double *__restrict__ tide_tab, int tide_k,
                                              double tide_val)
 {
+    static_assert(OW <= 61, "one neighbour lane below, two above");
     const int logical = wave::xcd_tile((int)blockIdx.x, (int)gridDim.x);
     const int bd = logical / nstrip, strip = logical - bd * nstrip;
     const int jlo = b.ys - 1 + bd * R, jhi = min(jlo + R, b.ye + 2);
     const double tide = tide_tab ? tide_tab[tide_k] : tide_val;
     if constexpr (sizeof(T) == 8)
-        band::tile<T, ROWM, R, OW, PF, NEXT, STREAM>(f, tab, p, o, fl, W, 0u, b, strip, jlo, jhi,
-                                                     tide);
+        band::tile<T, ROWM, R, PF, NEXT, STREAM>(f, tab, p, o, fl, W, 0u, b, OW, strip, jlo, jhi,
+                                                 tide);
     else
-        band::tile<T, ROWM, R, OW, PF, NEXT, STREAM>(f, tab, p, o, fl, W, 0u, b, strip, jlo, jhi,
-                                                     wave::split(tide));
+        band::tile<T, ROWM, R, PF, NEXT, STREAM>(f, tab, p, o, fl, W, 0u, b, OW, strip, jlo, jhi,
+                                                 wave::split(tide));
 }
 
 template <typename T>

@@ -27,7 +27,8 @@ struct alignas(16) EnsTile {
     unsigned off;
     int W, xs, xe, ys, ye;
     int strip, band, dom, cols;
-    int pad[2];
+    int rec;  // the domain's first record in the table of metrics by row
+    int pad;
 };
 static_assert(sizeof(EnsTile) == 48, "tile descriptor: 12 dwords");
 
@@ -49,6 +50,33 @@ struct EnsShape {
 // True when a kernel instantiation exists for the shape's launch form, rows,
 // columns and prefetch depth.
 bool ens_shape_supported(const EnsShape &shape);
+
+// Shapes that run band tiles (nemo_band.h): no Flather launch follows them.
+bool ens_band(const EnsShape &shape);
+
+// Tiles of a band shape. The shape of a new ensemble (4 rows, columns per
+// domain, prefetch 2) leaves them to the library, which picks them by the
+// number of tiles that bands of one and of two rows would give; the others
+// are taken as they are.
+struct EnsBand {
+    int rows, cols, prefetch;
+    bool stream;  // non-temporal stores
+};
+EnsBand ens_band_tiles(const EnsShape &shape, int precision, bool by_row, long one_row_tiles,
+                       long two_row_tiles);
+
+// One step of every domain in band tiles, Flather faces included. tab: the
+// table of metrics by row (null: they vary along a row in some domain);
+// u_prev / v_prev: the velocities at the end of the previous step; cu / cv:
+// sqrt(g / h) at the Flather faces (null: no Flather face).
+void launch_ens_band(hipStream_t s, const EnsBand &tiles_of, const StepIn<double> &in,
+                     const double *tab, const StepScalars<double> &p, const StepOut<double> &out,
+                     const double *u_prev, const double *v_prev, const EnsTile *tiles,
+                     int ntiles, const double *tide);
+void launch_ens_band(hipStream_t s, const EnsBand &tiles_of, const MixedIn &in, const float *tab,
+                     const StepScalars<float> &p, const MixedOut &out, const float *u_prev,
+                     const float *v_prev, const float *cu, const float *cv,
+                     const EnsTile *tiles, int ntiles, const double *tide);
 
 // FP64 step of every domain: state `in` -> `out` (arena base pointers).
 // tide: the bc_ssh elevation of each domain for this step.

@@ -1,28 +1,31 @@
 // Batched ensemble step (CDNA4 / gfx950): one launch per step advances
 // every domain of the ensemble.
 //
-// Work list: every domain is cut into tiles of one overlapped-wavefront strip
-// (OW output columns: 61, or 56 so that every strip's stores start on a
-// 64-byte boundary, or per domain whichever of the two suits its width) by
-// one band (R rows); the list holds one self-contained descriptor per tile
-// (domain geometry, strip, band, width), domain by domain. Two launch forms run wave::tile_f64 /
-// tile_mixed on the domain's arrays of each tile:
+// Work list: every domain is cut into tiles of one strip (OW output columns:
+// 61, or 56 so that every strip's stores start on a 64-byte boundary, or per
+// domain whichever of the two suits its width) by one band (R rows); the list
+// holds one self-contained descriptor per tile (domain geometry, strip, band,
+// width), domain by domain. Two launch forms run on the domain's arrays of
+// each tile:
 //
+//  * one wavefront per tile: a grid of one-wavefront workgroups, one per
+//    tile of the list, as the single-domain kernels launch, so that the
+//    dispatcher starts a new tile wherever a wavefront slot frees up. Bands
+//    of up to 8 rows are band tiles (nemo_band.h), which write the Flather
+//    faces themselves; 16-row ones run wave::tile_f64 / tile_mixed;
 //  * persistent: a fixed number of workgroups (a multiple of 8) of 1, 2 or
 //    4 wavefronts; every wavefront takes tiles from the list with a stride,
 //    so uneven domain sizes cost nothing but the partial tiles at their
-//    edges;
-//  * one wavefront per tile: a grid of one-wavefront workgroups, one per
-//    tile of the list, as the single-domain kernels launch, so that the
-//    dispatcher starts a new tile wherever a wavefront slot frees up.
+//    edges. These run wave::tile_f64 / tile_mixed.
 //
-// Either form runs the tile body with the loads of the next row issued at
-// the top of the row that needs them (PF = 0) or one row earlier (PF = 1).
+// Every form has the loads of the next row issued at the top of the row that
+// needs them (PF = 0), or one or two rows earlier.
 //
 // XCD locality: the dispatcher hands workgroup b to XCD b % 8. The list is
 // cut into 8 contiguous chunks and the workgroups of XCD x take tiles of
 // chunk x only, so neighbouring strips of a domain (which share the cache
 // lines of their overlap columns) are processed under one L2.
+#include "nemo_band.h"
 #include "nemo_ensemble.h"
 #include "nemo_hip_common.h"
 #include "nemo_wave.h"
@@ -47,23 +50,14 @@ __device__ __forceinline__ Walk walk(int ntiles)
     return Walk{t0 + k * wpb + wave, min(t0 + chunk, ntiles), per * wpb};
 }
 
-// Tile `tl` of the FP64 step; OW = 0 takes the tile width from the tile
-// (wavefront-uniform branch between the 61- and 56-column bodies).
 template <int R, int OW, int PF>
 __device__ __forceinline__ void ens_tile_f64(const StepIn<double> &f,
                                              const StepScalars<double> &p,
                                              const StepOut<double> &o, const EnsTile &tl,
                                              double tide)
 {
-    if constexpr (OW == 0) {
-        if (tl.cols == 61)
-            ens_tile_f64<R, 61, PF>(f, p, o, tl, tide);
-        else
-            ens_tile_f64<R, 56, PF>(f, p, o, tl, tide);
-    } else {
-        wave::tile_f64<R, OW, PF>(f, p, o, tl.W, tl.off, Bounds{tl.xs, tl.xe, tl.ys, tl.ye},
-                                  tl.strip, tl.band, tide);
-    }
+    wave::tile_f64<R, OW, PF>(f, p, o, tl.W, tl.off, Bounds{tl.xs, tl.xe, tl.ys, tl.ye},
+                              tl.strip, tl.band, tide);
 }
 
 template <int R, int OW, int PF>
@@ -71,16 +65,32 @@ __device__ __forceinline__ void ens_tile_mixed(const MixedIn &f, const StepScala
                                                const MixedOut &o, const EnsTile &tl,
                                                double tide)
 {
-    if constexpr (OW == 0) {
-        if (tl.cols == 61)
-            ens_tile_mixed<R, 61, PF>(f, p, o, tl, tide);
-        else
-            ens_tile_mixed<R, 56, PF>(f, p, o, tl, tide);
-    } else {
-        wave::tile_mixed<R, OW, PF>(f, p, o, tl.W, tl.off,
-                                    Bounds{tl.xs, tl.xe, tl.ys, tl.ye}, tl.strip, tl.band,
-                                    wave::split(tide));
-    }
+    wave::tile_mixed<R, OW, PF>(f, p, o, tl.W, tl.off, Bounds{tl.xs, tl.xe, tl.ys, tl.ye},
+                                tl.strip, tl.band, wave::split(tide));
+}
+
+// Band tile, one wavefront each; the grid has exactly ntiles workgroups. The
+// strip's width comes with the tile. ROWM: every domain has a table of metrics
+// by row (records tl.rec and on).
+template <typename T, bool ROWM, int R, int PF, bool STREAM>
+__global__ __launch_bounds__(64) void k_ens_band(typename band::Types<T>::In f,
+                                                 const T *__restrict__ tab, StepScalars<T> p,
+                                                 typename band::Types<T>::Out o,
+                                                 band::Flather<T> fl,
+                                                 const EnsTile *__restrict__ tiles,
+                                                 const double *__restrict__ tide)
+{
+    const EnsTile tl = tiles[wave::xcd_tile((int)blockIdx.x, (int)gridDim.x)];
+    const Bounds b{tl.xs, tl.xe, tl.ys, tl.ye};
+    const int jlo = tl.ys - 1 + tl.band * R, jhi = min(jlo + R, tl.ye + 2);
+    const T *const rec = ROWM ? tab + (size_t)tl.rec * band::ROW_WIDTH : nullptr;
+    const double td = tide[tl.dom];
+    if constexpr (sizeof(T) == 8)
+        band::tile<T, ROWM, R, PF, true, STREAM>(f, rec, p, o, fl, tl.W, tl.off, b, tl.cols,
+                                                 tl.strip, jlo, jhi, td);
+    else
+        band::tile<T, ROWM, R, PF, true, STREAM>(f, rec, p, o, fl, tl.W, tl.off, b, tl.cols,
+                                                 tl.strip, jlo, jhi, wave::split(td));
 }
 
 template <int R, int OW, int PF>
@@ -154,11 +164,27 @@ void check_shape(const EnsShape &sh)
     X(4, 61, 0) X(8, 61, 0) X(16, 61, 0) X(32, 61, 0) X(64, 61, 0) X(4, 56, 0)         \
     X(8, 56, 0) X(16, 56, 0) X(32, 56, 0) X(64, 56, 0) X(4, 61, 1) X(8, 61, 1)         \
     X(16, 61, 1) X(4, 56, 1) X(8, 56, 1) X(16, 56, 1)
-#define NEMO_ENS_GRID(X)                                                               \
-    X(4, 61, 0) X(8, 61, 0) X(16, 61, 0) X(4, 56, 0) X(8, 56, 0) X(16, 56, 0)          \
-    X(4, 61, 1) X(8, 61, 1) X(16, 61, 1) X(4, 56, 1) X(8, 56, 1) X(16, 56, 1)          \
-    X(4, 0, 0) X(8, 0, 0) X(4, 0, 1) X(8, 0, 1) X(4, 61, 2) X(8, 61, 2) X(4, 56, 2)     \
-    X(8, 56, 2) X(4, 0, 2) X(8, 0, 2)
+#define NEMO_ENS_GRID(X) X(16, 61, 0) X(16, 56, 0) X(16, 61, 1) X(16, 56, 1)
+
+// Tiles of the default shape, by how many bands of one and of two rows there
+// are (the reasons are those of the single domain: a wavefront with a SIMD to
+// itself wants one row, a full chip fewer halo rows; non-temporal stores where
+// a step's output is gone from the last-level cache before the next step).
+// Measured on ensembles of uneven domains, us a step:
+//   points       one row / two / four / four, non-temporal
+//   FP64 by row  54 k 6.8 / 7.0 / 11;  0.4 M 19.5 / 16.4 / 18;  1.2 M 50 / 36 /
+//                39 / 45;  2.9 M 133 / 93 / 86 / 83;  24 M 1029 / 711 / 679 / 647
+//   FP64         54 k 5.9 / 7.2 / 12;  0.4 M 18.4 / 19.6 / 22;  1.0 M 44.4 /
+//                43.4 / 48;  7.2 M 353 / 345 / 351, two rows non-temporal 334
+//   FP32 by row  54 k 4.2 / 5.4 / 8.9;  1.2 M 18.2 / 19.0 / 22;  2.9 M 33.7 /
+//                33.0 / 41 / 55;  24 M 441 / 394 / 410 / 442
+//   FP32         1.0 M 22 / 25 / 28;  2.9 M 85 / 76 / 76;  7.2 M 211 / 202 / 211
+// The overlapped-wavefront tiles took 13, 33, 68, 180 (2.9 M) and 81 us (FP32,
+// 2.9 M), with a Flather launch after each step.
+constexpr long kEnsOneRowTilesByRowF64 = 3500, kEnsOneRowTilesF64 = 12000;
+constexpr long kEnsOneRowTilesF32 = 24000;
+constexpr long kEnsTwoRowTilesByRowF64 = 24000, kEnsCachedTilesF64 = 48000;
+
 
 void unsupported(const EnsShape &sh)
 {
@@ -179,7 +205,79 @@ bool ens_shape_supported(const EnsShape &sh)
         NEMO_ENS_GRID(NEMO_ENS_HAS)
     }
 #undef NEMO_ENS_HAS
-    return false;
+    return ens_band(sh);
+}
+
+bool ens_band(const EnsShape &sh)
+{
+    return sh.blocks == 0 && (sh.rows == 4 || sh.rows == 8) &&
+           (sh.cols == 61 || sh.cols == 56 || sh.cols == 0) && sh.prefetch >= 0 &&
+           sh.prefetch <= 2;
+}
+
+EnsBand ens_band_tiles(const EnsShape &sh, int precision, bool by_row, long one_row_tiles,
+                       long two_row_tiles)
+{
+    if (sh.rows != 4 || sh.cols != 0 || sh.prefetch != 2)
+        return EnsBand{sh.rows, sh.cols, sh.prefetch, false};
+    const long one = precision == 32 ? kEnsOneRowTilesF32
+                     : by_row        ? kEnsOneRowTilesByRowF64
+                                     : kEnsOneRowTilesF64;
+    if (one_row_tiles <= one) return EnsBand{1, 61, 0, false};
+    if (precision == 32) return EnsBand{2, 61, 0, false};
+    if (by_row)
+        return two_row_tiles <= kEnsTwoRowTilesByRowF64 ? EnsBand{2, 61, 0, false}
+                                                        : EnsBand{4, 0, 0, true};
+    return EnsBand{2, 61, 0, two_row_tiles > kEnsCachedTilesF64};
+}
+
+template <typename T, typename In, typename Out>
+void launch_band(hipStream_t s, const EnsBand &bt, const In &in, const T *tab,
+                 const StepScalars<T> &p, const Out &out, const T *u_prev, const T *v_prev,
+                 const T *cu, const T *cv, const EnsTile *tiles, int ntiles, const double *tide)
+{
+    if (ntiles <= 0) return;
+    const band::Flather<T> fl{u_prev, v_prev, cu, cv, sizeof(T) == 8 || cu};
+    const dim3 grid((unsigned)ntiles), block(64);
+    auto run = [&](auto kernel) {
+        kernel<<<grid, block, 0, s>>>(in, tab, p, out, fl, tiles, tide);
+        NEMO_LAUNCH_CHECK();
+    };
+    if constexpr (sizeof(T) == 8) {
+        if (bt.stream && bt.rows == 4 && tab) return run(k_ens_band<T, true, 4, 0, true>);
+        if (bt.stream && bt.rows == 2 && !tab) return run(k_ens_band<T, false, 2, 0, true>);
+    }
+#define NEMO_ENS_BAND(R, PF)                                                           \
+    if (bt.rows == R && bt.prefetch == PF && !bt.stream)                               \
+        return tab ? run(k_ens_band<T, true, R, PF, false>)                            \
+                   : run(k_ens_band<T, false, R, PF, false>);
+    NEMO_ENS_BAND(1, 0)
+    NEMO_ENS_BAND(2, 0)
+    NEMO_ENS_BAND(4, 0)
+    NEMO_ENS_BAND(4, 1)
+    NEMO_ENS_BAND(4, 2)
+    NEMO_ENS_BAND(8, 0)
+    NEMO_ENS_BAND(8, 1)
+    NEMO_ENS_BAND(8, 2)
+#undef NEMO_ENS_BAND
+    NEMO_FATAL("ensemble launch: no band kernel for %d rows, prefetch %d", bt.rows, bt.prefetch);
+}
+
+void launch_ens_band(hipStream_t s, const EnsBand &bt, const StepIn<double> &in,
+                     const double *tab, const StepScalars<double> &p, const StepOut<double> &out,
+                     const double *u_prev, const double *v_prev, const EnsTile *tiles,
+                     int ntiles, const double *tide)
+{
+    launch_band<double>(s, bt, in, tab, p, out, u_prev, v_prev, nullptr, nullptr, tiles, ntiles,
+                        tide);
+}
+
+void launch_ens_band(hipStream_t s, const EnsBand &bt, const MixedIn &in, const float *tab,
+                     const StepScalars<float> &p, const MixedOut &out, const float *u_prev,
+                     const float *v_prev, const float *cu, const float *cv,
+                     const EnsTile *tiles, int ntiles, const double *tide)
+{
+    launch_band<float>(s, bt, in, tab, p, out, u_prev, v_prev, cu, cv, tiles, ntiles, tide);
 }
 
 void launch_ens_f64(hipStream_t s, const EnsShape &sh, const StepIn<double> &in,

@@ -1,7 +1,7 @@
 // C ABI of the batched ensemble (no counterpart in the reference): many
 // independent NEMOLite2D domains of uneven size, bathymetry and tide,
-// advanced together by one launch per step (plus one Flather
-// launch over every domain's boundary segments).
+// advanced together by one launch per step (and, in the shapes that do not run
+// band tiles, one Flather launch over every domain's boundary segments).
 //
 // Memory: one arena per field holding every domain back to back, each at an
 // element offset rounded to 64 (rows stay 512-B aligned in FP64); the state
@@ -16,6 +16,7 @@
 // nemo_ens_autotune times each
 // on the ensemble itself with HIP events and keeps the fastest, restoring the
 // state it advanced.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <limits>
@@ -59,6 +60,12 @@ struct EnsContext {
     // constant arenas by C-ABI index (A_HT, ..., A_DY_T) + Coriolis factors
     void *cst[A_COUNT] = {};
     void *fcor_u = nullptr, *fcor_v = nullptr;
+    // band tiles: the domains' tables of metrics by row, back to back (null:
+    // the metrics of some domain vary along a row), and the FP32 Flather
+    // factors at their faces (null: FP64, or no Flather face)
+    void *row_tab = nullptr;
+    float *cu = nullptr, *cv = nullptr;
+    std::vector<int> rec;  // first record of each domain
     // prognostic arenas: prog[set][k], k = t, t_lo (FP32 only), u, v, su, sv
     void *prog[2][kProg] = {};
     DeviceFlather fl_u, fl_v;
@@ -66,6 +73,7 @@ struct EnsContext {
     bool paired = false;
     std::vector<EnsShape> shapes;
     int shape = 0;
+    long one_row_tiles = 0, two_row_tiles = 0;  // of 61-column strips
     std::map<std::pair<int, int>, std::pair<EnsTile *, int>> lists;  // (rows, cols) -> list
     double *d_tide = nullptr, *h_tide = nullptr;
     int tide_cap = 0;                                 // steps
@@ -154,7 +162,7 @@ struct EnsContext {
         for (hipEvent_t e : ev) (void)hipEventDestroy(e);
         for (void *p : raw) (void)hipFree(p);
         for (auto &kv : lists) (void)hipFree(kv.second.first);
-        void *more[] = {d_tide};
+        void *more[] = {d_tide, row_tab};
         for (void *p : more)
             if (p) (void)hipFree(p);
         if (h_tide) (void)hipHostFree(h_tide);
@@ -249,12 +257,32 @@ void build_shapes(EnsContext &C)
             }
 }
 
+// Tiles of every domain with R-row bands of 61-column strips.
+long tiles_of(const EnsContext &C, int rows)
+{
+    long n = 0;
+    for (const EnsDomain &e : C.hdom) {
+        const Bounds b{e.xs, e.xe, e.ys, e.ye};
+        n += (long)wave::strips(b, 61) * wave::bands(b, rows);
+    }
+    return n;
+}
+
+// Rows and columns of the tile list of a shape.
+std::pair<int, int> list_key(const EnsContext &C, const EnsShape &sh)
+{
+    if (!ens_band(sh)) return {sh.rows, sh.cols};
+    const EnsBand bt =
+        ens_band_tiles(sh, C.prec, C.row_tab != nullptr, C.one_row_tiles, C.two_row_tiles);
+    return {bt.rows, bt.cols};
+}
+
 // One tile list per (rows, columns) that some launch shape uses.
 void build_lists(EnsContext &C, hipStream_t s)
 {
     std::vector<std::vector<EnsTile>> host;  // alive until the copies are done
     for (const EnsShape &sh : C.shapes) {
-        const int rows = sh.rows, cols = sh.cols;
+        const auto [rows, cols] = list_key(C, sh);
         if (C.lists.count({rows, cols})) continue;
         std::vector<EnsTile> L;
         std::vector<int> ow(C.ndom), ns(C.ndom), nb(C.ndom);
@@ -268,7 +296,7 @@ void build_lists(EnsContext &C, hipStream_t s)
         auto push = [&](int d, int band, int strip) {
             const EnsDomain &e = C.hdom[d];
             L.push_back(EnsTile{e.off, e.W, e.xs, e.xe, e.ys, e.ye, strip, band, d, ow[d],
-                                {0, 0}});
+                                C.rec[d], 0});
         };
         for (int d = 0; d < C.ndom; d++)
             for (int band = 0; band < nb[d]; band++)
@@ -305,6 +333,48 @@ void build_flather_lists(EnsContext &C, void *const *arrays, hipStream_t s)
     }
     C.fl_u.upload(U, s);
     C.fl_v.upload(V, s);
+    if (C.prec == 64 || (U.idx.empty() && V.idx.empty())) return;
+    // the factors as arenas, read at the Flather faces only
+    std::vector<float> c(C.total);
+    for (int dir = 0; dir < 2; dir++) {
+        const HostFlather &L = dir ? V : U;
+        std::fill(c.begin(), c.end(), 0.0f);
+        for (size_t k = 0; k < L.idx.size(); k++) c[(size_t)L.idx[k]] = (float)L.coef[k];
+        float *&dst = dir ? C.cv : C.cu;
+        dst = static_cast<float *>(arena(C, sizeof(float), s));
+        NEMO_HIP_CHECK(hipMemcpyAsync(dst, c.data(), C.total * sizeof(float),
+                                      hipMemcpyHostToDevice, s));
+        NEMO_HIP_CHECK(hipStreamSynchronize(s));  // c is reused
+    }
+}
+
+// The tables of metrics by row of every domain; dropped when one domain has
+// none. The arenas are the ensemble's own and do not change, so one look at
+// creation stands.
+template <typename T, typename In>
+void build_row_tables(EnsContext &C, const In &in, hipStream_t s)
+{
+    size_t values = 0;
+    for (const EnsDomain &e : C.hdom) {
+        C.rec.push_back((int)(values / kRowTableWidth));
+        values += row_table_values(Bounds{e.xs, e.xe, e.ys, e.ye});
+    }
+    T *const tab = dev_alloc<T>(values);
+    C.row_tab = tab;
+    int *bad = dev_alloc<int>(1), host_bad = 0;
+    NEMO_HIP_CHECK(hipMemcpy(bad, &host_bad, sizeof(int), hipMemcpyHostToDevice));
+    for (int d = 0; d < C.ndom; d++) {
+        const EnsDomain &e = C.hdom[d];
+        launch_row_metrics(s, in, e.W, e.off, Bounds{e.xs, e.xe, e.ys, e.ye},
+                           tab + (size_t)C.rec[d] * kRowTableWidth, bad, 1);
+    }
+    NEMO_HIP_CHECK(hipStreamSynchronize(s));
+    NEMO_HIP_CHECK(hipMemcpy(&host_bad, bad, sizeof(int), hipMemcpyDeviceToHost));
+    NEMO_HIP_CHECK(hipFree(bad));
+    if (host_bad) {
+        NEMO_HIP_CHECK(hipFree(C.row_tab));
+        C.row_tab = nullptr;
+    }
 }
 
 double tide_value(const EnsContext &C, int d, int istep)
@@ -342,19 +412,35 @@ void launch_pair(EnsContext &C, int par, int row, hipStream_t s, hipEvent_t e0 =
 {
     const int q = 1 - par;
     const EnsShape &sh = C.shapes[C.shape];
-    const auto &L = C.lists.at({sh.rows, sh.cols});
+    const auto &L = C.lists.at(list_key(C, sh));
     const double *tide = C.d_tide + (size_t)row * C.ndom;
+    const int prev = C.paired ? par : q;  // the previous step's velocities
+    const bool band = ens_band(sh);
+    const EnsBand bt =
+        ens_band_tiles(sh, C.prec, C.row_tab != nullptr, C.one_row_tiles, C.two_row_tiles);
     if (e0) NEMO_HIP_CHECK(hipEventRecord(e0, s));
     if (C.prec == 64) {
         const StepScalars<double> p{C.P.rdt, C.P.visc, C.P.g, 1.0 + C.P.cbfr * C.P.rdt};
-        launch_ens_f64(s, sh, C.in64(par), p, C.out64(q), L.first, L.second, tide);
+        if (band)
+            launch_ens_band(s, bt, C.in64(par), static_cast<const double *>(C.row_tab), p,
+                            C.out64(q), static_cast<const double *>(C.prog[prev][2]),
+                            static_cast<const double *>(C.prog[prev][3]), L.first, L.second,
+                            tide);
+        else
+            launch_ens_f64(s, sh, C.in64(par), p, C.out64(q), L.first, L.second, tide);
     } else {
         const StepScalars<float> p{(float)C.P.rdt, (float)C.P.visc, (float)C.P.g,
                                    (float)(1.0 + C.P.cbfr * C.P.rdt)};
-        launch_ens_mixed(s, sh, C.in32(par), p, C.out32(q), L.first, L.second, tide);
+        if (band)
+            launch_ens_band(s, bt, C.in32(par), static_cast<const float *>(C.row_tab), p,
+                            C.out32(q), static_cast<const float *>(C.prog[prev][2]),
+                            static_cast<const float *>(C.prog[prev][3]), C.cu, C.cv, L.first,
+                            L.second, tide);
+        else
+            launch_ens_mixed(s, sh, C.in32(par), p, C.out32(q), L.first, L.second, tide);
     }
     if (e1) NEMO_HIP_CHECK(hipEventRecord(e1, s));
-    const int prev = C.paired ? par : q;  // the previous step's velocities
+    if (band) return;  // its tiles write the Flather faces
     if (C.prec == 64)
         launch_flather(s, C.fl_u.view(), C.fl_v.view(), static_cast<double *>(C.prog[q][2]),
                        static_cast<double *>(C.prog[q][3]),
@@ -532,11 +618,15 @@ void *nemo_ens_create(int ndom, void *const *arrays, const int *geom,
         NEMO_HIP_CHECK(hipStreamSynchronize(s));  // fu / fv / tm8 go out of scope
     }
     build_flather_lists(*C, arrays, s);
+    if (precision == 64)
+        build_row_tables<double>(*C, C->in64(0), s);
+    else
+        build_row_tables<float>(*C, C->in32(0), s);
+    C->one_row_tiles = tiles_of(*C, 1);
+    C->two_row_tiles = tiles_of(*C, 2);
     build_shapes(*C);
     build_lists(*C, s);
-    // default: one wavefront per tile, 4 rows, 61 or 56 columns per domain,
-    // loads three rows ahead, in both precisions (the fastest shape on a
-    // 256-domain ensemble of sides 64..1024 on MI355X)
+    // default: the shape that leaves the tiles to the library
     for (size_t k = 0; k < C->shapes.size(); k++) {
         const EnsShape &sh = C->shapes[k];
         if (sh.blocks == 0 && sh.rows == 4 && sh.cols == 0 && sh.prefetch == 2)

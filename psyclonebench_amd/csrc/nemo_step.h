@@ -104,6 +104,7 @@ const char *march_variant_kernel(int variant);
 // (memory that the device can write) when they do vary or a divisor is out of
 // the table's range (2^+-kDivisorExp).
 constexpr int kDivisorExp = 100;
+constexpr int kRowTableWidth = 32;  // values a record
 size_t row_table_values(const Bounds &b);
 void launch_row_metrics(hipStream_t s, const StepIn<double> &f, int W, unsigned base,
                         const Bounds &b, double *tab, int *bad, int mark);

@@ -16,6 +16,7 @@ from psyclonebench_amd import _native
 from psyclonebench_amd.ensemble import EnsembleStepper, ensemble_configs
 from psyclonebench_amd.model import Model
 from psyclonebench_amd.psy import MixedStepper, TimeStepper
+from test_gpu_band import live_model as band_model
 
 pytestmark = pytest.mark.gpu
 
@@ -231,3 +232,27 @@ def test_ensemble_random_masks_match_oracle_and_mixed():
                            f"f32 domain {d} {n}")
         single.release()
     ens.release()
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("metrics", ["row", "point"])
+@pytest.mark.parametrize("sizes", [((3, 3), (40, 33), (130, 61)), ((61, 64), (700, 620)),
+                                   ((57, 4), (1101, 1400)), ((2501, 2403),)],
+                         ids=["one", "two", "more", "largest"])
+def test_ensemble_default_tiles_equal_the_persistent_kernel(sizes, metrics, precision):
+    """The default shape, whose tiles follow the ensemble's size, has the bits
+    of the persistent kernel with its separate Flather launch, on random masks
+    and metrics."""
+    print("default tiles", sizes, metrics, precision, flush=True)
+    models = [band_model(nx, ny, metrics, seed=20 + k) for k, (nx, ny) in enumerate(sizes)]
+    out = []
+    for persistent in (False, True):
+        ens = EnsembleStepper(models, precision=precision)
+        if persistent:
+            ens.set_shape([s[2] > 0 for s in ens.shapes()].index(True))
+        ens.run(3)
+        out.append([{n: ens.fetch(d, n) for n in FIELDS} for d in range(len(models))])
+        ens.release()
+    for d in range(len(models)):
+        for n in FIELDS:
+            assert_bitwise(out[0][d][n], out[1][d][n], f"domain {d} {n}")
