@@ -79,22 +79,29 @@ void launch_conv(hipStream_t s, int cin, int cout, Epilogue epi, const ConvArgs 
 // wavefronts). Both give the same bits.
 void set_conv_form(int form);
 int conv_form();
-// dW partial sums: partial[block][TAPS][co][ci] over the pixels of each of
-// the dw_blocks(nx, ny) workgroups
+// Gradient partial sums of a layer: partial[block][TAPS * co * ci + co], the
+// weights' [TAPS][co][ci] and the biases', over the pixels of each of the
+// dw_blocks(nx, ny) workgroups. The unused rows (output channels from 4) and
+// columns (input channels from IN0C) of the narrow layers are not written.
 int dw_blocks(int nx, int ny);
 void launch_dw(hipStream_t s, int co, int ci, const __bf16 *dpre, const __bf16 *in,
                float *partial, int nx, int ny);
-int bias_blocks();
-void launch_bias_partial(hipStream_t s, int co, const __bf16 *dpre, float *partial,
-                         int nx, int ny);
-// out[i] = sum over b < nblk of partial[b*n + i]
-void launch_reduce(hipStream_t s, const float *partial, int nblk, int n, float *out);
+// grads = the sums of every layer's nblk partials, and sums of squares of
+// the gradient (grad_squares() values) for its norm
+int grad_squares();
+void launch_reduce(hipStream_t s, float *const *partial, int nblk, float *grads, float *square);
+// The bf16 copies of every layer's weights (launch_weights_bf16).
+struct WeightCopies {
+    __bf16 *fwd[NLAYER], *flip[NLAYER];
+};
 // Adam (kind 1) or SGD with momentum (kind 0) over the FP32 master params,
 // the gradient first scaled to a global norm of at most max_norm (if > 0);
-// norm_scale (2 floats, device) receives the gradient norm and that factor
+// norm_scale (2 floats, device) receives the gradient norm (from square, see
+// launch_reduce) and that factor; the weights' bf16 copies follow
 void launch_optimizer(hipStream_t s, int kind, float *w, const float *g, float *m,
-                      float *v, int n, float lr, float b1, float b2, float eps,
-                      float bc1, float bc2, float max_norm, float *norm_scale);
+                      float *v, float lr, float b1, float b2, float eps, float bc1, float bc2,
+                      const float *square, float max_norm, float *norm_scale,
+                      const WeightCopies &copies);
 // bf16 weights of layer l: forward [TAPS][cout][cin] and the flipped,
 // transposed copy for the input-gradient convolution [TAPS][cin][cout]
 void launch_weights_bf16(hipStream_t s, const float *w, int cin, int cout,

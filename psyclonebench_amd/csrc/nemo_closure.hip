@@ -13,8 +13,8 @@
 //
 // Weight gradient: dW[tap][co][ci] = sum_px dPre[px][co] * X[px + tap][ci],
 // a GEMM whose reduction runs over pixels, on v_mfma_f32_16x16x32_bf16 with
-// its operands staged pixel-fastest in LDS (k_dw); every workgroup sums its
-// pixels into a partial dW, and a second pass adds the partials in a fixed
+// its operands read from LDS by transposing loads (k_dw); every workgroup sums
+// its pixels into a partial dW, and a second pass adds the partials in a fixed
 // order.
 #include <cmath>
 #include <type_traits>
@@ -650,230 +650,268 @@ dim3 out_grid(int nx, int ny)
     return dim3((unsigned)(8 * ((per_xcd + 3) / 4)));
 }
 
-// Weight gradient, dW[tap][co][ci] = sum over pixels of dPre[px][co] *
-// X[px + tap][ci]: a GEMM whose K runs over pixels, on
-// v_mfma_f32_16x16x32_bf16 (16 co x 16 ci x 32 pixels). Its operands want 8
-// consecutive pixels of one channel per lane, while the activations store
-// channels fastest, so a workgroup stages them in LDS transposed ([channel]
-// [pixel]) as it marches down a 32-pixel column strip: per output row one
-// dPre row and one new input row, the input rows in a ring of the 5 kernel
-// rows. Each input row is staged at 4 pixel shifts so that the fragment of
-// every horizontal tap is an aligned read (dx 0..3: 16 bytes from shift dx;
-// dx 4: two 8-byte reads from shift 0). Wave w accumulates the taps w, w+4,
-// ...; the global loads of the row DW_PF rows ahead are in flight during
-// the current row's MFMAs. Every workgroup writes its partial dW; k_reduce adds the partials
-// in a fixed order. CI == CIN0 is layer 0: its input is the IN0C-channel
-// network input, and staged channels IN0C..15 stay zero.
-constexpr int DW_LEN = 40;  // staged pixels per row and shift (36 used)
-constexpr int DW_PF = 4;    // rows whose global loads are in flight
+// Weight and bias gradients of one layer: dW[tap][co][ci] = sum over pixels of
+// dPre[px][co] * X[px + tap][ci], db[co] = sum of dPre[px][co]: a GEMM whose K
+// runs over pixels, on v_mfma_f32_16x16x32_bf16 (16 x 16 x 32 pixels). Its
+// operands want 8 consecutive pixels of one channel per lane, while the
+// activations store channels fastest. They are staged in LDS as they are and
+// read with the transposing LDS load (ds_read_b64_tr_b16: 16 lanes read 4
+// pixels x 16 channels, lane i gets channel i of the 4 pixels), so that the
+// tap's shift is a pixel offset of the read.
+//
+// A workgroup has two teams of four wavefronts; each marches down its own
+// rows of a 32-pixel column strip, staging DW_G rows at a time into one of
+// two buffers while the next rows' global loads are in flight: one barrier
+// for DW_G rows. A wavefront owns a 16 x 16 block of (co, ci) for all taps
+// (100 accumulator registers): it reads every dPre row once into a window of
+// five, every X row at five shifts, and runs 25 MFMAs on them.
+//
+// The narrow layers fill the other dimension of the 16 x 16 block with taps,
+// again through the addresses of the read: the network input (4 stored
+// channels a pixel) with the columns (dx, ci), four shifts in one fragment;
+// the output layer (4 used channels) with the rows (dy, co), from four dPre
+// rows. That leaves 5 MFMAs a row and wavefront. Block rows and columns that
+// stand for dy or dx beyond 4 are computed from whatever is in LDS and left
+// out. Rows outside a team's range are staged as zeros.
+//
+// Team 1 hands its sums to team 0 through LDS, which writes one partial per
+// workgroup (about one workgroup a CU: the partials, 100 KB each, are traffic
+// too). Measured at 512^2 against operands transposed by scalar LDS stores at
+// four shifts, with the bias sums in launches of their own (7.8 us each):
+// 32 -> 32 channels 39.4 -> 20.0 us (671 TFLOP/s), output layer 33.6 -> 10.7,
+// network input 22.5 -> 12.0. The narrow layers are bound by their loads and
+// partials. The skipped rows branch on wavefront-uniform conditions; a second
+// copy of the loop without them spilled registers.
+constexpr int DW_G = 5;           // rows staged together: the window of dPre rows
+constexpr int DW_MIN_ROWS = 6;    // of a team: with the 4 halo rows, two groups
+
+__device__ __forceinline__ bf16x4 lds_transposed(const char *p)
+{
+    typedef __attribute__((ext_vector_type(4))) short s16x4;
+    typedef __attribute__((address_space(3))) s16x4 *lds_ptr;
+    return __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)p));
+}
 
 template <int CO, int CI>
-__global__ __launch_bounds__(256) void k_dw(const __bf16 *__restrict__ dpre,
-                                            const __bf16 *__restrict__ in,
-                                            float *__restrict__ partial, int nx, int ny,
-                                            int rows_per_block)
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_dw(
+    const __bf16 *__restrict__ dpre, const __bf16 *__restrict__ in, float *__restrict__ partial,
+    int nx, int ny, int team_rows)
 {
-    constexpr int MB = CO / 16, NB = CI / 16, MAXT = 7;
-    constexpr bool NET_IN = CI == CIN0;
-    constexpr int XQ = NET_IN ? 36 : 36 * (CI / 8);  // 16-byte (8-byte) chunks of an input row
-    constexpr int DQ = 32 * (CO / 8);                // 16-byte chunks of a dPre row
-    static_assert(XQ <= 256 && DQ <= 256, "one chunk per thread");
-    __shared__ __attribute__((aligned(16))) __bf16 xs[5][4][CI][DW_LEN];
-    __shared__ __attribute__((aligned(16))) __bf16 dsh[CO][32];
-    const int tid = (int)threadIdx.x, lane = tid & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n16 = lane & 15, kg = (lane >> 4) * 8;
+    constexpr bool NET_IN = CI == CIN0, NET_OUT = CO == COUT4;
+    static_assert((CO == HID || NET_OUT) && (CI == HID || NET_IN) && !(NET_IN && NET_OUT),
+                  "one narrow dimension at most");
+    constexpr int NA = NET_OUT ? 1 : 5, NB = NET_IN ? 1 : 5;
+    // staged rows in bytes: X 2 planes of 36 pixels x 16 channels (network
+    // input: 40 pixels x 4 channels, 36 of them filled), dPre 2 planes of 32
+    // pixels x 16 channels (output layer: 32 pixels x 4 channels)
+    constexpr int XROW = NET_IN ? 320 : 2304, DROW = NET_OUT ? 256 : 2048;
+    // groups of rows kept: 2 buffers; the output layer reads dPre rows back to
+    // r - 4 from LDS: 3
+    constexpr int XBUF = 2 * DW_G * XROW, DG = NET_OUT ? 3 : 2, TEAM = XBUF + DG * DW_G * DROW;
+    // chunks a group stages: 16 bytes (output layer's dPre: 8 bytes)
+    constexpr int XC = NET_IN ? 18 : 144, DC = NET_OUT ? 32 : 128;  // a row
+    constexpr int XN = DW_G * XC, DN = DW_G * DC, XR = (XN + 255) / 256, DR = (DN + 255) / 256;
+    constexpr int EXCHANGE = NB * 4 * 64 * (int)sizeof(f32x4);
+    static_assert(2 * TEAM >= EXCHANGE, "the exchange reuses the stage");
+    __shared__ __attribute__((aligned(16))) char lds[2 * TEAM];
+
+    const int lane = (int)threadIdx.x & 63, tid = (int)threadIdx.x & 255;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int team = wave >> 2, w = wave & 3;
+    const int mb = w & 1, nb = w >> 1;  // co half, ci half; a narrow layer: tap tile
     const int Wp = nx + 4, nstrip = nx >> 5;
     const size_t PL = plane_elems(nx, ny);
     const int strip = (int)blockIdx.x % nstrip, chunk = (int)blockIdx.x / nstrip;
-    const int x0 = strip * 32, ya = chunk * rows_per_block;
-    const int yb = min(ya + rows_per_block, ny);
+    const int x0 = strip * 32;
+    const int ya = (chunk * 2 + team) * team_rows, yb = min(ya + team_rows, ny);
+    const int groups = (team_rows + 4 + DW_G - 1) / DW_G;
+    char *const xs = lds + team * TEAM, *const ds = xs + XBUF;
 
-    if constexpr (NET_IN) {
-        // channels IN0C..15 are never staged: zero them once
-        bf16x8 *z = reinterpret_cast<bf16x8 *>(&xs[0][0][0][0]);
-        for (int q = tid; q < (int)(sizeof(xs) / 16); q += 256) z[q] = bf16x8{};
+    if constexpr (NET_OUT) {  // the rows before the first
+        for (int q = tid; q < DG * DW_G * DROW / 16; q += 256)
+            reinterpret_cast<bf16x8 *>(ds)[q] = bf16x8{};
         __syncthreads();
     }
 
-    auto load_x = [&](int r, bf16x8 &xr) __attribute__((always_inline)) {  // padded input row r
-        if (tid < XQ) {
-            if constexpr (NET_IN) {
-                const bf16x4 v =
-                    *reinterpret_cast<const bf16x4 *>(in + ((size_t)r * Wp + x0 + tid) * IN0C);
-                xr = __builtin_shufflevector(v, bf16x4{}, 0, 1, 2, 3, 4, 5, 6, 7);
+    bf16x8 xr[XR];
+    std::conditional_t<NET_OUT, bf16x4, bf16x8> dr[DR];
+    auto load = [&](int r0) __attribute__((always_inline)) {  // rows r0 .. r0 + DW_G - 1
+#pragma unroll
+        for (int k = 0; k < XR; k++) {
+            const int c = tid + 256 * k, row = c / XC, q = c - row * XC;
+            if (c < XN) {
+                const size_t px = (size_t)min(r0 + row, ny + 3) * Wp + x0;  // padded row
+                if constexpr (NET_IN)
+                    xr[k] = *reinterpret_cast<const bf16x8 *>(in + px * IN0C + q * 8);
+                else
+                    xr[k] = *reinterpret_cast<const bf16x8 *>(in + (size_t)(q / 72) * PL +
+                                                              px * 16 + (q % 72) * 8);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < DR; k++) {
+            const int c = tid + 256 * k, row = c / DC, q = c - row * DC, y = r0 + row;
+            dr[k] = {};
+            if (c < DN && y < yb) {  // interior row
+                const size_t px = pad_index(y, x0, nx) * 16;
+                if constexpr (NET_OUT)
+                    dr[k] = *reinterpret_cast<const bf16x4 *>(dpre + px + q * 16);
+                else
+                    dr[k] = *reinterpret_cast<const bf16x8 *>(dpre + (size_t)(q >> 6) * PL + px +
+                                                              (q & 63) * 8);
+            }
+        }
+    };
+    auto stage = [&](int g) __attribute__((always_inline)) {
+        char *const x = xs + (g & 1) * DW_G * XROW, *const d = ds + (g % DG) * DW_G * DROW;
+#pragma unroll
+        for (int k = 0; k < XR; k++) {
+            const int c = tid + 256 * k, row = c / XC, q = c - row * XC;
+            if (c < XN) *reinterpret_cast<bf16x8 *>(x + row * XROW + q * 16) = xr[k];
+        }
+#pragma unroll
+        for (int k = 0; k < DR; k++) {
+            const int c = tid + 256 * k;
+            if (c < DN) *reinterpret_cast<decltype(&dr[0])>(d + c * (int)sizeof(dr[0])) = dr[k];
+        }
+    };
+
+    // this lane's part of a transposed read: pixel, 4-channel chunk
+    const int px = (lane >> 4) * 8 + ((lane & 15) >> 2), c4 = lane & 3;
+    auto fragment = [&](const char *p, int px_bytes) __attribute__((always_inline)) {
+        const bf16x4 lo = lds_transposed(p), hi = lds_transposed(p + 4 * px_bytes);
+        return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+    f32x4 acc[NA][NB], acc_b = {};
+#pragma unroll
+    for (int a = 0; a < NA; a++)
+#pragma unroll
+        for (int b = 0; b < NB; b++) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const __bf16 one = (__bf16)1.0f;
+    const bf16x8 ones = {one, one, one, one, one, one, one, one};
+    bf16x8 A[DW_G] = {};  // dPre rows, row r in A[(r - ya) % 5]; output layer: A[0]
+
+    // the rows of group g
+    auto compute = [&](int g) __attribute__((always_inline)) {
+        const int r0 = ya + g * DW_G;
+        const char *const x = xs + (g & 1) * DW_G * XROW +
+                              (NET_IN ? (px + 4 * nb + c4) * 8 : (nb * 36 + px) * 32 + c4 * 8);
+        const char *const d = ds + (g & 1) * DW_G * DROW + (mb * 32 + px) * 32 + c4 * 8;
+        // the fragments of row u, read one row ahead of their MFMAs
+        bf16x8 B[2][NB], An[2];
+        auto read = [&](int u) __attribute__((always_inline)) {
+            if constexpr (NET_OUT) {  // rows (dy, co), dy = 4 mb + c4
+                int row = (g % DG) * DW_G + u - (4 * mb + c4);
+                row += row < 0 ? DG * DW_G : 0;
+                An[u & 1] = fragment(ds + row * DROW + px * 8, 8);
             } else {
-                const int p = tid / (CI / 8), c8 = tid - p * (CI / 8);
-                xr = *reinterpret_cast<const bf16x8 *>(
-                    in + (size_t)(c8 >> 1) * PL + ((size_t)r * Wp + x0 + p) * 16 + (c8 & 1) * 8);
+                An[u & 1] = fragment(d + u * DROW, 32);
+            }
+#pragma unroll
+            for (int b = 0; b < NB; b++)
+                B[u & 1][b] = fragment(x + u * XROW + b * 32, NET_IN ? 8 : 32);
+        };
+        read(0);
+#pragma unroll
+        for (int u = 0; u < DW_G; u++) {
+            A[NET_OUT ? 0 : u] = An[u & 1];
+            if (u + 1 < DW_G) read(u + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            if (NET_OUT ? w == 0 : nb == 0)
+                acc_b = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[NET_OUT ? 0 : u], ones, acc_b,
+                                                                0, 0, 0);
+#pragma unroll
+            for (int a = 0; a < NA; a++) {
+                const int y = r0 + u - a;
+                if (!NET_OUT && (y < ya || y >= yb)) continue;  // wavefront-uniform
+#pragma unroll
+                for (int b = 0; b < NB; b++)
+                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        A[NET_OUT ? 0 : (u + DW_G - a) % DW_G], B[u & 1][b], acc[a][b], 0, 0, 0);
             }
         }
     };
-    auto store_x = [&](int r, const bf16x8 &xr) __attribute__((always_inline)) {
-        if (tid < XQ) {
-            const int slot = r % 5;
-            const int p = NET_IN ? tid : tid / (CI / 8);
-            const int cb = NET_IN ? 0 : (tid - p * (CI / 8)) * 8;
-            constexpr int NCH = NET_IN ? IN0C : 8;
-#pragma unroll
-            for (int s = 0; s < 4; s++) {
-                const int j = p - s;
-                if (j >= 0) {
-#pragma unroll
-                    for (int k = 0; k < NCH; k++) xs[slot][s][cb + k][j] = xr[k];
-                }
-            }
-        }
-    };
-    auto load_d = [&](int y, bf16x8 &dr) __attribute__((always_inline)) {  // interior row y
-        if (tid < DQ) {
-            const int p = tid / (CO / 8), c8 = tid - p * (CO / 8);
-            dr = *reinterpret_cast<const bf16x8 *>(
-                dpre + (size_t)(c8 >> 1) * PL + pad_index(y, x0 + p, nx) * 16 + (c8 & 1) * 8);
-        }
-    };
-    auto store_d = [&](const bf16x8 &dr) __attribute__((always_inline)) {
-        if (tid < DQ) {
-            const int p = tid / (CO / 8), cb = (tid - p * (CO / 8)) * 8;
-#pragma unroll
-            for (int k = 0; k < 8; k++) dsh[cb + k][p] = dr[k];
-        }
-    };
-
-    f32x4 acc[MAXT][MB][NB];
-#pragma unroll
-    for (int t = 0; t < MAXT; t++)
-#pragma unroll
-        for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-            for (int nb = 0; nb < NB; nb++) acc[t][mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    // the ring holds padded input rows y .. y+4 while output row y is reduced;
-    // registers xr[u] / dr[u] hold the rows that arrive DW_PF rows later
-    for (int r = ya; r < ya + 4; r++) {
-        bf16x8 xr = {};
-        load_x(r, xr);
-        store_x(r, xr);
+    load(ya);
+    for (int g = 0; g < groups; g++) {
+        stage(g);
+        __syncthreads();
+        if (g + 1 < groups) load(ya + (g + 1) * DW_G);
+        compute(g);
     }
-    bf16x8 xr[DW_PF], dr[DW_PF];
+
+    // team 1's sums to team 0, and out
+    constexpr int PSIZE = TAPS * CO * CI + CO;
+    float *const out = partial + (size_t)blockIdx.x * PSIZE;
+    f32x4 *const ex = reinterpret_cast<f32x4 *>(lds);
+    const int n16 = lane & 15, m4 = (lane >> 4) * 4;
 #pragma unroll
-    for (int u = 0; u < DW_PF; u++) {
-        xr[u] = bf16x8{};
-        dr[u] = bf16x8{};
-        if (ya + u < yb) {
-            load_x(ya + 4 + u, xr[u]);
-            load_d(ya + u, dr[u]);
-        }
-    }
-    for (int y0 = ya; y0 < yb; y0 += DW_PF) {
+    for (int a = 0; a < NA; a++) {
+        __syncthreads();
+        if (team == 1)
 #pragma unroll
-        for (int u = 0; u < DW_PF; u++) {
-            const int y = y0 + u;
-            if (y < yb) {  // workgroup-uniform
-                store_x(y + 4, xr[u]);
-                store_d(dr[u]);
-                __syncthreads();
-                if (y + DW_PF < yb) {
-                    load_x(y + 4 + DW_PF, xr[u]);
-                    load_d(y + DW_PF, dr[u]);
-                }
-                bf16x8 A[MB];
+            for (int b = 0; b < NB; b++) ex[(b * 4 + w) * 64 + lane] = acc[a][b];
+        __syncthreads();
+        if (team == 0)
 #pragma unroll
-                for (int mb = 0; mb < MB; mb++)
-                    A[mb] = *reinterpret_cast<const bf16x8 *>(&dsh[mb * 16 + n16][kg]);
+            for (int b = 0; b < NB; b++) {
+                const f32x4 v = acc[a][b] + ex[(b * 4 + w) * 64 + lane];
 #pragma unroll
-                for (int t = 0; t < MAXT; t++) {
-                    const int tap = wv + 4 * t;
-                    if (tap < TAPS) {  // wavefront-uniform
-                        const int dy = tap / 5, dx = tap - 5 * (tap / 5);
-                        const int slot = (y + dy) % 5;
-#pragma unroll
-                        for (int nb = 0; nb < NB; nb++) {
-                            bf16x8 B;
-                            if (dx < 4) {
-                                B = *reinterpret_cast<const bf16x8 *>(
-                                    &xs[slot][dx][nb * 16 + n16][kg]);
-                            } else {
-                                const bf16x4 lo = *reinterpret_cast<const bf16x4 *>(
-                                    &xs[slot][0][nb * 16 + n16][4 + kg]);
-                                const bf16x4 hi = *reinterpret_cast<const bf16x4 *>(
-                                    &xs[slot][0][nb * 16 + n16][8 + kg]);
-                                B = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-                            }
-#pragma unroll
-                            for (int mb = 0; mb < MB; mb++)
-                                acc[t][mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                                    A[mb], B, acc[t][mb][nb], 0, 0, 0);
-                        }
+                for (int r = 0; r < 4; r++) {
+                    const int m = m4 + r;
+                    int dy = a, dx = b, co = mb * 16 + m, ci = nb * 16 + n16;
+                    if constexpr (NET_IN) {
+                        dx = 4 * nb + n16 / 4;
+                        ci = n16 % 4;
                     }
-                }
-                __syncthreads();
-            }
-        }
-    }
-    float *out = partial + (size_t)blockIdx.x * TAPS * CO * CI;
-#pragma unroll
-    for (int t = 0; t < MAXT; t++) {
-        const int tap = wv + 4 * t;
-        if (tap < TAPS) {
-#pragma unroll
-            for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-                for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const int co = mb * 16 + (lane >> 4) * 4 + r;
-                        out[((size_t)tap * CO + co) * CI + nb * 16 + n16] = acc[t][mb][nb][r];
+                    if constexpr (NET_OUT) {
+                        dy = 4 * mb + m / 4;
+                        co = m % 4;
                     }
-        }
+                    if (dy < 5 && dx < 5) out[((size_t)(dy * 5 + dx) * CO + co) * CI + ci] = v[r];
+                }
+            }
     }
-}
-
-// Partial bias gradient: per channel, the sum over this workgroup's pixels of
-// dPre. A thread reads one 16-byte chunk (8 channels of one pixel) per
-// iteration, CO / 8 chunks a pixel, so a wavefront's loads cover contiguous
-// pixels of each plane; the sums of the threads that share a chunk are added
-// in LDS in a fixed order.
-template <int CO>
-__global__ __launch_bounds__(256) void k_bias_partial(const __bf16 *__restrict__ dpre,
-                                                      float *__restrict__ partial, int nx,
-                                                      int ny)
-{
-    constexpr int NCH = CO / 8;     // chunks per pixel
-    constexpr int PPI = 256 / NCH;  // pixels per workgroup and iteration
-    __shared__ float red[256][9];
-    const int ch = (int)threadIdx.x % NCH, q = (int)threadIdx.x / NCH;
-    const size_t coff = (size_t)(ch >> 1) * plane_elems(nx, ny) + (size_t)(ch & 1) * 8;
-    const int npx = nx * ny;
-    float s[8] = {};
-#pragma unroll 4
-    for (int p = (int)blockIdx.x * PPI + q; p < npx; p += (int)gridDim.x * PPI) {
-        const int y = p / nx, x = p - y * nx;
-        const bf16x8 v = *reinterpret_cast<const bf16x8 *>(dpre + coff + pad_index(y, x, nx) * 16);
-#pragma unroll
-        for (int k = 0; k < 8; k++) s[k] += (float)v[k];
-    }
-#pragma unroll
-    for (int k = 0; k < 8; k++) red[threadIdx.x][k] = s[k];
     __syncthreads();
-    if ((int)threadIdx.x < CO) {
-        const int c = (int)threadIdx.x, chunk = c >> 3, k = c & 7;
-        float t = 0.0f;
-        for (int qq = 0; qq < PPI; qq++) t += red[qq * NCH + chunk][k];
-        partial[(size_t)blockIdx.x * CO + c] = t;
+    if (team == 1) ex[w * 64 + lane] = acc_b;
+    __syncthreads();
+    if (team == 0 && n16 == 0 && (NET_OUT ? w == 0 && m4 == 0 : nb == 0)) {
+        const f32x4 v = acc_b + ex[w * 64 + lane];
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            out[TAPS * CO * CI + (NET_OUT ? r : mb * 16 + m4 + r)] = v[r];
     }
 }
 
-// out[i] = sum over the nblk partials: a workgroup owns 64 consecutive
-// outputs, its wavefront w sums the w-th quarter of the partials (64-lane
-// coalesced rows, 8 loads in flight), and the 4 quarter sums are added in
-// order, so the result does not depend on timing.
-__global__ __launch_bounds__(256) void k_reduce(const float *__restrict__ partial, int nblk,
-                                                int n, float *__restrict__ out)
+// Gradients of every layer from the partials of k_dw, in one launch: a
+// workgroup owns 64 consecutive values of a layer, its wavefront w sums the
+// w-th quarter of the partials (64-lane coalesced rows, 8 loads in flight),
+// and the 4 quarter sums are added in order, so the result does not depend on
+// timing. The workgroup's sum of squares goes to square[workgroup], for the
+// norm. At 512^2 13.8 us (77 MB of partials), against 51 us in eight launches
+// and 8 us of a launch for the norm.
+struct GradPartials {
+    const float *partial[NLAYER];
+};
+constexpr int reduce_blocks(int l) { return (layer_psize(l) + 63) / 64; }
+constexpr int reduce_first(int l) { return l == 0 ? 0 : reduce_first(l - 1) + reduce_blocks(l - 1); }
+
+__global__ __launch_bounds__(256) void k_reduce(GradPartials p, int nblk,
+                                                float *__restrict__ grads,
+                                                float *__restrict__ square)
 {
     __shared__ float red[4][64];
     const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
-    const int i = (int)blockIdx.x * 64 + lane;
+    int first = 0, n = layer_psize(0), off = 0;
+    const float *partial = p.partial[0];
+#pragma unroll
+    for (int l = 1; l < NLAYER; l++)
+        if ((int)blockIdx.x >= reduce_first(l)) {
+            first = reduce_first(l);
+            n = layer_psize(l);
+            off = layer_offset(l);
+            partial = p.partial[l];
+        }
+    const int i = ((int)blockIdx.x - first) * 64 + lane;
     const int q = (nblk + 3) / 4, b0 = w * q, b1 = min(b0 + q, nblk);
     float s = 0.0f;
     if (i < n) {
@@ -882,55 +920,79 @@ __global__ __launch_bounds__(256) void k_reduce(const float *__restrict__ partia
     }
     red[w][lane] = s;
     __syncthreads();
-    if (w == 0 && i < n) out[i] = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
+    if (w != 0) return;
+    const float g = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
+    if (i < n) grads[off + i] = g;
+    float sq = i < n ? g * g : 0.0f;
+    for (int k = 32; k > 0; k >>= 1) sq += __shfl_xor(sq, k);
+    if (lane == 0) square[blockIdx.x] = sq;
 }
 
-// Global gradient norm, and the factor that scales it down to max_norm
-// (1 when max_norm <= 0 or the norm is below it): norm_scale = {norm, factor}.
-// One workgroup of 1024 threads, 8 loads in flight per thread, then a tree
-// in LDS: a fixed order, and a few memory latencies for the ~77K values.
-__global__ __launch_bounds__(1024) void k_grad_norm(const float *__restrict__ g, int n,
-                                                    float max_norm,
-                                                    float *__restrict__ norm_scale)
+// bf16 copies of one weight: forward [tap][cout][cin] and the flipped,
+// transposed one of the input-gradient convolution.
+__device__ __forceinline__ void store_bf16(int i, int cin, int cout, float v, __bf16 *fwd,
+                                           __bf16 *flip)
 {
-    __shared__ float red[1024];
+    const int tap = i / (cin * cout), r = i - tap * cin * cout;
+    const int co = r / cin, ci = r - co * cin;
+    const __bf16 b = (__bf16)v;
+    fwd[i] = b;
+    if (flip) flip[((size_t)(TAPS - 1 - tap) * cin + ci) * cout + co] = b;
+}
+
+// Global gradient norm and the factor that scales it down to max_norm (1 when
+// max_norm <= 0 or the norm is below it), norm_scale = {norm, factor}; the
+// update of the FP32 parameters; their bf16 copies. Every workgroup adds the
+// nsq sums of squares itself, in the same order (a few loads a thread and a
+// tree in LDS), which costs less than a launch between.
+__global__ __launch_bounds__(256) void k_optimizer(int kind, float *__restrict__ w,
+                                                   const float *__restrict__ g,
+                                                   float *__restrict__ m, float *__restrict__ v,
+                                                   float lr, float b1, float b2, float eps,
+                                                   float bc1, float bc2,
+                                                   const float *__restrict__ square, int nsq,
+                                                   float max_norm, float *__restrict__ norm_scale,
+                                                   WeightCopies copies)
+{
+    __shared__ float red[256];
     float s = 0.0f;
 #pragma unroll 8
-    for (int i = (int)threadIdx.x; i < n; i += 1024) s += g[i] * g[i];
+    for (int i = (int)threadIdx.x; i < nsq; i += 256) s += square[i];
     red[threadIdx.x] = s;
     __syncthreads();
-    for (int k = 512; k > 0; k >>= 1) {
+    for (int k = 128; k > 0; k >>= 1) {
         if ((int)threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        const float nrm = sqrtf(red[0]);
-        norm_scale[0] = nrm;
-        // a non-finite gradient skips the update
-        norm_scale[1] = !isfinite(nrm) ? 0.0f
-                        : (max_norm > 0.0f && nrm > max_norm) ? max_norm / nrm : 1.0f;
-    }
-}
-
-__global__ void k_optimizer(int kind, float *__restrict__ w, const float *__restrict__ g,
-                            float *__restrict__ m, float *__restrict__ v, int n, float lr,
-                            float b1, float b2, float eps, float bc1, float bc2,
-                            const float *__restrict__ norm_scale)
-{
+    const float nrm = sqrtf(red[0]);
+    // a non-finite gradient skips the update
+    const float factor = !isfinite(nrm) ? 0.0f
+                         : (max_norm > 0.0f && nrm > max_norm) ? max_norm / nrm : 1.0f;
     const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (i >= n) return;
-    if (norm_scale[1] == 0.0f) return;  // non-finite gradient: no update
-    const float gi = g[i] * norm_scale[1];
+    if (i == 0) {
+        norm_scale[0] = nrm;
+        norm_scale[1] = factor;
+    }
+    if (i >= param_count() || factor == 0.0f) return;
+    const float gi = g[i] * factor;
+    float wi;
     if (kind == 1) {  // Adam
         const float mi = b1 * m[i] + (1.0f - b1) * gi;
         const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
         m[i] = mi;
         v[i] = vi;
-        w[i] -= lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
+        wi = w[i] - lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
     } else {          // SGD with momentum b1
         const float mi = b1 * m[i] + gi;
         m[i] = mi;
-        w[i] -= lr * mi;
+        wi = w[i] - lr * mi;
+    }
+    w[i] = wi;
+#pragma unroll
+    for (int l = 0; l < NLAYER; l++) {
+        const int k = i - layer_offset(l);
+        if (k >= 0 && k < layer_wsize(l))
+            store_bf16(k, layer_cin(l), layer_cout(l), wi, copies.fwd[l], copies.flip[l]);
     }
 }
 
@@ -938,13 +1000,7 @@ __global__ void k_weights_bf16(const float *__restrict__ w, int cin, int cout,
                                __bf16 *__restrict__ fwd, __bf16 *__restrict__ flip)
 {
     const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    const int n = TAPS * cin * cout;
-    if (i >= n) return;
-    const int tap = i / (cin * cout), r = i - tap * cin * cout;
-    const int co = r / cin, ci = r - co * cin;
-    const __bf16 b = (__bf16)w[i];
-    fwd[i] = b;
-    if (flip) flip[((size_t)(TAPS - 1 - tap) * cin + ci) * cout + co] = b;
+    if (i < TAPS * cin * cout) store_bf16(i, cin, cout, w[i], fwd, flip);
 }
 
 __global__ void k_pack(CoarseState c, Norm nm, __bf16 *__restrict__ in0,
@@ -1206,19 +1262,18 @@ void launch_conv(hipStream_t s, int cin, int cout, Epilogue epi, const ConvArgs 
     NEMO_LAUNCH_CHECK();
 }
 
-// dW workgroups: nx / 32 column strips x row chunks, about 512 in all, two
-// per CU (at least 8 rows a chunk, so the 4-row ring fill stays a small
-// overhead)
-static int dw_rows_per_block(int nx, int ny)
+// Rows of a team of k_dw: nx / 32 column strips x row chunks of two teams,
+// about 256 workgroups in all, one per CU.
+static int dw_team_rows(int nx, int ny)
 {
     const long nstrip = nx / 32;
-    return (int)std::max(8L, (ny * nstrip + 511) / 512);
+    return (int)std::max((long)DW_MIN_ROWS, (ny * nstrip + 511) / 512);
 }
 
 int dw_blocks(int nx, int ny)
 {
-    const int rpb = dw_rows_per_block(nx, ny);
-    return (nx / 32) * ((ny + rpb - 1) / rpb);
+    const int rows = 2 * dw_team_rows(nx, ny);
+    return (nx / 32) * ((ny + rows - 1) / rows);
 }
 
 void launch_dw(hipStream_t s, int co, int ci, const __bf16 *dpre, const __bf16 *in,
@@ -1226,48 +1281,37 @@ void launch_dw(hipStream_t s, int co, int ci, const __bf16 *dpre, const __bf16 *
 {
     if (nx % 32 != 0 || nx <= 0 || ny <= 0)
         NEMO_FATAL("closure dW: interior %d x %d (nx a positive multiple of 32)", nx, ny);
-    const int rpb = dw_rows_per_block(nx, ny);
-    const dim3 grid((unsigned)dw_blocks(nx, ny)), block(256);
+    const int rows = dw_team_rows(nx, ny);
+    const dim3 grid((unsigned)dw_blocks(nx, ny)), block(512);
     if (co == 32 && ci == 32)
-        k_dw<32, 32><<<grid, block, 0, s>>>(dpre, in, partial, nx, ny, rpb);
+        k_dw<32, 32><<<grid, block, 0, s>>>(dpre, in, partial, nx, ny, rows);
     else if (co == 32 && ci == 16)
-        k_dw<32, 16><<<grid, block, 0, s>>>(dpre, in, partial, nx, ny, rpb);
+        k_dw<32, 16><<<grid, block, 0, s>>>(dpre, in, partial, nx, ny, rows);
     else if (co == 16 && ci == 32)
-        k_dw<16, 32><<<grid, block, 0, s>>>(dpre, in, partial, nx, ny, rpb);
+        k_dw<16, 32><<<grid, block, 0, s>>>(dpre, in, partial, nx, ny, rows);
     else
         NEMO_FATAL("closure dW: unsupported %d x %d", co, ci);
     NEMO_LAUNCH_CHECK();
 }
 
-int bias_blocks() { return 128; }
+int grad_squares() { return reduce_first(NLAYER); }
 
-void launch_bias_partial(hipStream_t s, int co, const __bf16 *dpre, float *partial,
-                         int nx, int ny)
+void launch_reduce(hipStream_t s, float *const *partial, int nblk, float *grads, float *square)
 {
-    const dim3 grid((unsigned)bias_blocks()), block(256);
-    if (co == 32)
-        k_bias_partial<32><<<grid, block, 0, s>>>(dpre, partial, nx, ny);
-    else if (co == 16)
-        k_bias_partial<16><<<grid, block, 0, s>>>(dpre, partial, nx, ny);
-    else
-        NEMO_FATAL("closure bias gradient: %d channels", co);
-    NEMO_LAUNCH_CHECK();
-}
-
-void launch_reduce(hipStream_t s, const float *partial, int nblk, int n, float *out)
-{
-    k_reduce<<<dim3((unsigned)((n + 63) / 64)), dim3(256), 0, s>>>(partial, nblk, n, out);
+    GradPartials p;
+    for (int l = 0; l < NLAYER; l++) p.partial[l] = partial[l];
+    k_reduce<<<dim3((unsigned)grad_squares()), dim3(256), 0, s>>>(p, nblk, grads, square);
     NEMO_LAUNCH_CHECK();
 }
 
 void launch_optimizer(hipStream_t s, int kind, float *w, const float *g, float *m,
-                      float *v, int n, float lr, float b1, float b2, float eps,
-                      float bc1, float bc2, float max_norm, float *norm_scale)
+                      float *v, float lr, float b1, float b2, float eps, float bc1, float bc2,
+                      const float *square, float max_norm, float *norm_scale,
+                      const WeightCopies &copies)
 {
-    k_grad_norm<<<dim3(1), dim3(1024), 0, s>>>(g, n, max_norm, norm_scale);
-    NEMO_LAUNCH_CHECK();
-    k_optimizer<<<grid_for(n), dim3(256), 0, s>>>(kind, w, g, m, v, n, lr, b1, b2, eps,
-                                                  bc1, bc2, norm_scale);
+    k_optimizer<<<grid_for(param_count()), dim3(256), 0, s>>>(
+        kind, w, g, m, v, lr, b1, b2, eps, bc1, bc2, square, grad_squares(), max_norm,
+        norm_scale, copies);
     NEMO_LAUNCH_CHECK();
 }
 

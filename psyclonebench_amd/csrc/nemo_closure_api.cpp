@@ -27,7 +27,9 @@ struct ClosureContext {
     __bf16 *wf[NLAYER] = {}, *wx[NLAYER] = {};
     __bf16 *in0 = nullptr, *act[NLAYER - 1] = {}, *pre[NLAYER - 1] = {}, *dpre[NLAYER] = {};
     float *pred = nullptr, *target = nullptr, *gate = nullptr;
-    float *dw_partial = nullptr, *b_partial = nullptr, *loss_partial = nullptr;
+    // gradient partials of each layer (their unused elements stay 0) and the
+    // sums of squares of the gradient
+    float *dw_partial[NLAYER] = {}, *square = nullptr, *loss_partial = nullptr;
     double *fssh = nullptr, *fu = nullptr, *fv = nullptr;
     double *guard_partial = nullptr;
     int *flag = nullptr, *trips = nullptr;
@@ -50,8 +52,8 @@ struct ClosureContext {
 
     ~ClosureContext()
     {
-        void *all[] = {params, grads, mom1, mom2, in0, pred, target, dw_partial, b_partial,
-                       loss_partial, fssh, fu, fv, guard_partial, flag, trips, norm_scale,
+        void *all[] = {params, grads, mom1, mom2, in0, pred, target, square, loss_partial,
+                       fssh, fu, fv, guard_partial, flag, trips, norm_scale,
                        gate};
         for (void *p : all)
             if (p) (void)hipFree(p);
@@ -59,6 +61,7 @@ struct ClosureContext {
             if (wf[l]) (void)hipFree(wf[l]);
             if (wx[l]) (void)hipFree(wx[l]);
             if (dpre[l]) (void)hipFree(dpre[l]);
+            if (dw_partial[l]) (void)hipFree(dw_partial[l]);
         }
         for (int l = 0; l < NLAYER - 1; l++) {
             if (act[l]) (void)hipFree(act[l]);
@@ -175,12 +178,7 @@ void backward(ClosureContext &C, hipStream_t s)
     for (int l = NLAYER - 1; l >= 0; l--) {
         const int ci = layer_cin(l), co = layer_cout(l);
         const __bf16 *x = l == 0 ? C.in0 : C.act[l - 1];
-        launch_dw(s, co, ci, C.dpre[l], x, C.dw_partial, C.nx, C.ny);
-        launch_reduce(s, C.dw_partial, dw_blocks(C.nx, C.ny), layer_wsize(l),
-                      C.grads + layer_offset(l));
-        launch_bias_partial(s, co, C.dpre[l], C.b_partial, C.nx, C.ny);
-        launch_reduce(s, C.b_partial, bias_blocks(), co,
-                      C.grads + layer_offset(l) + layer_wsize(l));
+        launch_dw(s, co, ci, C.dpre[l], x, C.dw_partial[l], C.nx, C.ny);
         if (l > 0) {  // gradient of the layer's input, times gelu' of the layer below
             ConvArgs a{};
             a.in = C.dpre[l];
@@ -192,6 +190,7 @@ void backward(ClosureContext &C, hipStream_t s)
             launch_conv(s, co, ci, EPI_DX, a);
         }
     }
+    launch_reduce(s, C.dw_partial, dw_blocks(C.nx, C.ny), C.grads, C.square);
 }
 
 void optimizer_step(ClosureContext &C, hipStream_t s)
@@ -199,9 +198,13 @@ void optimizer_step(ClosureContext &C, hipStream_t s)
     C.step++;
     const float bc1 = 1.0f - std::pow(C.b1, (float)C.step);
     const float bc2 = 1.0f - std::pow(C.b2, (float)C.step);
-    launch_optimizer(s, C.opt_kind, C.params, C.grads, C.mom1, C.mom2, param_count(), C.lr,
-                     C.b1, C.b2, C.eps, bc1, bc2, C.max_norm, C.norm_scale);
-    refresh_bf16(C, s);
+    WeightCopies copies;
+    for (int l = 0; l < NLAYER; l++) {
+        copies.fwd[l] = C.wf[l];
+        copies.flip[l] = C.wx[l];
+    }
+    launch_optimizer(s, C.opt_kind, C.params, C.grads, C.mom1, C.mom2, C.lr, C.b1, C.b2, C.eps,
+                     bc1, bc2, C.square, C.max_norm, C.norm_scale, copies);
 }
 
 // host float -> bf16, round to nearest even (as the device conversion)
@@ -280,8 +283,9 @@ void *nemo_cl_create(int nx, int ny, int coarse_width, int coarse_height,
     C->pred = zeros<float>(npx * 4, s);
     C->gate = zeros<float>(npx, s);
     C->target = zeros<float>(npx * 4, s);
-    C->dw_partial = zeros<float>((size_t)dw_blocks(nx, ny) * TAPS * HID * HID, s);
-    C->b_partial = zeros<float>((size_t)bias_blocks() * HID, s);
+    for (int l = 0; l < NLAYER; l++)
+        C->dw_partial[l] = zeros<float>((size_t)dw_blocks(nx, ny) * layer_psize(l), s);
+    C->square = zeros<float>((size_t)grad_squares(), s);
     C->loss_partial = zeros<float>((size_t)loss_blocks() * 3, s);
     C->norm_scale = zeros<float>(2, s);
     const size_t nc = (size_t)coarse_width * coarse_height;

@@ -131,6 +131,29 @@ def test_gradients_match_oracle(weights):
     net.release()
 
 
+@pytest.mark.parametrize("nx, ny", [(32, 3), (32, 12), (96, 37), (256, 400)])
+def test_gradient_partials_over_sizes(nx, ny):
+    """Weight and bias gradients where the row chunks change: fewer rows than
+    one team takes, an idle second team, a remainder, more than two groups of
+    rows a team. The bound is that of the gradients against the oracle."""
+    print("gradients", nx, ny, flush=True)
+    p = net_params(8)
+    net = ClosureNet(coarse_test_model(nx, ny), params=p)
+    rng = np.random.default_rng(9)
+    x, t = rng.standard_normal((ny, nx, 4)), rng.standard_normal((ny, nx, 3))
+    _, g = net.grad_host(x, t)
+    net.release()
+    _, go = co.loss_and_grad(p.astype(np.float64), x, t, quant=True)
+    offs = layer_offsets()
+    for l, (cin, cout) in enumerate(co.LAYERS):
+        n = 25 * cin * cout
+        for what, sl in (("weights", slice(offs[l], offs[l] + n)),
+                         ("biases", slice(offs[l] + n, offs[l] + n + cout))):
+            e = rel(g[sl], go[sl])
+            print(f"layer {l} {what}: {e:.2e}", flush=True)
+            assert e < GRAD_TOL
+
+
 def test_adam_step_matches_formula():
     m = coarse_test_model(64, 16)
     p = net_params(5)
