@@ -124,10 +124,11 @@ void forward(ClosureContext &C, hipStream_t s, bool training, bool gated, bool t
         a.nx = C.nx;
         a.ny = C.ny;
         if (l < NLAYER - 1) {
-            a.out = C.act[l];
+            __bf16 *const out = C.act[training ? l : l & 1];
+            a.out = out;
             a.pre = training ? C.pre[l] : nullptr;
             launch_conv(s, layer_cin(l), layer_cout(l), EPI_HIDDEN, a);
-            x = C.act[l];
+            x = out;
         } else {
             a.outf = C.pred;
             a.gate = gated ? C.gate : nullptr;
