@@ -28,6 +28,7 @@
 #include "nemo_ensemble.h"
 #include "nemo_hip_common.h"
 #include "nemo_host.h"
+#include "nemo_readback.h"
 #include "nemo_wave.h"
 #include "nemolite2d_hip.h"
 
@@ -70,6 +71,7 @@ struct EnsContext {
     void *prog[2][kProg] = {};
     DeviceFlather fl_u, fl_v;
     int parity = 0;
+    ReadBack reader;
     bool paired = false;
     std::vector<EnsShape> shapes;
     int shape = 0;
@@ -740,25 +742,17 @@ void nemo_ens_read(void *h, int domain, int field, double *out)
     static const int kField[] = {0, 2, 3, 4, 5};  // sshn_t, un, vn, sshn_u, sshn_v
     if (field < 0 || field > 4) NEMO_FATAL("unknown ensemble field %d", field);
     hipStream_t s = lib_stream();
-    NEMO_HIP_CHECK(hipStreamSynchronize(s));
     const size_t n = (size_t)C.geo[domain].total;
     const size_t o = (size_t)C.hdom[domain].off;
     const void *src = C.prog[C.parity][kField[field]];
     if (C.prec == 64) {
+        NEMO_HIP_CHECK(hipStreamSynchronize(s));
         NEMO_HIP_CHECK(hipMemcpy(out, static_cast<const double *>(src) + o,
                                  n * sizeof(double), hipMemcpyDeviceToHost));
         return;
     }
-    std::vector<float> a(n), lo;
-    NEMO_HIP_CHECK(hipMemcpy(a.data(), static_cast<const float *>(src) + o,
-                             n * sizeof(float), hipMemcpyDeviceToHost));
-    if (field == 0) {
-        lo.resize(n);
-        NEMO_HIP_CHECK(hipMemcpy(lo.data(), static_cast<const float *>(C.prog[C.parity][1]) + o,
-                                 n * sizeof(float), hipMemcpyDeviceToHost));
-    }
-    for (size_t k = 0; k < n; k++)
-        out[k] = field == 0 ? (double)a[k] + (double)lo[k] : (double)a[k];
+    const float *lo = field == 0 ? static_cast<const float *>(C.prog[C.parity][1]) + o : nullptr;
+    C.reader.read(s, static_cast<const float *>(src) + o, lo, n, out);
 }
 
 void nemo_ens_destroy(void *h)

@@ -66,6 +66,5 @@ void launch_flather_f32(hipStream_t s, const FlatherList &lu, const FlatherList 
                         const float *su, const float *sv);
 void launch_to_f32(hipStream_t s, const double *src, float *dst, long n);
 void launch_split_f64(hipStream_t s, const double *src, float *hi, float *lo, long n);
-void launch_to_f64(hipStream_t s, const float *src, const float *lo, double *dst, long n);
 
 }  // namespace nemo

@@ -110,14 +110,6 @@ __global__ void k_split_f64(const double *__restrict__ src, float *__restrict__ 
     lo[k] = (float)(s - (double)h);
 }
 
-__global__ void k_to_f64(const float *__restrict__ src, const float *__restrict__ lo,
-                         double *__restrict__ dst, long n)
-{
-    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    dst[k] = lo ? (double)src[k] + (double)lo[k] : (double)src[k];
-}
-
 inline dim3 blocks_for(long n) { return dim3((unsigned)((n + 255) / 256)); }
 
 }  // namespace
@@ -208,12 +200,6 @@ void launch_to_f32(hipStream_t s, const double *src, float *dst, long n)
 void launch_split_f64(hipStream_t s, const double *src, float *hi, float *lo, long n)
 {
     k_split_f64<<<blocks_for(n), dim3(256), 0, s>>>(src, hi, lo, n);
-    NEMO_LAUNCH_CHECK();
-}
-
-void launch_to_f64(hipStream_t s, const float *src, const float *lo, double *dst, long n)
-{
-    k_to_f64<<<blocks_for(n), dim3(256), 0, s>>>(src, lo, dst, n);
     NEMO_LAUNCH_CHECK();
 }
 

@@ -12,6 +12,7 @@
 #include "nemo_hip_common.h"
 #include "nemo_host.h"
 #include "nemo_mixed.h"
+#include "nemo_readback.h"
 #include "nemolite2d_hip.h"
 
 namespace nemo {
@@ -33,6 +34,7 @@ struct MixedContext {
     float *t_hi[2] = {}, *t_lo[2] = {}, *u[2] = {}, *v[2] = {}, *su[2] = {}, *sv[2] = {};
     DeviceFlather fl_u, fl_v;
     int parity = 0;
+    ReadBack reader;
     bool paired = false;
     double *d_tide = nullptr, *h_tide = nullptr;
     int tide_cap = 0;
@@ -353,7 +355,6 @@ void nemo_mp_read(void *h, int field, double *out)
 {
     MixedContext &C = *static_cast<MixedContext *>(h);
     hipStream_t s = lib_stream();
-    NEMO_HIP_CHECK(hipStreamSynchronize(s));
     const int p = C.parity;
     const size_t n = (size_t)C.G.total;
     const float *src = nullptr, *lo = nullptr;
@@ -365,10 +366,7 @@ void nemo_mp_read(void *h, int field, double *out)
     case 4: src = C.sv[p]; break;
     default: NEMO_FATAL("nemo_mp_read: unknown field %d", field);
     }
-    std::vector<float> a(n), b(lo ? n : 0);
-    NEMO_HIP_CHECK(hipMemcpy(a.data(), src, n * sizeof(float), hipMemcpyDeviceToHost));
-    if (lo) NEMO_HIP_CHECK(hipMemcpy(b.data(), lo, n * sizeof(float), hipMemcpyDeviceToHost));
-    for (size_t k = 0; k < n; k++) out[k] = lo ? (double)a[k] + (double)b[k] : (double)a[k];
+    C.reader.read(s, src, lo, n, out);
 }
 
 void nemo_mp_destroy(void *h)

@@ -174,3 +174,22 @@ def test_mixed_random_mask_against_fp64():
         assert rmax <= tol, (n, rmax)
     ref.release()
     mp.release()
+
+
+@pytest.mark.parametrize("nx, ny", [(3, 3), (509, 508), (509, 509), (509, 510), (1400, 1150)])
+def test_read_back_of_the_uploaded_state(nx, ny):
+    """A record read before the first step holds the uploaded values, at one
+    chunk of 2^18 values, a row less and more, and several: the velocities
+    rounded to FP32, ssh as the sum of its two FP32 words."""
+    rng = np.random.default_rng(nx + ny)
+    m = Model(NemoConfig(jpiglo=nx + 2, jpjglo=ny + 2))
+    for n in ("sshn_t", "un", "vn", "sshn_u", "sshn_v"):
+        m.array(n)[:] = rng.uniform(-1, 1, m.array(n).shape)
+    st = MixedStepper(m)
+    for n in ("un", "vn", "sshn_u", "sshn_v"):
+        assert_bitwise(st.fetch(n), m.array(n).astype(np.float32).astype(np.float64), n)
+    s = m.array("sshn_t")
+    hi = s.astype(np.float32)
+    lo = (s - hi.astype(np.float64)).astype(np.float32)
+    assert_bitwise(st.fetch("sshn_t"), hi.astype(np.float64) + lo.astype(np.float64), "sshn_t")
+    st.release()
