@@ -126,6 +126,10 @@ __device__ __forceinline__ void store(T *__restrict__ base, unsigned off, T v)
         *q = v;
 }
 
+// The outputs of a point: its new u, its new v, its new ssh with the face ssh
+// that follow from it. No part needs another's result.
+enum Part { PART_U = 1, PART_V = 2, PART_SSH = 4, ALL_PARTS = 7 };
+
 // Keeps an evaluation where it stands: without it the compiler moves the
 // arithmetic of a face under the branch of its store, one branch a face, and
 // the faces of a row no longer overlap.
@@ -238,17 +242,24 @@ __device__ __forceinline__ void flather_rows(const typename Types<T>::In &f,
 // are register renaming). NEXT: write the new face ssh (false where the step
 // updates the caller's arrays in place and a second kernel follows). STREAM:
 // non-temporal stores. QUICK: uniform_quotient for the row's divisors.
+// PARTS: the outputs this wavefront evaluates and writes (enum Part).
+// tide_of(): the elevation of open cells; one-row bands read it behind their
+// loads.
 // Returns the first row that is not done: jhi (or jlo + R), or with QUICK a
 // row with a numerator outside its range.
-template <typename T, bool ROWM, int R, int PF, bool NEXT, bool STREAM, bool QUICK>
+template <typename T, bool ROWM, int R, int PF, bool NEXT, bool STREAM, bool QUICK, int PARTS,
+          typename Tide>
 __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__restrict__ tab,
                                     const StepScalars<T> &p, const typename Types<T>::Out &o,
                                     const Flather<T> &fl, int W, unsigned base,
                                     const Bounds &b, int ow, int strip, int jlo, int jhi,
-                                    typename Types<T>::Tide tide)
+                                    Tide tide_of)
 {
     constexpr bool MIXED = sizeof(T) == 4;
+    constexpr bool DO_U = PARTS & PART_U, DO_V = PARTS & PART_V, DO_SSH = PARTS & PART_SSH;
     const int l0 = first_lane(ow);
+    typename Types<T>::Tide tide{};
+    if constexpr (DO_SSH && R > 1) tide = tide_of();
     constexpr bool SHORT = R <= 2;  // Flather faces from the registers
     static_assert(PF >= 0 && PF <= 2 && R >= 1 && R <= 16, "unrolled band");
     using S = typename Types<T>::NewSsh;
@@ -330,6 +341,21 @@ __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__r
             return divide(a, p.fric);
     };
 
+    // One-row bands, whose time is their latency, issue the loads of all three
+    // rows at once, and touch the lines of the row records so that the reads
+    // that follow find them in the scalar cache (FP32 128^2 2.97 -> 2.75 us a
+    // step, 256^2 3.61 -> 3.36; FP64 without the table 48^2 3.5 -> 3.3). FP64
+    // with the table is better off with the last row's loads behind the first
+    // arithmetic (181^2 4.28 against 4.50).
+    constexpr bool TOGETHER = PF == 0 && R == 1 && (MIXED || !ROWM);
+    constexpr int LINES = ROW_WIDTH * (int)sizeof(T) / 64;  // of a record
+    unsigned warm[3 * LINES] = {};
+    if constexpr (TOGETHER && ROWM) {
+#pragma unroll
+        for (int l = 0; l < 3 * LINES; l++)
+            warm[l] = reinterpret_cast<const unsigned *>(rec(jlo - 1 + l / LINES))[l % LINES * 16];
+    }
+
     // ---- row jlo-1: what row jlo takes from it, then rows jlo and on ------
     const unsigned cs = at_row(jlo - 1);
     const T un_s = ld32(f.un, cs), vn_s = ld32(f.vn, cs);
@@ -351,11 +377,23 @@ __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__r
         load_point(jlo + k - 1, k - 1);
     }
 
+    if constexpr (TOGETHER) {
+        load_state(jlo + 1, 1);
+        tm[2] = ld32(f.tmask, at_row(jlo + 2));
+        load_point(jlo, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (ROWM) {
+#pragma unroll
+            for (int l = 0; l < 3 * LINES; l++) asm volatile("" ::"s"(warm[l]));
+        }
+    }
+    if constexpr (DO_SSH && R == 1) tide = tide_of();
+
     // carried from row to row: new ssh, its product with the cell area, the
     // continuity flux north, total depths, and the north face of row j-1:
     // mean velocity, momentum flux, shear quotient (u), flux, strain (v)
-    S ssh;
-    T cell, fn, du, dv, dt, vm_s, us, qs, gs, ss_v;
+    S ssh{};
+    T cell = T(0), fn, du, dv, dt, vm_s, us, qs = T(0), gs, ss_v = T(0);
     bool shut_s;   // a dry cell south of U(i, j)
     int open = 0;  // negative once the band has seen an open cell
 
@@ -388,16 +426,20 @@ __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__r
         const T full = upwind_hi(v) * un_s + part;
         shut_s = tm_s <= 0 || m_e <= 0;
         us = (shut_s ? part : full) * v * dep;
-        qs = over(un[0] - un_s, r0, M_E2US, R_E2US, ROWM ? T(0) : e2u_s + e2u[0]);
+        if constexpr (DO_U)
+            qs = over(un[0] - un_s, r0, M_E2US, R_E2US, ROWM ? T(0) : e2u_s + e2u[0]);
         du = hu[0] + su[0];
         dv = hv[0] + sv[0];
         dt = ht[0] + st[0];
         const T w = T(0.5) * (vn_s + vn[0]) * (ROWM ? r1[M_E1T] : e1t[0]);
         gs = (upwind_hi(w) * vn_s + upwind_lo(w) * vn[0]) * w * dt;
-        ss_v = over(vn[0] - vn_s, r1, M_E2T, R_E2T, ROWM ? T(0) : e2t[0]) * dt;
+        if constexpr (DO_V)
+            ss_v = over(vn[0] - vn_s, r1, M_E2T, R_E2T, ROWM ? T(0) : e2t[0]) * dt;
         fn = dv * vn[0];
-        ssh = new_ssh(r1, 0, du, fn, dv_s * vn_s, tm_s, tm[0], tm[1]);
-        cell = (ROWM ? r1[M_AT] : art[0]) * high(ssh);
+        if constexpr (DO_SSH) {
+            ssh = new_ssh(r1, 0, du, fn, dv_s * vn_s, tm_s, tm[0], tm[1]);
+            cell = (ROWM ? r1[M_AT] : art[0]) * high(ssh);
+        }
     }
 
     int done = min(jhi, jlo + R);
@@ -405,7 +447,7 @@ __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__r
 #pragma unroll UNROLL
     for (int jj = 0; jj < R; jj++) {
         const int j = jlo + jj;
-        if (j >= jhi) break;  // wavefront-uniform
+        if ((R > 1 || jj > 0) && j >= jhi) break;  // wavefront-uniform
         if constexpr (PF >= 1) {
             if (jj + PF < R && j + PF < jhi) {  // rows the band still needs
                 load_state(j + 1 + PF, 1 + PF);
@@ -413,7 +455,7 @@ __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__r
                 load_point(j + PF, PF);
             }
             __builtin_amdgcn_sched_barrier(0);
-        } else {
+        } else if (!TOGETHER || jj > 0) {
             load_state(j + 1, 1);
             tm[2] = ld32(f.tmask, at_row(j + 2));
             load_point(j, 0);
@@ -426,8 +468,12 @@ __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__r
         // ---- row j+1: depths, continuity + bc_ssh ----
         const T du1 = hu[1] + su[1], dv1 = hv[1] + sv[1], dt1 = ht[1] + st[1];
         const T fn1 = dv1 * vn[1];
-        const S ssh1 = new_ssh(r1, 1, du1, fn1, fn, tm[0], tm[1], tm[2]);
-        const T cell1 = (ROWM ? r1[M_AT] : art[1]) * high(ssh1);
+        S ssh1{};
+        T cell1 = T(0);
+        if constexpr (DO_SSH && (NEXT || R > 1)) {
+            ssh1 = new_ssh(r1, 1, du1, fn1, fn, tm[0], tm[1], tm[2]);
+            cell1 = (ROWM ? r1[M_AT] : art[1]) * high(ssh1);
+        }
 
         // ---- corner faces: u through the north side, v through the east ----
         const int m_e = from_above(tm[0]), m_ne = from_above(tm[1]);
@@ -454,13 +500,14 @@ __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__r
             v_east = (m_e <= 0 || m_ne <= 0 ? a : full) * u * dep;
             v_west_e = (tm[0] <= 0 || tm[1] <= 0 ? z : full) * u * dep;
         }
-        const T qn = over(un[1] - un[0], r0, M_E2US, R_E2US, e2us);
-        const T qe = over(vn_e - vn[0], r0, M_E1V2, R_E1V2, e1v2);
+        T qn = T(0), qe = T(0);
+        if constexpr (DO_U) qn = over(un[1] - un[0], r0, M_E2US, R_E2US, e2us);
+        if constexpr (DO_V) qe = over(vn_e - vn[0], r0, M_E1V2, R_E1V2, e1v2);
 
         // ---- U(i,j): momentum_u, else bc_solid_u ----
-        T u_new;
-        bool u_on;
-        {
+        T u_new = T(0);
+        bool u_on = false;
+        if constexpr (DO_U) {
             const T u = T(0.5) * (un[0] + un_e) * (ROWM ? r0[M_E2T] : from_above(e2t[0]));
             const T fe = (upwind_hi(u) * un[0] + upwind_lo(u) * un_e) * u * dt_e;
             const T se = over(un_e - un[0], r0, M_E1T, R_E1T,
@@ -484,9 +531,9 @@ __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__r
             u_on = own && (wet || solid);
         }
         // ---- V(i,j): momentum_v, else bc_solid_v ----
-        T v_new, v_flux, v_strain;
-        bool v_on;
-        {
+        T v_new = T(0), v_flux = T(0), v_strain = T(0);
+        bool v_on = false;
+        if constexpr (DO_V) {
             const T v = T(0.5) * (vn[0] + vn[1]) * (ROWM ? r1[M_E1T] : e1t[1]);
             v_flux = (upwind_hi(v) * vn[0] + upwind_lo(v) * vn[1]) * v * dt1;
             v_strain = over(vn[1] - vn[0], r1, M_E2T, R_E2T, ROWM ? T(0) : e2t[1]) * dt1;
@@ -513,7 +560,7 @@ __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__r
         }
         // ---- next_sshu(i,j), next_sshv(i,j) ----
         T su_new = T(0), sv_new = T(0);
-        if constexpr (NEXT) {
+        if constexpr (NEXT && DO_SSH) {
             const T s0 = high(ssh), s_e = from_above(s0), cell_e = from_above(cell);
             T mu = over(T(0.5) * (cell + cell_e), r0, M_ARU, R_ARU, ROWM ? T(0) : aru[0]);
             T mv = over(T(0.5) * (cell + cell1), r0, M_ARV, R_ARV, ROWM ? T(0) : arv[0]);
@@ -531,7 +578,7 @@ __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__r
 
         // ---- stores ----
         const bool col_t = own && i >= b.xs && i <= b.xe;
-        if (col_t && in_t) {
+        if (DO_SSH && col_t && in_t) {
             if constexpr (MIXED) {
                 store<STREAM>(o.ssh_hi, c, ssh.hi);
                 store<STREAM>(o.ssh_lo, c, ssh.lo);
@@ -539,9 +586,9 @@ __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__r
                 store<STREAM>(o.ssh, c, ssh);
             }
         }
-        if (u_on) store<STREAM>(o.u, c, u_new);
-        if (v_on) store<STREAM>(o.v, c, v_new);
-        if constexpr (NEXT) {
+        if (DO_U && u_on) store<STREAM>(o.u, c, u_new);
+        if (DO_V && v_on) store<STREAM>(o.v, c, v_new);
+        if constexpr (NEXT && DO_SSH) {
             if (col_t && in_t && i <= b.xe - 1 && tm[0] + m_e > 0)
                 store<STREAM>(o.sshu, c, su_new);
             if (col_t && in_v && tm[0] + tm[1] > 0) store<STREAM>(o.sshv, c, sv_new);
@@ -550,7 +597,7 @@ __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__r
         // ---- Flather faces next to the points this lane owns (rare) ----
         const int any_open = tm_s | tm[0] | tm[1] | tm[2];  // negative: an open cell
         if constexpr (SHORT) {
-            if (fl.on && __any(any_open < 0)) {
+            if ((DO_U || DO_V) && fl.on && __any(any_open < 0)) {
                 const int m_ee = from_above(m_e);
                 const T hu_w = from_below(hu[0]), hu_e = from_above(hu[0]);
                 const T su_w = from_below(su[0]), su_e = from_above(su[0]);
@@ -559,7 +606,7 @@ __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__r
                         hv_n = hv[1], sv_m = sv_s, hv_m = hv_s;
                 T *const ou = o.u, *const ov = o.v;
                 const T *const up = fl.u_prev, *const vp = fl.v_prev;
-                if (own) {
+                if (DO_U && own)
                     flather_faces(
                         ou, f.sshn_u, fl.cu, p.g, c, 1u, base, m_w, tm[0], m_e, m_ee,
                         i - 1 >= b.xs - 1, i <= b.xe, i + 1 <= b.xe, i == b.xs - 1,
@@ -567,6 +614,7 @@ __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__r
                         [=] { return ld32(up, c); }, [=] { return su_w; },
                         [=] { return su_c; }, [=] { return su_e; }, [=] { return hu_w; },
                         [=] { return hu_c; }, [=] { return hu_e; });
+                if (DO_V && own)
                     flather_faces(
                         ov, f.sshn_v, fl.cv, p.g, c, (unsigned)W, base, tm_s, tm[0], tm[1],
                         tm[2], j - 1 >= b.ys - 1 && j - 1 <= b.ye, j <= b.ye, j + 1 <= b.ye,
@@ -574,7 +622,6 @@ __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__r
                         [=] { return ld32(vp, c); }, [=] { return sv_m; },
                         [=] { return sv_c; }, [=] { return sv_n; }, [=] { return hv_m; },
                         [=] { return hv_c; }, [=] { return hv_n; });
-                }
             }
             hv_s = hv[0];
             sv_s = sv[0];
@@ -622,20 +669,21 @@ __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__r
 // Rows jlo .. jhi-1 (at most R) of one strip: the quick form, and plain
 // divisions from a row on whose numerators leave its range (a wave front that
 // runs into a basin at rest).
-template <typename T, bool ROWM, int R, int PF, bool NEXT, bool STREAM>
+template <typename T, bool ROWM, int R, int PF, bool NEXT, bool STREAM, int PARTS, typename Tide>
 __device__ __forceinline__ void tile(const typename Types<T>::In &f, const T *__restrict__ tab,
                                      const StepScalars<T> &p, const typename Types<T>::Out &o,
                                      const Flather<T> &fl, int W, unsigned base,
                                      const Bounds &b, int ow, int strip, int jlo, int jhi,
-                                     typename Types<T>::Tide tide)
+                                     Tide tide_of)
 {
+    static_assert(PARTS == ALL_PARTS || R <= 2, "the faces of longer bands follow all parts");
     constexpr bool QUICK = ROWM && sizeof(T) == 8;
-    const int next = rows<T, ROWM, R, PF, NEXT, STREAM, QUICK>(f, tab, p, o, fl, W, base, b, ow,
-                                                               strip, jlo, jhi, tide);
+    const int next = rows<T, ROWM, R, PF, NEXT, STREAM, QUICK, PARTS>(
+        f, tab, p, o, fl, W, base, b, ow, strip, jlo, jhi, tide_of);
     if constexpr (QUICK)
         if (next < jhi)
-            rows<T, ROWM, R, 0, NEXT, STREAM, false>(f, tab, p, o, fl, W, base, b, ow, strip,
-                                                     next, jhi, tide);
+            rows<T, ROWM, R, 0, NEXT, STREAM, false, PARTS>(f, tab, p, o, fl, W, base, b, ow,
+                                                            strip, next, jhi, tide_of);
 }
 
 }  // namespace band

@@ -10,7 +10,9 @@ namespace {
 
 using band::Flather;
 
-template <typename T, bool ROWM, int R, int OW, int PF, bool NEXT, bool STREAM>
+// SPLIT: wavefronts a tile, each with its part of the outputs: 1 (all) or 2 (u;
+// v and ssh).
+template <typename T, bool ROWM, int R, int OW, int PF, bool NEXT, bool STREAM, int SPLIT>
 __global__ __launch_bounds__(64) void k_band(typename band::Types<T>::In f,
                                              const T *__restrict__ tab, StepScalars<T> p,
                                              typename band::Types<T>::Out o, Flather<T> fl,
@@ -19,16 +21,29 @@ __global__ __launch_bounds__(64) void k_band(typename band::Types<T>::In f,
                                              double tide_val)
 {
     static_assert(OW <= 61, "one neighbour lane below, two above");
-    const int logical = wave::xcd_tile((int)blockIdx.x, (int)gridDim.x);
+    static_assert(SPLIT == 1 || SPLIT == 2, "parts of a tile");
+    const int item = wave::xcd_tile((int)blockIdx.x, (int)gridDim.x);
+    const int logical = item / SPLIT, part = item - logical * SPLIT;
     const int bd = logical / nstrip, strip = logical - bd * nstrip;
     const int jlo = b.ys - 1 + bd * R, jhi = min(jlo + R, b.ye + 2);
-    const double tide = tide_tab ? tide_tab[tide_k] : tide_val;
-    if constexpr (sizeof(T) == 8)
-        band::tile<T, ROWM, R, PF, NEXT, STREAM>(f, tab, p, o, fl, W, 0u, b, OW, strip, jlo, jhi,
-                                                 tide);
+    auto tide = [&]() __attribute__((always_inline)) {
+        const double t = tide_tab ? tide_tab[tide_k] : tide_val;
+        if constexpr (sizeof(T) == 8)
+            return t;
+        else
+            return wave::split(t);
+    };
+    auto run = [&](auto parts) __attribute__((always_inline)) {
+        band::tile<T, ROWM, R, PF, NEXT, STREAM, decltype(parts)::value>(
+            f, tab, p, o, fl, W, 0u, b, OW, strip, jlo, jhi, tide);
+    };
+    using band::PART_SSH, band::PART_U, band::PART_V;
+    if constexpr (SPLIT == 1)
+        run(std::integral_constant<int, band::ALL_PARTS>{});
+    else if (part == 0)
+        run(std::integral_constant<int, PART_U>{});
     else
-        band::tile<T, ROWM, R, PF, NEXT, STREAM>(f, tab, p, o, fl, W, 0u, b, OW, strip, jlo, jhi,
-                                                 wave::split(tide));
+        run(std::integral_constant<int, PART_V | PART_SSH>{});
 }
 
 template <typename T>
@@ -46,12 +61,12 @@ struct Args {
     double tide_val;
 };
 
-template <typename T, bool ROWM, int R, int OW, int PF, bool NEXT, bool STREAM>
+template <typename T, bool ROWM, int R, int OW, int PF, bool NEXT, bool STREAM, int SPLIT = 1>
 void launch(const Args<T> &a)
 {
     const int nstrip = wave::strips(a.b, OW);
-    const dim3 grid((unsigned)(nstrip * wave::bands(a.b, R)));
-    k_band<T, ROWM, R, OW, PF, NEXT, STREAM><<<grid, dim3(64), 0, a.s>>>(
+    const dim3 grid((unsigned)(nstrip * wave::bands(a.b, R) * SPLIT));
+    k_band<T, ROWM, R, OW, PF, NEXT, STREAM, SPLIT><<<grid, dim3(64), 0, a.s>>>(
         a.f, a.tab, a.p, a.o, a.fl, a.W, a.b, nstrip, a.tide_tab, a.tide_k, a.tide_val);
     NEMO_LAUNCH_CHECK();
 }
@@ -206,6 +221,18 @@ long tiles(const Bounds &b, int rows, int ow)
 // without: 1800^2 82 / 88, 2048^2 102 / 113, 4096^2 404 / 423). Below, and in
 // FP32, the next step finds it there (1024^2 31.1 / 25.4, 1500^2 61 / 54;
 // FP32 1500^2 79 / 69, 2048^2 116 / 110 with the read-back).
+// The smallest grids leave most SIMDs without a wavefront even so, and a step
+// takes one wavefront's chain of arithmetic. There two wavefronts share a tile
+// (SPLIT), each reading all of it and evaluating half of its outputs. One / two
+// wavefronts a tile:
+//   FP64 by row  48^2 4.4 / 3.4;  128^2 4.6 / 3.9;  256^2 5.7 / 5.4;  320^2 6.4 /
+//                6.6
+//   FP64         48^2 4.0 / 3.3;  128^2 4.4 / 4.0;  181^2 4.7 / 4.6;  256^2 5.9 /
+//                6.1
+//   FP32         48^2 2.8 / 2.4;  128^2 3.1 / 2.8;  256^2 3.8 / 3.4;  320^2 3.9 /
+//                3.8;  400^2 4.6 / 4.7
+// (three wavefronts a tile are no better anywhere but at 48^2, by 0.1 us).
+constexpr long kSplitTilesByRowF64 = 1400, kSplitTilesF64 = 600, kSplitTilesF32 = 1950;
 constexpr long kOneRowTilesF64 = 12000, kOneRowTilesByRowF64 = 3500;
 constexpr long kTwoRowTilesF64 = 48000, kTwoRowTilesByRowF64 = 24000;
 constexpr long kOneRowTilesF32 = 16000, kTwoRowTilesF32 = 20000;
@@ -234,14 +261,18 @@ void launch_band_f64(hipStream_t s, const StepIn<double> &f, const double *tab,
     const Flather<double> fl{u_prev, v_prev, nullptr, nullptr, 1};
     const Args<double> a{s, f, tab, p, o, fl, W, b, tide_tab, tide_k, tide_val};
     if (tab) {
-        if (tiles(b, 1, 61) <= kOneRowTilesByRowF64)
+        if (tiles(b, 1, 61) <= kSplitTilesByRowF64)
+            launch<double, true, 1, 61, 0, true, false, 2>(a);
+        else if (tiles(b, 1, 61) <= kOneRowTilesByRowF64)
             launch<double, true, 1, 61, 0, true, false>(a);
         else if (tiles(b, 2, 61) <= kTwoRowTilesByRowF64)
             launch<double, true, 2, 61, 0, true, false>(a);
         else
             launch<double, true, 8, 56, 0, true, true>(a);
     } else {
-        if (tiles(b, 1, 61) <= kOneRowTilesF64)
+        if (tiles(b, 1, 61) <= kSplitTilesF64)
+            launch<double, false, 1, 61, 0, true, false, 2>(a);
+        else if (tiles(b, 1, 61) <= kOneRowTilesF64)
             launch<double, false, 1, 61, 0, true, false>(a);
         else if (tiles(b, 2, 61) <= kTwoRowTilesF64)
             launch<double, false, 2, 61, 0, true, false>(a);
@@ -266,6 +297,11 @@ void launch_band_f32(hipStream_t s, int rows, int cols, int prefetch, const Mixe
     const Flather<float> fl{u_prev, v_prev, cu, cv, cu != nullptr};
     const Args<float> a{s, f, tab, p, o, fl, W, b, tide_tab, tide_k, tide_val};
     if (band_f32_auto(rows, cols, prefetch)) {
+        if (tiles(b, 1, 61) <= kSplitTilesF32) {
+            tab ? launch<float, true, 1, 61, 0, true, false, 2>(a)
+                : launch<float, false, 1, 61, 0, true, false, 2>(a);
+            return;
+        }
         if (tiles(b, 1, 61) <= kOneRowTilesF32) {
             tab ? launch<float, true, 1, 61, 0, true, false>(a)
                 : launch<float, false, 1, 61, 0, true, false>(a);

@@ -84,13 +84,14 @@ __global__ __launch_bounds__(64) void k_ens_band(typename band::Types<T>::In f,
     const Bounds b{tl.xs, tl.xe, tl.ys, tl.ye};
     const int jlo = tl.ys - 1 + tl.band * R, jhi = min(jlo + R, tl.ye + 2);
     const T *const rec = ROWM ? tab + (size_t)tl.rec * band::ROW_WIDTH : nullptr;
-    const double td = tide[tl.dom];
-    if constexpr (sizeof(T) == 8)
-        band::tile<T, ROWM, R, PF, true, STREAM>(f, rec, p, o, fl, tl.W, tl.off, b, tl.cols,
-                                                 tl.strip, jlo, jhi, td);
-    else
-        band::tile<T, ROWM, R, PF, true, STREAM>(f, rec, p, o, fl, tl.W, tl.off, b, tl.cols,
-                                                 tl.strip, jlo, jhi, wave::split(td));
+    auto tide_of = [&]() __attribute__((always_inline)) {
+        if constexpr (sizeof(T) == 8)
+            return tide[tl.dom];
+        else
+            return wave::split(tide[tl.dom]);
+    };
+    band::tile<T, ROWM, R, PF, true, STREAM, band::ALL_PARTS>(
+        f, rec, p, o, fl, tl.W, tl.off, b, tl.cols, tl.strip, jlo, jhi, tide_of);
 }
 
 template <int R, int OW, int PF>

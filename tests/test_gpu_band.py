@@ -160,3 +160,37 @@ def test_mixed_band_equals_the_other_kernels(nx, ny, metrics):
         ref = ref or out
         for n in out:
             assert_bitwise(out[n], ref[n], f"{nx}x{ny} {metrics} {rows}x{cols} p{pf} {n}")
+
+
+@pytest.mark.parametrize("metrics", ["row", "point"])
+@pytest.mark.parametrize("nx, ny", [(170, 180), (250, 231), (301, 299), (331, 330)])
+def test_shared_tiles_equal_oracle(nx, ny, metrics):
+    """Both sides of the lines below which two wavefronts share a tile, in
+    FP64 against the oracle and in FP32 against the 48-column kernel."""
+    print("shared tiles", nx, ny, metrics, flush=True)
+    m = live_model(nx, ny, metrics, seed=11)
+    ref = oracle_steps(m, [a.copy() for a in m.arrays()], 1, 4)
+    st = TimeStepper(m.copy(), mode=2)
+    st.run(4)
+    check(st, ref, f"{nx}x{ny} {metrics}")
+    out = []
+    for rows, cols in ((32, 61), (16, 48)):
+        mp = MixedStepper(m, rows=rows, cols=cols)
+        mp.run(4)
+        out.append({n: mp.fetch(n) for n in ("sshn_t", "un", "vn", "sshn_u", "sshn_v")})
+        mp.release()
+    for n in out[0]:
+        assert_bitwise(out[0][n], out[1][n], f"FP32 {nx}x{ny} {metrics} {n}")
+
+
+def test_numerators_outside_the_quick_range_in_one_row_tiles():
+    """The falling state where one wavefront evaluates a tile of one row."""
+    m = live_model(420, 300, "row", seed=12)
+    fall = 10.0 ** (-np.linspace(0.0, 300.0, m.grid.W))[None, :]
+    for n in ("ssha_t", "sshn_t", "sshn_u", "sshn_v", "un", "vn", "ua", "va"):
+        m.array(n)[:] *= fall
+    m.cfg.tide_amp = 0.0
+    ref = oracle_steps(m, [a.copy() for a in m.arrays()], 1, 3)
+    st = TimeStepper(m.copy(), mode=2)
+    st.run(3)
+    check(st, ref, "falling state")
