@@ -21,6 +21,7 @@ constexpr int HID = 32;    // hidden channels
 constexpr int CIN0 = 16;   // input channels of the layer-0 weights (4 used: u, v, ssh, depth)
 constexpr int IN0C = 4;    // channels of the stored network input
 constexpr int COUT4 = 16;  // output channels as computed (3 used: du, dv, dssh)
+constexpr int OUT4C = 4;   // channels of the stored output gradient
 constexpr int NLAYER = 4;
 
 // Layer l: weights [TAPS][cout][cin] then bias[cout], FP32 master copy.
@@ -62,7 +63,7 @@ struct Norm {
 enum Epilogue { EPI_HIDDEN = 0, EPI_OUTPUT = 1, EPI_DX = 2 };
 
 struct ConvArgs {
-    const __bf16 *in;     // padded NHWC, cin channels
+    const __bf16 *in;     // padded NHWC, cin channels (16: the 4 stored ones)
     const __bf16 *w;      // [TAPS][cout][cin]
     const float *bias;    // cout (EPI_HIDDEN, EPI_OUTPUT)
     __bf16 *out;          // padded NHWC, cout channels (EPI_HIDDEN act, EPI_DX grad)
@@ -109,22 +110,29 @@ void launch_weights_bf16(hipStream_t s, const float *w, int cin, int cout,
 // coarse state -> padded network input (IN0C channels) and the activity gate
 void launch_pack(hipStream_t s, const CoarseState &c, const Norm &nm, __bf16 *in0,
                  float *gate, int nx, int ny);
-// target[(y*nx+x)*4 + k] = (F_k - C_k) / out_scale_k, k = u, v, ssh
-void launch_target(hipStream_t s, const double *fssh, const double *fu, const double *fv,
-                   const CoarseState &c, const Norm &nm, float *target, int nx, int ny);
 // Per-channel weights (u, v, ssh) of the squared error in the loss.
 struct LossWeights {
     float w[3];
 };
 
-// Weighted MSE loss over the 3 used channels, sum_c w_c sum_p d_c^2 / (3 npx):
-// gradient into dpre4 (COUT4 channels, 16-channel plane) and per-block
-// partial sums of the unweighted squared error per channel. With a mask
-// (pitch W), the ssh of cells not corrected (Norm::ssh_wet) is left out.
-int loss_blocks();
-void launch_loss(hipStream_t s, const float *pred, const float *target, __bf16 *dpre4,
-                 float *partial, int nx, int ny, const int *tmask, int W, int ssh_wet,
-                 const float *gate, const LossWeights &lw);
+// Fields the target is taken from, target_k = (F_k - C_k) / out_scale_k, k =
+// u, v, ssh: the filtered fine state and the coarse state (pitch c.W).
+struct LossFields {
+    const double *fssh, *fu, *fv;
+    CoarseState c;
+    Norm nm;
+};
+
+// Weighted MSE loss over the 3 used channels, sum_c w_c sum_p d_c^2 / (3 npx),
+// against target[(y*nx+x)*4 + k] or, where fields is not null, the target they
+// give: gradient into dpre4 (OUT4C channels a padded pixel) and per-block
+// partial sums of the unweighted squared error per channel (loss_blocks(nx,
+// ny) blocks). With a mask (pitch W), the ssh of cells not corrected
+// (Norm::ssh_wet) is left out.
+int loss_blocks(int nx, int ny);
+void launch_loss(hipStream_t s, const float *pred, const float *target, const LossFields *fields,
+                 __bf16 *dpre4, float *partial, int nx, int ny, const int *tmask, int W,
+                 int ssh_wet, const float *gate, const LossWeights &lw);
 
 // ---- fine <-> coarse plumbing ----------------------------------------------
 // Box filter of the fine state onto the coarse grid (factor f): T cells by

@@ -106,8 +106,7 @@ __device__ __forceinline__ Band xcd_band(int items)
     return Band{first, last - first, (int)(blockIdx.x >> 3), (int)(gridDim.x >> 3)};
 }
 
-// 32 output channels. KIND 1: 16 input channels. KIND 2: 32 input channels.
-// (The network input layer, 4 channels, is k_conv_in.)
+// 32 input and 32 output channels. (From 4 channels: k_conv_in.)
 // EPI_HIDDEN: bias, GELU, optional pre-activation; EPI_DX: times gelu'(gpre).
 // NT tiles per wavefront pass, WPB wavefronts per workgroup, two workgroups
 // per CU (the LDS weights):
@@ -117,15 +116,13 @@ __device__ __forceinline__ Band xcd_band(int items)
 //   LDS weight read per MFMA, twice the wavefronts to hide the activation
 //   loads and overlap one wavefront's epilogue with another's MFMAs.
 // Every tile sees the same MFMA sequence in both forms: the same bits.
-template <int KIND, int EPI, int NT, int WPB>
+template <int EPI, int NT, int WPB>
 __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(4 / NT, 4 / NT)))
 void k_conv_sh(ConvArgs a)
 {
-    static_assert(KIND == 1 || KIND == 2, "16 or 32 input channels");
     static_assert(EPI == EPI_HIDDEN || EPI == EPI_DX, "epilogue");
     static_assert((NT == 2 && WPB == 4) || (NT == 1 && WPB == 8), "launch form");
-    constexpr int NC = KIND == 2 ? 2 : 1;
-    constexpr int CIN = KIND == 2 ? 32 : 16;
+    constexpr int NC = 2, CIN = 32;
     constexpr int ROW = CIN + 8;  // LDS row of one output channel, padded by 8
     constexpr int NROWS = TAPS * 32;
     __shared__ __attribute__((aligned(16))) __bf16 wsh[NROWS * ROW];
@@ -316,7 +313,8 @@ void k_conv_sh(ConvArgs a)
     }
 }
 
-// Network input layer (4 -> 32 channels) as an implicit GEMM with the taps in
+// 32 channels from 4: the network input layer (EPI_HIDDEN) and the input
+// gradient of the output layer (EPI_DX), as an implicit GEMM with the taps in
 // K: 25 taps x 4 channels (100, padded to 112 = 7 chunks of 16), so one
 // accumulator holds the whole 5x5 sum of a 32-pixel tile and no horizontal
 // shift-sum or tile overlap is needed. Each half h of the wavefront carries
@@ -331,7 +329,8 @@ void k_conv_sh(ConvArgs a)
 // the kernel keeps its registers under 128 for 4 wavefronts per SIMD
 // instead of sharing one loaded fragment among five accumulators. Tiles sit
 // at x0 = min(32 t, nx - 32); the last one overlaps its neighbour and stores
-// only x >= 32 t.
+// only x >= 32 t. The output layer's gradient, stored in 4 channels as well,
+// takes 14.0 us at 512^2 here, 15.9 with 16 channels in the shift-sum form.
 constexpr int IN_CHUNKS = 7;
 
 // Kernel tap (dy * 5 + dx) of chunk c, half h, slot q; -1: a zero K slot.
@@ -342,15 +341,20 @@ __device__ __forceinline__ int in_tap(int c, int h, int q)
     return h == 0 && q == 0 ? 24 : -1;
 }
 
+template <int EPI>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_conv_in(
     ConvArgs a)
 {
+    static_assert(EPI == EPI_HIDDEN || EPI == EPI_DX, "epilogue");
+    static_assert(CIN0 == COUT4, "one stride of the weights");
     // the bias sits in LDS: an LDS read in the epilogue waits on the LDS
     // counter only, where a global load would wait for every store and
     // every prefetched fragment before it
     __shared__ __attribute__((aligned(16))) float bsh[HID];
-    if (threadIdx.x < HID) bsh[threadIdx.x] = a.bias[threadIdx.x];
-    __syncthreads();
+    if constexpr (EPI == EPI_HIDDEN) {
+        if (threadIdx.x < HID) bsh[threadIdx.x] = a.bias[threadIdx.x];
+        __syncthreads();
+    }
     const int lane = (int)(threadIdx.x & 63), n = lane & 31, h = lane >> 5;
     const int nx = a.nx, Wp = nx + 4, T = (nx + 31) / 32;
     const size_t PL = plane_elems(nx, a.ny);
@@ -441,15 +445,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
             for (int g = 0; g < 4; g++) {
                 const int co = g * 8 + h * 4;
                 const size_t o = (size_t)(co >> 4) * PL + px + (co & 15);
-                const f32x4 bias = *reinterpret_cast<const f32x4 *>(&bsh[co]);
-                bf16x4 p, r;
+                bf16x4 r;
+                if constexpr (EPI == EPI_HIDDEN) {
+                    const f32x4 bias = *reinterpret_cast<const f32x4 *>(&bsh[co]);
+                    bf16x4 p;
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const float v = acc[4 * g + j] + bias[j];
-                    p[j] = (__bf16)v;
-                    r[j] = (__bf16)gelu(v);
+                    for (int j = 0; j < 4; j++) {
+                        const float v = acc[4 * g + j] + bias[j];
+                        p[j] = (__bf16)v;
+                        r[j] = (__bf16)gelu(v);
+                    }
+                    if (a.pre) *reinterpret_cast<bf16x4 *>(a.pre + o) = p;
+                } else {
+                    const bf16x4 gp = *reinterpret_cast<const bf16x4 *>(a.gpre + o);
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        r[j] = (__bf16)(acc[4 * g + j] * gelu_grad((float)gp[j]));
                 }
-                if (a.pre) *reinterpret_cast<bf16x4 *>(a.pre + o) = p;
                 *reinterpret_cast<bf16x4 *>(a.out + o) = r;
             }
         }
@@ -753,12 +765,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             const int c = tid + 256 * k, row = c / DC, q = c - row * DC, y = r0 + row;
             dr[k] = {};
             if (c < DN && y < yb) {  // interior row
-                const size_t px = pad_index(y, x0, nx) * 16;
+                const size_t px = pad_index(y, x0, nx);
                 if constexpr (NET_OUT)
-                    dr[k] = *reinterpret_cast<const bf16x4 *>(dpre + px + q * 16);
+                    dr[k] = *reinterpret_cast<const bf16x4 *>(dpre + (px + q) * OUT4C);
                 else
-                    dr[k] = *reinterpret_cast<const bf16x8 *>(dpre + (size_t)(q >> 6) * PL + px +
-                                                              (q & 63) * 8);
+                    dr[k] = *reinterpret_cast<const bf16x8 *>(dpre + (size_t)(q >> 6) * PL +
+                                                              px * 16 + (q & 63) * 8);
             }
         }
     };
@@ -1026,25 +1038,23 @@ __global__ void k_pack(CoarseState c, Norm nm, __bf16 *__restrict__ in0,
     *reinterpret_cast<bf16x4 *>(in0 + pad_index(y, x, nx) * IN0C) = lo;
 }
 
-__global__ void k_target(const double *__restrict__ fssh, const double *__restrict__ fu,
-                         const double *__restrict__ fv, CoarseState c, Norm nm,
-                         float *__restrict__ target, int nx, int ny)
+// The target of one point: (filtered fine state - coarse state) / out_scale.
+__device__ __forceinline__ float4 target_of(const LossFields &f, size_t k)
 {
-    const int p = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (p >= nx * ny) return;
-    const int y = p / nx, x = p - y * nx;
-    const size_t k = (size_t)(y + 1) * c.W + (x + 1);
     float4 t;
-    t.x = (float)(fu[k] - c.u[k]) / nm.out_scale[0];
-    t.y = (float)(fv[k] - c.v[k]) / nm.out_scale[1];
-    t.z = (float)(fssh[k] - c.ssh[k]) / nm.out_scale[2];
+    t.x = (float)(f.fu[k] - f.c.u[k]) / f.nm.out_scale[0];
+    t.y = (float)(f.fv[k] - f.c.v[k]) / f.nm.out_scale[1];
+    t.z = (float)(f.fssh[k] - f.c.ssh[k]) / f.nm.out_scale[2];
     t.w = 0.0f;
-    reinterpret_cast<float4 *>(target)[p] = t;
+    return t;
 }
 
-
+// FIELDS: the targets come from the model's fields, else from `target`. Four
+// points a thread in a row cost four memory latencies at 512^2 (10.8 us, and a
+// launch for the targets, 5.0): one point now, 7.4 us.
+template <bool FIELDS>
 __global__ __launch_bounds__(256) void k_loss(const float *__restrict__ pred,
-                                              const float *__restrict__ target,
+                                              const float *__restrict__ target, LossFields f,
                                               __bf16 *__restrict__ dpre4,
                                               float *__restrict__ partial, int nx, int ny,
                                               const int *__restrict__ tmask, int W,
@@ -1058,23 +1068,26 @@ __global__ __launch_bounds__(256) void k_loss(const float *__restrict__ pred,
     for (int p = (int)(blockIdx.x * blockDim.x + threadIdx.x); p < npx;
          p += (int)(gridDim.x * blockDim.x)) {
         const float4 a = reinterpret_cast<const float4 *>(pred)[p];
-        const float4 b = reinterpret_cast<const float4 *>(target)[p];
         const int y = p / nx, x = p - y * nx;
-        const bool ssh_free =
-            !tmask || ssh_cell(tmask, (size_t)(y + 1) * W + (x + 1), W, ssh_wet);
+        const size_t k = (size_t)(y + 1) * W + (x + 1);
+        float4 b;
+        if constexpr (FIELDS)
+            b = target_of(f, k);
+        else
+            b = reinterpret_cast<const float4 *>(target)[p];
+        const bool ssh_free = !tmask || ssh_cell(tmask, k, W, ssh_wet);
         const float d0 = a.x - b.x, d1 = a.y - b.y, d2 = ssh_free ? a.z - b.z : 0.0f;
         s0 += d0 * d0;
         s1 += d1 * d1;
         s2 += d2 * d2;
         // the output is gated (pred = gate * raw output): d loss / d raw
         const float gs = gate ? scale * gate[p] : scale;
-        bf16x8 lo = {}, hi = {};
+        bf16x4 lo = {};
         lo[0] = (__bf16)(gs * lw.w[0] * d0);
         lo[1] = (__bf16)(gs * lw.w[1] * d1);
         lo[2] = (__bf16)(gs * lw.w[2] * d2);
-        bf16x8 *dst = reinterpret_cast<bf16x8 *>(dpre4 + pad_index(y, x, nx) * COUT4);
-        dst[0] = lo;
-        dst[1] = hi;
+        static_assert(OUT4C == 4, "one 8-byte pixel");
+        *reinterpret_cast<bf16x4 *>(dpre4 + pad_index(y, x, nx) * OUT4C) = lo;
     }
     red[0][threadIdx.x] = s0;
     red[1][threadIdx.x] = s1;
@@ -1241,21 +1254,19 @@ void launch_conv(hipStream_t s, int cin, int cout, Epilogue epi, const ConvArgs 
     const dim3 grid = conv_grid(2), block(256), block8(512);
     const bool one = g_conv_form == 1;
     if (cin == 16 && cout == 32 && epi == EPI_HIDDEN)  // the network input: 4 used channels
-        k_conv_in<<<conv_grid(4), block, 0, s>>>(a);
+        k_conv_in<EPI_HIDDEN><<<conv_grid(4), block, 0, s>>>(a);
     else if (cin == 32 && cout == 32 && epi == EPI_HIDDEN && one)
-        k_conv_sh<2, EPI_HIDDEN, 1, 8><<<grid, block8, 0, s>>>(a);
+        k_conv_sh<EPI_HIDDEN, 1, 8><<<grid, block8, 0, s>>>(a);
     else if (cin == 32 && cout == 32 && epi == EPI_HIDDEN)
-        k_conv_sh<2, EPI_HIDDEN, 2, 4><<<grid, block, 0, s>>>(a);
+        k_conv_sh<EPI_HIDDEN, 2, 4><<<grid, block, 0, s>>>(a);
     else if (cin == 32 && cout == 16 && epi == EPI_OUTPUT)
         k_conv_out<false><<<out_grid(a.nx, a.ny), block, 0, s>>>(a, GuardSums{});
-    else if (cin == 16 && cout == 32 && epi == EPI_DX && one)
-        k_conv_sh<1, EPI_DX, 1, 8><<<grid, block8, 0, s>>>(a);
-    else if (cin == 16 && cout == 32 && epi == EPI_DX)
-        k_conv_sh<1, EPI_DX, 2, 4><<<grid, block, 0, s>>>(a);
+    else if (cin == 16 && cout == 32 && epi == EPI_DX)  // 4 stored channels
+        k_conv_in<EPI_DX><<<conv_grid(4), block, 0, s>>>(a);
     else if (cin == 32 && cout == 32 && epi == EPI_DX && one)
-        k_conv_sh<2, EPI_DX, 1, 8><<<grid, block8, 0, s>>>(a);
+        k_conv_sh<EPI_DX, 1, 8><<<grid, block8, 0, s>>>(a);
     else if (cin == 32 && cout == 32 && epi == EPI_DX)
-        k_conv_sh<2, EPI_DX, 2, 4><<<grid, block, 0, s>>>(a);
+        k_conv_sh<EPI_DX, 2, 4><<<grid, block, 0, s>>>(a);
     else
         NEMO_FATAL("closure conv: unsupported %d -> %d channels, epilogue %d", cin, cout,
                    (int)epi);
@@ -1330,23 +1341,22 @@ void launch_pack(hipStream_t s, const CoarseState &c, const Norm &nm, __bf16 *in
     NEMO_LAUNCH_CHECK();
 }
 
-void launch_target(hipStream_t s, const double *fssh, const double *fu, const double *fv,
-                   const CoarseState &c, const Norm &nm, float *target, int nx, int ny)
+int loss_blocks(int nx, int ny)
 {
-    k_target<<<grid_for((long)nx * ny), dim3(256), 0, s>>>(fssh, fu, fv, c, nm, target,
-                                                           nx, ny);
-    NEMO_LAUNCH_CHECK();
+    return (int)std::min(4096L, ((long)nx * ny + 255) / 256);
 }
 
-int loss_blocks() { return 256; }
-
-void launch_loss(hipStream_t s, const float *pred, const float *target, __bf16 *dpre4,
-                 float *partial, int nx, int ny, const int *tmask, int W, int ssh_wet,
-                 const float *gate, const LossWeights &lw)
+void launch_loss(hipStream_t s, const float *pred, const float *target, const LossFields *fields,
+                 __bf16 *dpre4, float *partial, int nx, int ny, const int *tmask, int W,
+                 int ssh_wet, const float *gate, const LossWeights &lw)
 {
-    k_loss<<<dim3((unsigned)loss_blocks()), dim3(256), 0, s>>>(pred, target, dpre4,
-                                                               partial, nx, ny, tmask, W,
-                                                               ssh_wet, gate, lw);
+    const dim3 grid((unsigned)loss_blocks(nx, ny)), block(256);
+    if (fields)
+        k_loss<true><<<grid, block, 0, s>>>(pred, nullptr, *fields, dpre4, partial, nx, ny, tmask,
+                                            W, ssh_wet, gate, lw);
+    else
+        k_loss<false><<<grid, block, 0, s>>>(pred, target, LossFields{}, dpre4, partial, nx, ny,
+                                             tmask, W, ssh_wet, gate, lw);
     NEMO_LAUNCH_CHECK();
 }
 

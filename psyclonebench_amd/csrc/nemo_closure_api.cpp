@@ -273,7 +273,7 @@ void *nemo_cl_create(int nx, int ny, int coarse_width, int coarse_height,
     for (int l = 0; l < NLAYER; l++) {
         C->wf[l] = zeros<__bf16>(layer_wsize(l), s);
         C->wx[l] = zeros<__bf16>(layer_wsize(l), s);
-        C->dpre[l] = zeros<__bf16>(C->padded(layer_cout(l)), s);
+        C->dpre[l] = zeros<__bf16>(C->padded(l == NLAYER - 1 ? OUT4C : layer_cout(l)), s);
     }
     C->in0 = zeros<__bf16>(C->padded(IN0C), s);
     for (int l = 0; l < NLAYER - 1; l++) {
@@ -287,7 +287,7 @@ void *nemo_cl_create(int nx, int ny, int coarse_width, int coarse_height,
     for (int l = 0; l < NLAYER; l++)
         C->dw_partial[l] = zeros<float>((size_t)dw_blocks(nx, ny) * layer_psize(l), s);
     C->square = zeros<float>((size_t)grad_squares(), s);
-    C->loss_partial = zeros<float>((size_t)loss_blocks() * 3, s);
+    C->loss_partial = zeros<float>((size_t)loss_blocks(nx, ny) * 3, s);
     C->norm_scale = zeros<float>(2, s);
     const size_t nc = (size_t)coarse_width * coarse_height;
     C->fssh = zeros<double>(nc, s);
@@ -425,8 +425,8 @@ void nemo_cl_train_step(void *h, double *ssh, double *u, double *v, double *sshu
     hipStream_t s = lib_stream();
     launch_pack(s, c, C.nm, C.in0, C.gate, C.nx, C.ny);
     forward(C, s, true, true, false);
-    launch_target(s, C.fssh, C.fu, C.fv, c, C.nm, C.target, C.nx, C.ny);
-    launch_loss(s, C.pred, C.target, C.dpre[NLAYER - 1], C.loss_partial, C.nx, C.ny, tmask,
+    const LossFields fields{C.fssh, C.fu, C.fv, c, C.nm};
+    launch_loss(s, C.pred, nullptr, &fields, C.dpre[NLAYER - 1], C.loss_partial, C.nx, C.ny, tmask,
                 C.Wc, C.nm.ssh_wet, C.gate, C.loss_w);
     backward(C, s);
     optimizer_step(C, s);
@@ -435,7 +435,7 @@ void nemo_cl_train_step(void *h, double *ssh, double *u, double *v, double *sshu
 double nemo_cl_last_loss(void *h)
 {
     ClosureContext &C = ctx(h);
-    std::vector<float> p((size_t)loss_blocks() * 3);
+    std::vector<float> p((size_t)loss_blocks(C.nx, C.ny) * 3);
     NEMO_HIP_CHECK(hipStreamSynchronize(lib_stream()));
     NEMO_HIP_CHECK(hipMemcpy(p.data(), C.loss_partial, p.size() * sizeof(float),
                              hipMemcpyDeviceToHost));
@@ -456,7 +456,7 @@ void nemo_cl_set_loss_weights(void *h, double wu, double wv, double wssh)
 void nemo_cl_last_stats(void *h, double *out)
 {
     ClosureContext &C = ctx(h);
-    std::vector<float> p((size_t)loss_blocks() * 3);
+    std::vector<float> p((size_t)loss_blocks(C.nx, C.ny) * 3);
     float ns[2];
     const int gblk = guard_blocks(C.nx, C.ny);
     std::vector<double> gp((size_t)gblk * 3);
@@ -469,7 +469,7 @@ void nemo_cl_last_stats(void *h, double *out)
     const double npx = (double)C.nx * C.ny;
     for (int c = 0; c < 3; c++) {
         double s = 0.0;
-        for (int b = 0; b < loss_blocks(); b++) s += p[(size_t)b * 3 + c];
+        for (int b = 0; b < loss_blocks(C.nx, C.ny); b++) s += p[(size_t)b * 3 + c];
         out[c] = s / npx;
     }
     out[3] = ns[0];
@@ -548,7 +548,7 @@ static void host_pair(ClosureContext &C, const float *in4, const float *target3,
     NEMO_HIP_CHECK(hipMemcpyAsync(C.target, t.data(), t.size() * sizeof(float),
                                   hipMemcpyHostToDevice, s));
     forward(C, s, true, false, false);
-    launch_loss(s, C.pred, C.target, C.dpre[NLAYER - 1], C.loss_partial, C.nx, C.ny,
+    launch_loss(s, C.pred, C.target, nullptr, C.dpre[NLAYER - 1], C.loss_partial, C.nx, C.ny,
                 nullptr, 0, 0, nullptr, C.loss_w);
     backward(C, s);
     NEMO_HIP_CHECK(hipStreamSynchronize(s));  // t goes out of scope

@@ -255,6 +255,40 @@ def test_filter_and_set_state():
     net.release()
 
 
+def test_training_step_equals_the_step_on_its_inputs():
+    """train_step takes its input and target from the model's fields; the same
+    input and target handed over from the host give the same loss and weights,
+    bit for bit (every interior cell wet and counted, no gate)."""
+    fine, coarse = _fine_and_coarse()
+    sf, sc = TimeStepper(fine, mode=2), TimeStepper(coarse, mode=2)
+    sf.run(3)
+    sc.run(1)
+    g = coarse.grid
+    inner = (slice(1, g.N - 1), slice(1, g.M - 1))
+    assert np.all(coarse.array("tmask")[inner] > 0)
+    p, out = net_params(12), []
+    for from_model in (True, False):
+        net = ClosureNet(coarse, params=p)
+        net.set_ssh_cells(True)
+        net.set_optimizer("sgd", lr=1e-2)
+        net.filter_fine(sf, 4)
+        if from_model:
+            net.train_step(sc)
+            loss = net.last_loss()
+        else:
+            names = ("un", "vn", "sshn_t")
+            state = [sc.fetch(n) for n in names]
+            x = np.stack([a[inner] for a in state] + [coarse.array("ht")[inner]], -1)
+            t = np.stack([(net.filtered(n, (g.H, g.W)) - a)[inner]
+                          for n, a in zip(names, state)], -1)
+            loss = net.train_host(x, t)
+        out.append((loss, net.params()))
+        net.release()
+    assert out[0][0] == out[1][0] > 0.0
+    assert_bitwise(out[0][1], out[1][1], "weights")
+    assert np.any(out[0][1] != p.astype(np.float32))
+
+
 def test_guard_keeps_plain_step_on_blowup():
     fine, coarse = _fine_and_coarse()
     sc = TimeStepper(coarse, mode=2)
