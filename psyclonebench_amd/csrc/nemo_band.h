@@ -109,6 +109,7 @@ template <typename T>
 struct Flather {
     const T *u_prev, *v_prev, *cu, *cv;
     int on;
+    T two_omega, d2r;  // in-place form (NEXT = false)
 };
 
 // First owned lane of a strip of ow columns: one neighbour lane below and two
@@ -240,7 +241,9 @@ __device__ __forceinline__ void flather_rows(const typename Types<T>::In &f,
 // of the launch or of the tile). At most R rows (jlo .. jhi-1), PF rows of
 // loads in flight beyond the next (the loop is unrolled, so the window shifts
 // are register renaming). NEXT: write the new face ssh (false where the step
-// updates the caller's arrays in place and a second kernel follows). STREAM:
+// updates the caller's arrays in place and a second kernel follows; there
+// f.fcor_u and f.fcor_v are the latitudes, and the tile evaluates the Coriolis
+// factors itself). STREAM:
 // non-temporal stores. QUICK: uniform_quotient for the row's divisors.
 // PARTS: the outputs this wavefront evaluates and writes (enum Part).
 // tide_of(): the elevation of open cells; one-row bands read it behind their
@@ -331,6 +334,12 @@ __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__r
             return divide(a, r[m]);
         else
             return divide(a, x);
+    };
+    auto coriolis = [&](T x) -> T {
+        if constexpr (NEXT)
+            return x;
+        else
+            return fl.two_omega * sin(x * fl.d2r);  // momentum_u_kern.c:251
     };
     T y_fric = T(0);
     if constexpr (QUICK) y_fric = refined_reciprocal(p.fric);
@@ -520,7 +529,7 @@ __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__r
             T vis = (se - sw) * along + ((shut_n ? T(0) : shear_n) - (shut_s ? T(0) : shear_s)) *
                                             (ROWM ? r0[M_E1U] : e1u[0]) * T(0.5);
             vis = p.visc * vis;
-            const T cor = T(0.5) * ((ROWM ? r0[M_FCU] : fcu[0]) * (vm_s + vm)) * area * du;
+            const T cor = T(0.5) * ((ROWM ? r0[M_FCU] : coriolis(fcu[0])) * (vm_s + vm)) * area * du;
             const T hpg = -p.g * du * along * (st_e - st[0]);
             const T acc = over(p.rdt * (adv + vis + cor + hpg), r0, M_ARU, R_ARU, area);
             T val = over_fric(divide(un[0] * du + acc, hu[0] + (ROWM ? r0[M_SAU] : sau[0])));
@@ -547,7 +556,7 @@ __device__ __forceinline__ int rows(const typename Types<T>::In &f, const T *__r
                     ((shut_e ? T(0) : shear_e) - (shut_w ? T(0) : shear_w)) *
                         (ROWM ? r0[M_E2V] : e2v[0]) * T(0.5);
             vis = p.visc * vis;
-            const T cor = -T(0.5) * ((ROWM ? r0[M_FCV] : fcv[0]) * (um + um_w)) * area * dv;
+            const T cor = -T(0.5) * ((ROWM ? r0[M_FCV] : coriolis(fcv[0])) * (um + um_w)) * area * dv;
             const T hpg = -p.g * dv * along * (st[1] - st[0]);
             const T acc = over(p.rdt * (adv + vis + cor + hpg), r0, M_ARV, R_ARV, area);
             T val = over_fric(divide(vn[0] * dv + acc, hv[0] + (ROWM ? r0[M_SAV] : sav[0])));

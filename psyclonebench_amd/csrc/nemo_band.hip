@@ -276,7 +276,7 @@ void launch_band_f64(hipStream_t s, const StepIn<double> &f, const double *tab,
                      const double *u_prev, const double *v_prev, int W, const Bounds &b,
                      const double *tide_tab, int tide_k, double tide_val)
 {
-    const Flather<double> fl{u_prev, v_prev, nullptr, nullptr, 1};
+    const Flather<double> fl{u_prev, v_prev, nullptr, nullptr, 1, 0.0, 0.0};
     const Args<double> a{s, f, tab, p, o, fl, W, b, tide_tab, tide_k, tide_val};
     if (tab) {
         if (tiles(b, 1, 61) <= kSplitTilesByRowF64)
@@ -312,7 +312,7 @@ void launch_band_f32(hipStream_t s, int rows, int cols, int prefetch, const Mixe
                      const float *cv, int W, const Bounds &b, const double *tide_tab, int tide_k,
                      double tide_val)
 {
-    const Flather<float> fl{u_prev, v_prev, cu, cv, cu != nullptr};
+    const Flather<float> fl{u_prev, v_prev, cu, cv, cu != nullptr, 0.0f, 0.0f};
     const Args<float> a{s, f, tab, p, o, fl, W, b, tide_tab, tide_k, tide_val};
     if (band_f32_auto(rows, cols, prefetch)) {
         if (tiles(b, 1, 61) <= kSplitTilesF32) {
@@ -357,11 +357,12 @@ void launch_band_f32(hipStream_t s, int rows, int cols, int prefetch, const Mixe
 }
 
 void launch_band_inplace(hipStream_t s, const StepIn<double> &f, const StepScalars<double> &p,
-                         const StepOut<double> &o, int W, const Bounds &b, double tide)
+                         const StepOut<double> &o, double omega, double d2r, int W,
+                         const Bounds &b, double tide)
 {
     // the after arrays hold the previous step's velocities until their faces
     // are written
-    const Flather<double> fl{o.u, o.v, nullptr, nullptr, 1};
+    const Flather<double> fl{o.u, o.v, nullptr, nullptr, 1, 2. * omega, d2r};
     const Args<double> a{s, f, nullptr, p, o, fl, W, b, nullptr, 0, tide};
     if (tiles(b, 1, 61) <= kOneRowTilesF64)
         launch<double, false, 1, 61, 0, false, false>(a);

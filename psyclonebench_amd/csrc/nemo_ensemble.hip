@@ -238,7 +238,7 @@ void launch_band(hipStream_t s, const EnsBand &bt, const In &in, const T *tab,
                  const T *cu, const T *cv, const EnsTile *tiles, int ntiles, const double *tide)
 {
     if (ntiles <= 0) return;
-    const band::Flather<T> fl{u_prev, v_prev, cu, cv, sizeof(T) == 8 || cu};
+    const band::Flather<T> fl{u_prev, v_prev, cu, cv, sizeof(T) == 8 || cu, T(0), T(0)};
     const dim3 grid((unsigned)ntiles), block(64);
     auto run = [&](auto kernel) {
         kernel<<<grid, block, 0, s>>>(in, tab, p, out, fl, tiles, tide);

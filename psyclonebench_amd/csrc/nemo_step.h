@@ -118,8 +118,10 @@ void launch_band_f64(hipStream_t s, const StepIn<double> &f, const double *tab,
 // The sweeps up to bc_flather of an in-place step (o.ssh, o.u, o.v are the
 // after arrays; o.sshu / o.sshv are not written), then, in launch_finish, the
 // copies now <- after and next_sshu/v. Together the unfused sequence.
+// f.fcor_u / f.fcor_v: the latitudes gphiu / gphiv.
 void launch_band_inplace(hipStream_t s, const StepIn<double> &f, const StepScalars<double> &p,
-                         const StepOut<double> &o, int W, const Bounds &b, double tide);
+                         const StepOut<double> &o, double omega, double d2r, int W,
+                         const Bounds &b, double tide);
 void launch_finish(hipStream_t s, double *un, const double *ua, double *vn, const double *va,
                    double *sshn_t, const double *ssha_t, double *sshn_u, double *sshn_v,
                    const int *tmask, const double *area_t, const double *area_u,
