@@ -43,8 +43,8 @@ extern "C" void c_invoke_time_step_noalloc(NEMO_HOST_ARRAYS, int istep, int inte
                      width, total_size};
     check_geometry(G);
     if (total_size > kNoallocMaxElems)
-        NEMO_FATAL("c_invoke_time_step_noalloc: total_size %d exceeds its limit of %d "
-                   "elements", total_size, kNoallocMaxElems);
+        NEMO_FATAL("c_invoke_time_step_noalloc: total_size %d exceeds the %d elements "
+                   "it takes", total_size, kNoallocMaxElems);
     hipStream_t s = static_cast<hipStream_t>(stream);
     // hipGetLastError also returns what earlier calls of other code on this
     // thread left behind (an event query's "not ready", say); clear it so
