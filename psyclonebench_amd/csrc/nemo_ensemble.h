@@ -61,6 +61,7 @@ bool ens_band(const EnsShape &shape);
 struct EnsBand {
     int rows, cols, prefetch;
     bool stream;  // non-temporal stores
+    bool split;   // two wavefronts a tile
 };
 EnsBand ens_band_tiles(const EnsShape &shape, int precision, bool by_row, long one_row_tiles,
                        long two_row_tiles);

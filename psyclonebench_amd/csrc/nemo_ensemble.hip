@@ -69,10 +69,11 @@ __device__ __forceinline__ void ens_tile_mixed(const MixedIn &f, const StepScala
                                 tl.strip, tl.band, wave::split(tide));
 }
 
-// Band tile, one wavefront each; the grid has exactly ntiles workgroups. The
-// strip's width comes with the tile. ROWM: every domain has a table of metrics
+// Band tile, one wavefront each, or two that share it (SPLIT = 2: u; v and ssh);
+// the grid has exactly SPLIT * ntiles workgroups. The strip's width comes with
+// the tile. ROWM: every domain has a table of metrics
 // by row (records tl.rec and on).
-template <typename T, bool ROWM, int R, int PF, bool STREAM>
+template <typename T, bool ROWM, int R, int PF, bool STREAM, int SPLIT = 1>
 __global__ __launch_bounds__(64) void k_ens_band(typename band::Types<T>::In f,
                                                  const T *__restrict__ tab, StepScalars<T> p,
                                                  typename band::Types<T>::Out o,
@@ -80,7 +81,9 @@ __global__ __launch_bounds__(64) void k_ens_band(typename band::Types<T>::In f,
                                                  const EnsTile *__restrict__ tiles,
                                                  const double *__restrict__ tide)
 {
-    const EnsTile tl = tiles[wave::xcd_tile((int)blockIdx.x, (int)gridDim.x)];
+    static_assert(SPLIT == 1 || SPLIT == 2, "parts of a tile");
+    const int item = wave::xcd_tile((int)blockIdx.x, (int)gridDim.x);
+    const EnsTile tl = tiles[item / SPLIT];
     const Bounds b{tl.xs, tl.xe, tl.ys, tl.ye};
     const int jlo = tl.ys - 1 + tl.band * R, jhi = min(jlo + R, tl.ye + 2);
     const T *const rec = ROWM ? tab + (size_t)tl.rec * band::ROW_WIDTH : nullptr;
@@ -90,8 +93,16 @@ __global__ __launch_bounds__(64) void k_ens_band(typename band::Types<T>::In f,
         else
             return wave::split(tide[tl.dom]);
     };
-    band::tile<T, ROWM, R, PF, true, STREAM, band::ALL_PARTS>(
-        f, rec, p, o, fl, tl.W, tl.off, b, tl.cols, tl.strip, jlo, jhi, tide_of);
+    auto run = [&](auto parts) __attribute__((always_inline)) {
+        band::tile<T, ROWM, R, PF, true, STREAM, decltype(parts)::value>(
+            f, rec, p, o, fl, tl.W, tl.off, b, tl.cols, tl.strip, jlo, jhi, tide_of);
+    };
+    if constexpr (SPLIT == 1)
+        run(std::integral_constant<int, band::ALL_PARTS>{});
+    else if (item % SPLIT == 0)
+        run(std::integral_constant<int, band::PART_U>{});
+    else
+        run(std::integral_constant<int, band::PART_V | band::PART_SSH>{});
 }
 
 template <int R, int OW, int PF>
@@ -182,6 +193,10 @@ void check_shape(const EnsShape &sh)
 //   FP32         1.0 M 22 / 25 / 28;  2.9 M 85 / 76 / 76;  7.2 M 211 / 202 / 211
 // The overlapped-wavefront tiles took 13, 33, 68, 180 (2.9 M) and 81 us (FP32,
 // 2.9 M), with a Flather launch after each step.
+// On the smallest two wavefronts share a tile, as in a single domain (one / two,
+// by row: 306 tiles FP64 4.1 / 3.4, FP32 3.2 / 2.7; 1193 tiles 5.7 / 5.3 and 3.9 /
+// 3.5).
+constexpr long kEnsSplitTilesByRowF64 = 1400, kEnsSplitTilesF64 = 600, kEnsSplitTilesF32 = 1950;
 constexpr long kEnsOneRowTilesByRowF64 = 3500, kEnsOneRowTilesF64 = 12000;
 constexpr long kEnsOneRowTilesF32 = 24000;
 constexpr long kEnsTwoRowTilesByRowF64 = 24000, kEnsCachedTilesF64 = 48000;
@@ -220,16 +235,19 @@ EnsBand ens_band_tiles(const EnsShape &sh, int precision, bool by_row, long one_
                        long two_row_tiles)
 {
     if (sh.rows != 4 || sh.cols != 0 || sh.prefetch != 2)
-        return EnsBand{sh.rows, sh.cols, sh.prefetch, false};
+        return EnsBand{sh.rows, sh.cols, sh.prefetch, false, false};
     const long one = precision == 32 ? kEnsOneRowTilesF32
                      : by_row        ? kEnsOneRowTilesByRowF64
                                      : kEnsOneRowTilesF64;
-    if (one_row_tiles <= one) return EnsBand{1, 61, 0, false};
-    if (precision == 32) return EnsBand{2, 61, 0, false};
+    const long split = precision == 32 ? kEnsSplitTilesF32
+                       : by_row        ? kEnsSplitTilesByRowF64
+                                       : kEnsSplitTilesF64;
+    if (one_row_tiles <= one) return EnsBand{1, 61, 0, false, one_row_tiles <= split};
+    if (precision == 32) return EnsBand{2, 61, 0, false, false};
     if (by_row)
-        return two_row_tiles <= kEnsTwoRowTilesByRowF64 ? EnsBand{2, 61, 0, false}
-                                                        : EnsBand{4, 0, 0, true};
-    return EnsBand{2, 61, 0, two_row_tiles > kEnsCachedTilesF64};
+        return two_row_tiles <= kEnsTwoRowTilesByRowF64 ? EnsBand{2, 61, 0, false, false}
+                                                        : EnsBand{4, 0, 0, true, false};
+    return EnsBand{2, 61, 0, two_row_tiles > kEnsCachedTilesF64, false};
 }
 
 template <typename T, typename In, typename Out>
@@ -239,17 +257,20 @@ void launch_band(hipStream_t s, const EnsBand &bt, const In &in, const T *tab,
 {
     if (ntiles <= 0) return;
     const band::Flather<T> fl{u_prev, v_prev, cu, cv, sizeof(T) == 8 || cu, T(0), T(0)};
-    const dim3 grid((unsigned)ntiles), block(64);
+    const dim3 grid((unsigned)(bt.split ? 2 * ntiles : ntiles)), block(64);
     auto run = [&](auto kernel) {
         kernel<<<grid, block, 0, s>>>(in, tab, p, out, fl, tiles, tide);
         NEMO_LAUNCH_CHECK();
     };
+    if (bt.split && bt.rows == 1)
+        return tab ? run(k_ens_band<T, true, 1, 0, false, 2>)
+                   : run(k_ens_band<T, false, 1, 0, false, 2>);
     if constexpr (sizeof(T) == 8) {
         if (bt.stream && bt.rows == 4 && tab) return run(k_ens_band<T, true, 4, 0, true>);
         if (bt.stream && bt.rows == 2 && !tab) return run(k_ens_band<T, false, 2, 0, true>);
     }
 #define NEMO_ENS_BAND(R, PF)                                                           \
-    if (bt.rows == R && bt.prefetch == PF && !bt.stream)                               \
+    if (bt.rows == R && bt.prefetch == PF && !bt.stream && !bt.split)                  \
         return tab ? run(k_ens_band<T, true, R, PF, false>)                            \
                    : run(k_ens_band<T, false, R, PF, false>);
     NEMO_ENS_BAND(1, 0)

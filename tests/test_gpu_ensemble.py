@@ -236,9 +236,10 @@ def test_ensemble_random_masks_match_oracle_and_mixed():
 
 @pytest.mark.parametrize("precision", [64, 32])
 @pytest.mark.parametrize("metrics", ["row", "point"])
-@pytest.mark.parametrize("sizes", [((3, 3), (40, 33), (130, 61)), ((61, 64), (700, 620)),
-                                   ((57, 4), (1101, 1400)), ((2501, 2403),)],
-                         ids=["one", "two", "more", "largest"])
+@pytest.mark.parametrize("sizes", [((3, 3), (40, 33), (130, 61)), ((300, 290), (200, 150)),
+                                   ((61, 64), (700, 620)), ((57, 4), (1101, 1400)),
+                                   ((2501, 2403),)],
+                         ids=["shared", "one", "two", "more", "largest"])
 def test_ensemble_default_tiles_equal_the_persistent_kernel(sizes, metrics, precision):
     """The default shape, whose tiles follow the ensemble's size, has the bits
     of the persistent kernel with its separate Flather launch, on random masks
