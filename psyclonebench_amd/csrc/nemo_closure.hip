@@ -106,7 +106,10 @@ __device__ __forceinline__ Band xcd_band(int items)
     return Band{first, last - first, (int)(blockIdx.x >> 3), (int)(gridDim.x >> 3)};
 }
 
-// 32 input and 32 output channels. (From 4 channels: k_conv_in.)
+// 32 output channels. KIND 1: 16 input channels, of which the 4 stored ones are
+// not zero (the output gradient). KIND 2: 32 input channels. (The network input
+// layer, 4 channels, is k_conv_in; for KIND 1 that form is 2 us faster at 512^2,
+// but its other order of summation flips roundings of the gradient to bf16.)
 // EPI_HIDDEN: bias, GELU, optional pre-activation; EPI_DX: times gelu'(gpre).
 // NT tiles per wavefront pass, WPB wavefronts per workgroup, two workgroups
 // per CU (the LDS weights):
@@ -116,13 +119,15 @@ __device__ __forceinline__ Band xcd_band(int items)
 //   LDS weight read per MFMA, twice the wavefronts to hide the activation
 //   loads and overlap one wavefront's epilogue with another's MFMAs.
 // Every tile sees the same MFMA sequence in both forms: the same bits.
-template <int EPI, int NT, int WPB>
+template <int KIND, int EPI, int NT, int WPB>
 __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(4 / NT, 4 / NT)))
 void k_conv_sh(ConvArgs a)
 {
     static_assert(EPI == EPI_HIDDEN || EPI == EPI_DX, "epilogue");
     static_assert((NT == 2 && WPB == 4) || (NT == 1 && WPB == 8), "launch form");
-    constexpr int NC = 2, CIN = 32;
+    static_assert(KIND == 1 || KIND == 2, "16 or 32 input channels");
+    constexpr int NC = KIND == 2 ? 2 : 1;
+    constexpr int CIN = KIND == 2 ? 32 : 16;
     constexpr int ROW = CIN + 8;  // LDS row of one output channel, padded by 8
     constexpr int NROWS = TAPS * 32;
     __shared__ __attribute__((aligned(16))) __bf16 wsh[NROWS * ROW];
@@ -157,7 +162,7 @@ void k_conv_sh(ConvArgs a)
 
     const int lane = (int)(threadIdx.x & 63), n = lane & 31, h = lane >> 5;
     const int nx = a.nx, Wp = nx + 4, T = (nx + 27) / 28;
-    constexpr int PXS = 16;  // elements per padded pixel of a plane
+    constexpr int PXS = KIND == 2 ? 16 : OUT4C;  // elements per padded pixel
     const size_t PL = plane_elems(nx, a.ny), RS = (size_t)Wp * PXS;  // row stride
     const Band bd = xcd_band(a.ny * T);
     const int wib = bd.local * WPB + (int)(threadIdx.x >> 6), nwb = bd.nlocal * WPB;
@@ -218,7 +223,7 @@ void k_conv_sh(ConvArgs a)
     // epilogue.
     int k = NT * wib;
     if (k >= bd.count) return;
-    const size_t coff = (size_t)h * 8;
+    const size_t coff = KIND == 2 ? (size_t)h * 8 : 0;
     // positions of the group at k, advanced by NT nwb items per group (no
     // division in the loop)
     const int step = NT * nwb, step_y = step / T, step_t = step - step_y * T;
@@ -257,8 +262,14 @@ void k_conv_sh(ConvArgs a)
         for (int c = 0; c < NC; c++) {
             const size_t o = (size_t)c * PL + (size_t)dy * RS;
 #pragma unroll
-            for (int j = 0; j < NT; j++)
-                buf[slot][c][j] = *reinterpret_cast<const bf16x8 *>(sp[j] + o);
+            for (int j = 0; j < NT; j++) {
+                if constexpr (KIND == 2)
+                    buf[slot][c][j] = *reinterpret_cast<const bf16x8 *>(sp[j] + o);
+                else
+                    buf[slot][c][j] = __builtin_shufflevector(
+                        *reinterpret_cast<const bf16x4 *>(sp[j] + o), bf16x4{}, 0, 1, 2, 3, 4, 5,
+                        6, 7);
+            }
         }
     };
     auto pair = [&](auto parity) __attribute__((always_inline)) {
@@ -288,16 +299,23 @@ void k_conv_sh(ConvArgs a)
             // channel-chunk-outer order: an accumulator comes back every
             // 5 NT MFMAs, past the latency of the previous one
 #pragma unroll
-            for (int c = 0; c < NC; c++)
+            for (int c = 0; c < NC; c++) {
+                bf16x8 x[NT];
+#pragma unroll
+                for (int j = 0; j < NT; j++) {
+                    x[j] = buf[(dy + P) & 1][c][j];
+                    if constexpr (KIND == 1) x[j] = h ? bf16x8{} : x[j];  // channels 8 .. 15
+                }
 #pragma unroll
                 for (int dx = 0; dx < 5; dx++) {
                     const bf16x8 w = *reinterpret_cast<const bf16x8 *>(
                         wsh + ((dy * 5 + dx) * 32 + n) * ROW + h * 8 + c * 16);
 #pragma unroll
                     for (int j = 0; j < NT; j++)
-                        acc[j][dx] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                            w, buf[(dy + P) & 1][c][j], acc[j][dx], 0, 0, 0);
+                        acc[j][dx] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, x[j], acc[j][dx],
+                                                                             0, 0, 0);
                 }
+            }
         }
         finish_group(cur, k);
         k += NT * nwb;
@@ -313,8 +331,7 @@ void k_conv_sh(ConvArgs a)
     }
 }
 
-// 32 channels from 4: the network input layer (EPI_HIDDEN) and the input
-// gradient of the output layer (EPI_DX), as an implicit GEMM with the taps in
+// Network input layer (4 -> 32 channels) as an implicit GEMM with the taps in
 // K: 25 taps x 4 channels (100, padded to 112 = 7 chunks of 16), so one
 // accumulator holds the whole 5x5 sum of a 32-pixel tile and no horizontal
 // shift-sum or tile overlap is needed. Each half h of the wavefront carries
@@ -329,8 +346,7 @@ void k_conv_sh(ConvArgs a)
 // the kernel keeps its registers under 128 for 4 wavefronts per SIMD
 // instead of sharing one loaded fragment among five accumulators. Tiles sit
 // at x0 = min(32 t, nx - 32); the last one overlaps its neighbour and stores
-// only x >= 32 t. The output layer's gradient, stored in 4 channels as well,
-// takes 14.0 us at 512^2 here, 15.9 with 16 channels in the shift-sum form.
+// only x >= 32 t.
 constexpr int IN_CHUNKS = 7;
 
 // Kernel tap (dy * 5 + dx) of chunk c, half h, slot q; -1: a zero K slot.
@@ -341,20 +357,15 @@ __device__ __forceinline__ int in_tap(int c, int h, int q)
     return h == 0 && q == 0 ? 24 : -1;
 }
 
-template <int EPI>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_conv_in(
     ConvArgs a)
 {
-    static_assert(EPI == EPI_HIDDEN || EPI == EPI_DX, "epilogue");
-    static_assert(CIN0 == COUT4, "one stride of the weights");
     // the bias sits in LDS: an LDS read in the epilogue waits on the LDS
     // counter only, where a global load would wait for every store and
     // every prefetched fragment before it
     __shared__ __attribute__((aligned(16))) float bsh[HID];
-    if constexpr (EPI == EPI_HIDDEN) {
-        if (threadIdx.x < HID) bsh[threadIdx.x] = a.bias[threadIdx.x];
-        __syncthreads();
-    }
+    if (threadIdx.x < HID) bsh[threadIdx.x] = a.bias[threadIdx.x];
+    __syncthreads();
     const int lane = (int)(threadIdx.x & 63), n = lane & 31, h = lane >> 5;
     const int nx = a.nx, Wp = nx + 4, T = (nx + 31) / 32;
     const size_t PL = plane_elems(nx, a.ny);
@@ -445,23 +456,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
             for (int g = 0; g < 4; g++) {
                 const int co = g * 8 + h * 4;
                 const size_t o = (size_t)(co >> 4) * PL + px + (co & 15);
-                bf16x4 r;
-                if constexpr (EPI == EPI_HIDDEN) {
-                    const f32x4 bias = *reinterpret_cast<const f32x4 *>(&bsh[co]);
-                    bf16x4 p;
+                const f32x4 bias = *reinterpret_cast<const f32x4 *>(&bsh[co]);
+                bf16x4 p, r;
 #pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const float v = acc[4 * g + j] + bias[j];
-                        p[j] = (__bf16)v;
-                        r[j] = (__bf16)gelu(v);
-                    }
-                    if (a.pre) *reinterpret_cast<bf16x4 *>(a.pre + o) = p;
-                } else {
-                    const bf16x4 gp = *reinterpret_cast<const bf16x4 *>(a.gpre + o);
-#pragma unroll
-                    for (int j = 0; j < 4; j++)
-                        r[j] = (__bf16)(acc[4 * g + j] * gelu_grad((float)gp[j]));
+                for (int j = 0; j < 4; j++) {
+                    const float v = acc[4 * g + j] + bias[j];
+                    p[j] = (__bf16)v;
+                    r[j] = (__bf16)gelu(v);
                 }
+                if (a.pre) *reinterpret_cast<bf16x4 *>(a.pre + o) = p;
                 *reinterpret_cast<bf16x4 *>(a.out + o) = r;
             }
         }
@@ -1254,19 +1257,21 @@ void launch_conv(hipStream_t s, int cin, int cout, Epilogue epi, const ConvArgs 
     const dim3 grid = conv_grid(2), block(256), block8(512);
     const bool one = g_conv_form == 1;
     if (cin == 16 && cout == 32 && epi == EPI_HIDDEN)  // the network input: 4 used channels
-        k_conv_in<EPI_HIDDEN><<<conv_grid(4), block, 0, s>>>(a);
+        k_conv_in<<<conv_grid(4), block, 0, s>>>(a);
     else if (cin == 32 && cout == 32 && epi == EPI_HIDDEN && one)
-        k_conv_sh<EPI_HIDDEN, 1, 8><<<grid, block8, 0, s>>>(a);
+        k_conv_sh<2, EPI_HIDDEN, 1, 8><<<grid, block8, 0, s>>>(a);
     else if (cin == 32 && cout == 32 && epi == EPI_HIDDEN)
-        k_conv_sh<EPI_HIDDEN, 2, 4><<<grid, block, 0, s>>>(a);
+        k_conv_sh<2, EPI_HIDDEN, 2, 4><<<grid, block, 0, s>>>(a);
     else if (cin == 32 && cout == 16 && epi == EPI_OUTPUT)
         k_conv_out<false><<<out_grid(a.nx, a.ny), block, 0, s>>>(a, GuardSums{});
-    else if (cin == 16 && cout == 32 && epi == EPI_DX)  // 4 stored channels
-        k_conv_in<EPI_DX><<<conv_grid(4), block, 0, s>>>(a);
+    else if (cin == 16 && cout == 32 && epi == EPI_DX && one)
+        k_conv_sh<1, EPI_DX, 1, 8><<<grid, block8, 0, s>>>(a);
+    else if (cin == 16 && cout == 32 && epi == EPI_DX)
+        k_conv_sh<1, EPI_DX, 2, 4><<<grid, block, 0, s>>>(a);
     else if (cin == 32 && cout == 32 && epi == EPI_DX && one)
-        k_conv_sh<EPI_DX, 1, 8><<<grid, block8, 0, s>>>(a);
+        k_conv_sh<2, EPI_DX, 1, 8><<<grid, block8, 0, s>>>(a);
     else if (cin == 32 && cout == 32 && epi == EPI_DX)
-        k_conv_sh<EPI_DX, 2, 4><<<grid, block, 0, s>>>(a);
+        k_conv_sh<2, EPI_DX, 2, 4><<<grid, block, 0, s>>>(a);
     else
         NEMO_FATAL("closure conv: unsupported %d -> %d channels, epilogue %d", cin, cout,
                    (int)epi);
