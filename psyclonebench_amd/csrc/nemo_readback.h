@@ -15,6 +15,7 @@
 #include <algorithm>
 #include <atomic>
 #include <exception>
+#include <mutex>
 #include <thread>
 #include <vector>
 
@@ -39,6 +40,8 @@ public:
     void read(hipStream_t s, const float *hi, const float *lo, size_t n, double *out)
     {
         if (n == 0) return;
+        // threads may read one handle at the same time; they share the stage
+        const std::lock_guard<std::mutex> one(mutex_);
         if (!stage_) {
             NEMO_HIP_CHECK(hipHostMalloc((void **)&stage_, kSlots * 2 * kChunk * sizeof(float),
                                          hipHostMallocDefault));
@@ -110,6 +113,7 @@ private:
     struct alignas(64) Done {
         std::atomic<size_t> chunks{0};
     };
+    std::mutex mutex_;
     float *stage_ = nullptr;
     hipEvent_t ready_[kSlots] = {};
 };

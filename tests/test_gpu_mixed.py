@@ -6,6 +6,8 @@ relmax = max|F - F_ref| / max|F_ref|, relrms = ||F - F_ref||_2 / ||F_ref||_2.
 Tolerances are stated in each test."""
 from __future__ import annotations
 
+from dataclasses import replace
+
 import numpy as np
 import pytest
 
@@ -192,4 +194,18 @@ def test_read_back_of_the_uploaded_state(nx, ny):
     hi = s.astype(np.float32)
     lo = (s - hi.astype(np.float64)).astype(np.float32)
     assert_bitwise(st.fetch("sshn_t"), hi.astype(np.float64) + lo.astype(np.float64), "sshn_t")
+    st.release()
+
+
+def test_threads_read_one_handle_at_the_same_time():
+    """Four threads read the fields of one handle over and over; every record
+    is the one that a single thread reads."""
+    from concurrent.futures import ThreadPoolExecutor
+    st = MixedStepper(Model(replace(c1_config(4), jpiglo=702, jpjglo=602)))
+    st.run(4)
+    names = ("sshn_t", "un", "vn", "sshn_u")
+    ref = {n: st.fetch(n) for n in names}
+    with ThreadPoolExecutor(4) as pool:
+        for n, got in zip(names * 5, pool.map(st.fetch, names * 5)):
+            assert_bitwise(got, ref[n], n)
     st.release()
