@@ -358,10 +358,13 @@ void run_steps(Context &C, int nsteps, int istep, hipStream_t s,
         if (nsteps == 0) return;
     }
     ensure_tide_table(C, nsteps);
-    // The table costs one pass over 13 arrays and saves about that much a
-    // step, so a single step goes without (20 steps at 4096^2: 0.3 of 8.3 ms).
+    // The table costs a launch, a wait (some 18 us together) and one pass over 13
+    // arrays, and saves about 15 us a step per million points: worth it from 2
+    // million points in all (4 steps at 400^2 95 us without, 102 with).
     bool by_row = false;
-    if (g_fused_variant == kDefaultVariant && nsteps > 1) by_row = metrics_by_row(C, s);
+    const long points = (long)(C.G.xe - C.G.xs + 1) * (C.G.ye - C.G.ys + 1);
+    if (g_fused_variant == kDefaultVariant && nsteps > 1 && points * nsteps >= 2000000)
+        by_row = metrics_by_row(C, s);
     NEMO_HIP_CHECK(hipStreamSynchronize(s));  // h_tide may still be in flight
     for (int k = 0; k < nsteps; k++) C.h_tide[k] = tide_at(istep + k, C.P.rdt);
     NEMO_HIP_CHECK(hipMemcpyAsync(C.d_tide, C.h_tide, (size_t)nsteps * sizeof(double),
