@@ -148,6 +148,10 @@ NEMO_API void nemo_hip_set_mode(int mode);
 /* Form in use by the context whose first slot is ssha_t_device:
  * 1 unfused, 2 fused, 0 no such context. */
 NEMO_API int nemo_hip_context_mode(void **ssha_t_device);
+/* 1 when the last fused steps of these slots' context read the metrics as one
+ * record a row (see nemo_hip_set_fused_variant), 0 when they read the arrays,
+ * -1 before the first step. */
+NEMO_API int nemo_hip_metrics_by_row(void **ssha_t_device);
 
 /* Waits for all queued work of the library. */
 NEMO_API void nemo_hip_synchronize(void);

@@ -88,6 +88,8 @@ def hip_lib() -> C.CDLL:
         lib.nemo_hip_set_mode.argtypes = [C.c_int]
         lib.nemo_hip_context_mode.argtypes = [_vpp]
         lib.nemo_hip_context_mode.restype = C.c_int
+        lib.nemo_hip_metrics_by_row.argtypes = [_vpp]
+        lib.nemo_hip_metrics_by_row.restype = C.c_int
         lib.nemo_hip_set_kernel_timing.argtypes = [C.c_int]
         lib.nemo_hip_fused_kernel_ms.restype = C.c_double
         lib.nemo_hip_set_fused_variant.argtypes = [C.c_int]

@@ -73,6 +73,7 @@ struct Context {
     double *row_tab = nullptr;
     int *row_bad = nullptr;
     int row_mark = 0;
+    bool by_row = false;  // the last steps read the table
     // n, parity, variant, metrics by row, hook key (0: plain steps)
     std::map<std::tuple<int, int, int, bool, unsigned long long>, hipGraphExec_t> graphs;
     void **slots[A_COUNT] = {};  // the caller's slots of the last call
@@ -288,6 +289,7 @@ void run_hook(const Context &C, const StepHook *hook, hipStream_t s)
 
 void step_fused(Context &C, int istep, hipStream_t s, const StepHook *hook = nullptr)
 {
+    C.by_row = false;
     launch_fused_pair(C, C.parity, s, nullptr, 0, tide_at(istep, C.P.rdt), false);
     C.parity = 1 - C.parity;
     run_hook(C, hook, s);
@@ -365,6 +367,7 @@ void run_steps(Context &C, int nsteps, int istep, hipStream_t s,
     const long points = (long)(C.G.xe - C.G.xs + 1) * (C.G.ye - C.G.ys + 1);
     if (g_fused_variant == kDefaultVariant && nsteps > 1 && points * nsteps >= 2000000)
         by_row = metrics_by_row(C, s);
+    C.by_row = by_row;
     NEMO_HIP_CHECK(hipStreamSynchronize(s));  // h_tide may still be in flight
     for (int k = 0; k < nsteps; k++) C.h_tide[k] = tide_at(istep + k, C.P.rdt);
     NEMO_HIP_CHECK(hipMemcpyAsync(C.d_tide, C.h_tide, (size_t)nsteps * sizeof(double),
@@ -635,6 +638,12 @@ int nemo_hip_context_mode(void **ssha_t_device)
 {
     auto it = g_contexts.find(ssha_t_device);
     return it == g_contexts.end() ? 0 : it->second->mode;
+}
+
+int nemo_hip_metrics_by_row(void **ssha_t_device)
+{
+    auto it = g_contexts.find(ssha_t_device);
+    return it == g_contexts.end() ? -1 : it->second->by_row ? 1 : 0;
 }
 
 void nemo_hip_synchronize(void) { NEMO_HIP_CHECK(hipStreamSynchronize(lib_stream())); }

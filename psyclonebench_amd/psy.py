@@ -101,6 +101,13 @@ class TimeStepper:
                       C.POINTER(C.c_void_p))
         return hip_lib().nemo_hip_context_mode(slot)
 
+    @property
+    def metrics_by_row(self) -> bool:
+        """Whether the last steps read the metrics as one record a row."""
+        slot = C.cast(C.byref(self.model.fields["ssha_t"].device_ptr),
+                      C.POINTER(C.c_void_p))
+        return hip_lib().nemo_hip_metrics_by_row(slot) == 1
+
     def fetch(self, name: str):
         """Host copy of a field (blocking read-back)."""
         return self.model.fields[name].get_data().copy()

@@ -1,0 +1,134 @@
+"""The table of metrics by row of the FP64 step, in calls long enough to use it
+(a call takes it from 2 million points in all): the tiles that read it, the
+rows whose numerators leave the range of its quotients, the divisors that it
+refuses and metrics written between two calls. Each test asserts which form
+ran; the oracle's bits are the bar."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+from helpers import assert_bitwise
+from psyclonebench_amd import _native
+from psyclonebench_amd.psy import TimeStepper
+from test_gpu_band import check, live_model, oracle_steps
+from test_zz_no_alloc import OUT as INPLACE, TOL, _run_noalloc
+
+pytestmark = pytest.mark.gpu
+
+QUICK_MIN = 2.0 ** -900  # smallest numerator of the table's quotients
+
+
+@pytest.fixture(autouse=True)
+def _release():
+    yield
+    _native.hip_lib().nemo_hip_release_all()
+
+
+def steps_of(nx: int, ny: int) -> int:
+    """Steps of a call that uses the table, at least two."""
+    return max(2, -(-2000000 // (nx * ny)))
+
+
+def run_both(m, what: str, by_row: bool = True):
+    """One step, then a call long enough for the table, against the oracle."""
+    m.cfg.rdt = 0.05  # the random state stays finite for some 50 steps
+    n = 1 + steps_of(m.grid.M - 2, m.grid.N - 2)
+    ref = oracle_steps(m, [a.copy() for a in m.arrays()], 1, n)
+    assert all(np.isfinite(ref[k]).all() for k in INPLACE), "the test's own state overflows"
+    st = TimeStepper(m.copy(), mode=2)
+    st.run(n)
+    assert st.metrics_by_row == by_row, what
+    check(st, ref, what)
+    return ref
+
+
+# two wavefronts a tile (up to 1400 tiles); one row (up to 3500); two rows (up
+# to 24000 of two); eight rows: odd extents on both sides of the lines
+@pytest.mark.parametrize("nx, ny", [(120, 401), (121, 402), (301, 232), (301, 299),
+                                    (420, 300), (701, 290), (701, 403), (1501, 1200),
+                                    (2301, 1260), (2501, 1403)])
+def test_tiles_by_row_equal_oracle(nx, ny):
+    print("by row", nx, ny, flush=True)
+    run_both(live_model(nx, ny, "row", seed=31), f"{nx}x{ny}")
+
+
+@pytest.mark.parametrize("nx, ny", [(301, 232), (420, 300), (701, 403), (2501, 1403)])
+def test_numerators_outside_the_quick_range_equal_oracle(nx, ny):
+    """Basins of 12 columns behind dry ones, whose states fall from size 1 to
+    10^-316 (subnormal) across the grid, with exact and signed zeros: tiles of
+    one, two and eight rows redo rows with plain divisions."""
+    print("falling basins", nx, ny, flush=True)
+    m = live_model(nx, ny, "row", seed=32)
+    g = m.grid
+    column = np.arange(g.W)
+    g.tmask[:, column % 13 == 12] = 0
+    fall = 10.0 ** (-316.0 * (column // 13) / (g.W // 13))[None, :]
+    for n in ("ssha_t", "sshn_t", "sshn_u", "sshn_v", "un", "vn", "ua", "va"):
+        m.array(n)[:] *= fall
+    m.array("un")[20:40] = 0.0
+    m.array("vn")[30:50] = -0.0
+    m.cfg.tide_amp = 0.0
+
+    def below(u):  # differences of two wet points of a column, a numerator of the step
+        wet = (g.tmask[1:, :] > 0) & (g.tmask[:-1, :] > 0)
+        d = np.abs(u[1:] - u[:-1])[wet]
+        return int(((d > 0.0) & (d < QUICK_MIN)).sum())
+
+    assert below(m.array("un")) > 1000
+    ref = run_both(m, f"falling basins {nx}x{ny}")
+    assert below(ref["ua"]) > 1000  # still out of the range after the last step
+
+
+@pytest.mark.parametrize("name, value", [(None, 0.0), ("area_u", 3e30), ("dx_t", 1e35),
+                                         ("area_v", 2e30), ("dy_t", 1e-31)])
+def test_divisors_outside_the_table_equal_oracle(name, value):
+    """One row of a divisor out of 2^+-100: the call reads the arrays."""
+    m = live_model(1301, 800, "row", seed=33)
+    if name:
+        m.array(name)[417] = value
+    run_both(m, f"{name} {value}", by_row=name is None)
+
+
+def test_metrics_written_between_calls_are_seen():
+    """Between calls that read the metrics by row: one point of one metric
+    changed on the device (the next call reads the arrays), the point put back,
+    then a whole row changed (the table of the next calls is a new one)."""
+    m = live_model(701, 403, "row", seed=34)
+    g, lib, n = m.grid, _native.hip_lib(), steps_of(701, 403)
+    host = [a.copy() for a in m.arrays()]
+    m.cfg.rdt = 0.05
+    st = TimeStepper(m.copy(), mode=2)
+    st.run(1)
+    oracle_steps(m, host, 1, 1)
+    a = host[oracle.ARRAY_NAMES.index("dx_v")]
+    point, row = a[33, 101], a[57, 0]
+    done = 1
+    for what, sl, value, by_row in (
+            ("unchanged", (0, 0), a[0, 0], True),
+            ("one point", (33, 101), 1.25 * point, False),
+            ("put back", (33, 101), point, True),
+            ("one row", (57, slice(None)), 0.75 * row, True)):
+        a[sl] = value
+        lib.c_write_to_device(a.ctypes.data, st.grid_slots.slots["dx_v"], 1, 1, g.W, g.H, True)
+        st.run(n)
+        ref = oracle_steps(m, host, done + 1, n)
+        done += n
+        assert st.metrics_by_row == by_row, what
+        check(st, ref, what)
+
+
+@pytest.mark.parametrize("nx, ny", [(3, 3), (61, 40), (509, 130), (1201, 900)])
+def test_inplace_step_at_random_latitudes(nx, ny):
+    """The allocation-free step at the sizes of its one- and two-row bands, with
+    the latitudes of every point random: the device's sine against libm's, so
+    the bound is the FP64 step's."""
+    m = live_model(nx, ny, "point", seed=35)
+    _native.hip_lib().nemo_hip_set_tide(m.cfg.tide_amp, m.cfg.tide_omega)
+    ref = oracle_steps(m, [a.copy() for a in m.arrays()], 1, 2)
+    got = _run_noalloc(m.copy(), 1, 2)
+    for n in INPLACE:
+        rel = float(np.max(np.abs(got[n] - ref[n]))) / float(np.max(np.abs(ref[n])))
+        print(f"{nx}x{ny} {n}: relmax {rel:.2e}", flush=True)
+        assert rel <= TOL
