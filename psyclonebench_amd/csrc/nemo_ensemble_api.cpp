@@ -86,6 +86,7 @@ struct EnsContext {
     // k * kArenaStagger bytes into its allocation
     std::vector<void *> raw;
 
+    double fric() const { return 1.0 + P.cbfr * P.rdt; }
     size_t esize() const { return prec == 64 ? sizeof(double) : sizeof(float); }
 
     StepIn<double> in64(int s) const
@@ -351,8 +352,9 @@ void build_flather_lists(EnsContext &C, void *const *arrays, hipStream_t s)
 }
 
 // The tables of metrics by row of every domain; dropped when one domain has
-// none. The arenas are the ensemble's own and do not change, so one look at
-// creation stands.
+// none (or, in FP64, the friction divisor is out of the table's range). The
+// arenas are the ensemble's own and do not change, so one look at creation
+// stands.
 template <typename T, typename In>
 void build_row_tables(EnsContext &C, const In &in, hipStream_t s)
 {
@@ -361,6 +363,7 @@ void build_row_tables(EnsContext &C, const In &in, hipStream_t s)
         C.rec.push_back((int)(values / kRowTableWidth));
         values += row_table_values(Bounds{e.xs, e.xe, e.ys, e.ye});
     }
+    if (sizeof(T) == 8 && !table_divisor(C.fric())) return;
     T *const tab = dev_alloc<T>(values);
     C.row_tab = tab;
     int *bad = dev_alloc<int>(1), host_bad = 0;
@@ -422,7 +425,7 @@ void launch_pair(EnsContext &C, int par, int row, hipStream_t s, hipEvent_t e0 =
         ens_band_tiles(sh, C.prec, C.row_tab != nullptr, C.one_row_tiles, C.two_row_tiles);
     if (e0) NEMO_HIP_CHECK(hipEventRecord(e0, s));
     if (C.prec == 64) {
-        const StepScalars<double> p{C.P.rdt, C.P.visc, C.P.g, 1.0 + C.P.cbfr * C.P.rdt};
+        const StepScalars<double> p{C.P.rdt, C.P.visc, C.P.g, C.fric()};
         if (band)
             launch_ens_band(s, bt, C.in64(par), static_cast<const double *>(C.row_tab), p,
                             C.out64(q), static_cast<const double *>(C.prog[prev][2]),
@@ -432,7 +435,7 @@ void launch_pair(EnsContext &C, int par, int row, hipStream_t s, hipEvent_t e0 =
             launch_ens_f64(s, sh, C.in64(par), p, C.out64(q), L.first, L.second, tide);
     } else {
         const StepScalars<float> p{(float)C.P.rdt, (float)C.P.visc, (float)C.P.g,
-                                   (float)(1.0 + C.P.cbfr * C.P.rdt)};
+                                   (float)C.fric()};
         if (band)
             launch_ens_band(s, bt, C.in32(par), static_cast<const float *>(C.row_tab), p,
                             C.out32(q), static_cast<const float *>(C.prog[prev][2]),

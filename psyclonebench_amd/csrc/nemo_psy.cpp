@@ -267,8 +267,7 @@ void launch_fused_pair(Context &C, int par, hipStream_t s, const double *tide_ta
 bool metrics_by_row(Context &C, hipStream_t s)
 {
     const Bounds bd{C.G.xs, C.G.xe, C.G.ys, C.G.ye};
-    const int e_fric = std::ilogb(C.scalars().fric);  // INT_MAX / INT_MIN: inf, NaN, 0
-    if (e_fric < -kDivisorExp || e_fric > kDivisorExp) return false;
+    if (!table_divisor(C.scalars().fric)) return false;
     if (!C.row_tab) {
         C.row_tab = dev_alloc<double>(row_table_values(bd));
         NEMO_HIP_CHECK(hipHostMalloc((void **)&C.row_bad, sizeof(int), hipHostMallocDefault));

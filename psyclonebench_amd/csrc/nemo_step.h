@@ -4,6 +4,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cmath>
+
 #include "nemo_point.h"
 
 namespace nemo {
@@ -104,6 +106,12 @@ const char *march_variant_kernel(int variant);
 // (memory that the device can write) when they do vary or a divisor is out of
 // the table's range (2^+-kDivisorExp).
 constexpr int kDivisorExp = 100;
+// The same for a divisor that the host knows: the friction factor of the step.
+inline bool table_divisor(double d)
+{
+    const int e = std::ilogb(d);  // INT_MAX / INT_MIN: inf, NaN, 0
+    return e >= -kDivisorExp && e <= kDivisorExp;
+}
 constexpr int kRowTableWidth = 32;  // values a record
 size_t row_table_values(const Bounds &b);
 void launch_row_metrics(hipStream_t s, const StepIn<double> &f, int W, unsigned base,
