@@ -51,8 +51,10 @@ struct EnsShape {
 // columns and prefetch depth.
 bool ens_shape_supported(const EnsShape &shape);
 
-// Shapes that run band tiles (nemo_band.h): no Flather launch follows them.
-bool ens_band(const EnsShape &shape);
+// Whether a shape runs band tiles (nemo_band.h), which no Flather launch
+// follows, on an ensemble with metrics by row or not and with that many tiles
+// of one row.
+bool ens_band(const EnsShape &shape, int precision, bool by_row, long one_row_tiles);
 
 // Tiles of a band shape. The shape of a new ensemble (4 rows, columns per
 // domain, prefetch 2) leaves them to the library, which picks them by the

@@ -10,9 +10,10 @@
 //
 //  * one wavefront per tile: a grid of one-wavefront workgroups, one per
 //    tile of the list, as the single-domain kernels launch, so that the
-//    dispatcher starts a new tile wherever a wavefront slot frees up. Bands
-//    of up to 8 rows are band tiles (nemo_band.h), which write the Flather
-//    faces themselves; 16-row ones run wave::tile_f64 / tile_mixed;
+//    dispatcher starts a new tile wherever a wavefront slot frees up. The
+//    default shape, and bands of 4 and 8 rows where they are the faster
+//    (ens_band), are band tiles (nemo_band.h), which write the Flather faces
+//    themselves; the others run wave::tile_f64 / tile_mixed;
 //  * persistent: a fixed number of workgroups (a multiple of 8) of 1, 2 or
 //    4 wavefronts; every wavefront takes tiles from the list with a stride,
 //    so uneven domain sizes cost nothing but the partial tiles at their
@@ -50,14 +51,23 @@ __device__ __forceinline__ Walk walk(int ntiles)
     return Walk{t0 + k * wpb + wave, min(t0 + chunk, ntiles), per * wpb};
 }
 
+// Tile `tl` of the FP64 step; OW = 0 takes the tile width from the tile
+// (wavefront-uniform branch between the 61- and 56-column bodies).
 template <int R, int OW, int PF>
 __device__ __forceinline__ void ens_tile_f64(const StepIn<double> &f,
                                              const StepScalars<double> &p,
                                              const StepOut<double> &o, const EnsTile &tl,
                                              double tide)
 {
-    wave::tile_f64<R, OW, PF>(f, p, o, tl.W, tl.off, Bounds{tl.xs, tl.xe, tl.ys, tl.ye},
-                              tl.strip, tl.band, tide);
+    if constexpr (OW == 0) {
+        if (tl.cols == 61)
+            ens_tile_f64<R, 61, PF>(f, p, o, tl, tide);
+        else
+            ens_tile_f64<R, 56, PF>(f, p, o, tl, tide);
+    } else {
+        wave::tile_f64<R, OW, PF>(f, p, o, tl.W, tl.off, Bounds{tl.xs, tl.xe, tl.ys, tl.ye},
+                                  tl.strip, tl.band, tide);
+    }
 }
 
 template <int R, int OW, int PF>
@@ -65,8 +75,15 @@ __device__ __forceinline__ void ens_tile_mixed(const MixedIn &f, const StepScala
                                                const MixedOut &o, const EnsTile &tl,
                                                double tide)
 {
-    wave::tile_mixed<R, OW, PF>(f, p, o, tl.W, tl.off, Bounds{tl.xs, tl.xe, tl.ys, tl.ye},
-                                tl.strip, tl.band, wave::split(tide));
+    if constexpr (OW == 0) {
+        if (tl.cols == 61)
+            ens_tile_mixed<R, 61, PF>(f, p, o, tl, tide);
+        else
+            ens_tile_mixed<R, 56, PF>(f, p, o, tl, tide);
+    } else {
+        wave::tile_mixed<R, OW, PF>(f, p, o, tl.W, tl.off, Bounds{tl.xs, tl.xe, tl.ys, tl.ye},
+                                    tl.strip, tl.band, wave::split(tide));
+    }
 }
 
 // Band tile, one wavefront each, or two that share it (SPLIT = 2: u; v and ssh);
@@ -176,7 +193,13 @@ void check_shape(const EnsShape &sh)
     X(4, 61, 0) X(8, 61, 0) X(16, 61, 0) X(32, 61, 0) X(64, 61, 0) X(4, 56, 0)         \
     X(8, 56, 0) X(16, 56, 0) X(32, 56, 0) X(64, 56, 0) X(4, 61, 1) X(8, 61, 1)         \
     X(16, 61, 1) X(4, 56, 1) X(8, 56, 1) X(16, 56, 1)
-#define NEMO_ENS_GRID(X) X(16, 61, 0) X(16, 56, 0) X(16, 61, 1) X(16, 56, 1)
+#define NEMO_ENS_GRID(X)                                                               \
+    X(4, 61, 1) X(4, 56, 1) X(4, 0, 1) X(4, 61, 2) X(4, 56, 2) X(8, 61, 0) X(8, 56, 0)  \
+    X(8, 0, 0) X(8, 61, 1) X(8, 56, 1) X(8, 0, 1) X(8, 61, 2) X(8, 56, 2) X(8, 0, 2)    \
+    X(16, 61, 0) X(16, 56, 0) X(16, 61, 1) X(16, 56, 1)
+// shapes whose tiles are always band tiles: 4 rows without prefetch, and the
+// default one
+#define NEMO_ENS_BAND_ONLY(X) X(4, 61, 0) X(4, 56, 0) X(4, 0, 0) X(4, 0, 2)
 
 // Tiles of the default shape, by how many bands of one and of two rows there
 // are (the reasons are those of the single domain: a wavefront with a SIMD to
@@ -201,6 +224,23 @@ constexpr long kEnsOneRowTilesByRowF64 = 3500, kEnsOneRowTilesF64 = 12000;
 constexpr long kEnsOneRowTilesF32 = 24000;
 constexpr long kEnsTwoRowTilesByRowF64 = 24000, kEnsCachedTilesF64 = 48000;
 
+// Shapes asked for by rows and prefetch run band tiles where these are the
+// faster. Time of a step with the overlapped-wavefront tile (and its Flather
+// launch) over that with the band tile, over ensembles of 146 to 73 thousand
+// one-row tiles:
+//   by row     every FP64 shape 1.00 .. 1.8, FP32 4 rows 1.04 .. 1.9, 8 rows
+//              without prefetch 1.08 .. 1.8; with it 0.89 .. 1.02 up to 9659
+//              tiles, 1.04 .. 1.6 from 22581
+//   by point   4 rows without prefetch 0.97 .. 1.2; with it 1.01 .. 1.07 up to
+//              2841 tiles, 0.93 .. 1.01 from 9659; 8 rows FP64 0.65 .. 1.03,
+//              FP32 without prefetch 1.02 .. 1.15 up to 2841 tiles and 0.90 ..
+//              1.02 from 5092, with it 0.75 .. 0.94
+constexpr long kEnsBandByRowTilesF32 = 10000, kEnsBandByPointTiles = 4000;
+
+bool default_shape(const EnsShape &sh)
+{
+    return sh.blocks == 0 && sh.rows == 4 && sh.cols == 0 && sh.prefetch == 2;
+}
 
 void unsupported(const EnsShape &sh)
 {
@@ -219,22 +259,28 @@ bool ens_shape_supported(const EnsShape &sh)
         NEMO_ENS_PERSISTENT(NEMO_ENS_HAS)
     } else {
         NEMO_ENS_GRID(NEMO_ENS_HAS)
+        NEMO_ENS_BAND_ONLY(NEMO_ENS_HAS)
     }
 #undef NEMO_ENS_HAS
-    return ens_band(sh);
+    return false;
 }
 
-bool ens_band(const EnsShape &sh)
+bool ens_band(const EnsShape &sh, int precision, bool by_row, long one_row_tiles)
 {
-    return sh.blocks == 0 && (sh.rows == 4 || sh.rows == 8) &&
-           (sh.cols == 61 || sh.cols == 56 || sh.cols == 0) && sh.prefetch >= 0 &&
-           sh.prefetch <= 2;
+    if (default_shape(sh)) return true;
+    if (sh.blocks || (sh.rows != 4 && sh.rows != 8)) return false;
+    if (sh.rows == 4 && sh.prefetch == 0) return true;
+    if (by_row)
+        return precision == 64 || sh.rows == 4 || sh.prefetch == 0 ||
+               one_row_tiles > kEnsBandByRowTilesF32;
+    return one_row_tiles <= kEnsBandByPointTiles &&
+           (sh.rows == 4 || (precision == 32 && sh.prefetch == 0));
 }
 
 EnsBand ens_band_tiles(const EnsShape &sh, int precision, bool by_row, long one_row_tiles,
                        long two_row_tiles)
 {
-    if (sh.rows != 4 || sh.cols != 0 || sh.prefetch != 2)
+    if (!default_shape(sh))
         return EnsBand{sh.rows, sh.cols, sh.prefetch, false, false};
     const long one = precision == 32 ? kEnsOneRowTilesF32
                      : by_row        ? kEnsOneRowTilesByRowF64
@@ -269,18 +315,26 @@ void launch_band(hipStream_t s, const EnsBand &bt, const In &in, const T *tab,
         if (bt.stream && bt.rows == 4 && tab) return run(k_ens_band<T, true, 4, 0, true>);
         if (bt.stream && bt.rows == 2 && !tab) return run(k_ens_band<T, false, 2, 0, true>);
     }
-#define NEMO_ENS_BAND(R, PF)                                                           \
-    if (bt.rows == R && bt.prefetch == PF && !bt.stream && !bt.split)                  \
-        return tab ? run(k_ens_band<T, true, R, PF, false>)                            \
-                   : run(k_ens_band<T, false, R, PF, false>);
-    NEMO_ENS_BAND(1, 0)
-    NEMO_ENS_BAND(2, 0)
-    NEMO_ENS_BAND(4, 0)
-    NEMO_ENS_BAND(4, 1)
-    NEMO_ENS_BAND(4, 2)
-    NEMO_ENS_BAND(8, 0)
-    NEMO_ENS_BAND(8, 1)
-    NEMO_ENS_BAND(8, 2)
+#define NEMO_ENS_BAND(R, PF, BY_ROW)                                                   \
+    if (bt.rows == R && bt.prefetch == PF && !bt.stream && !bt.split &&                \
+        (tab != nullptr) == BY_ROW)                                                    \
+        return run(k_ens_band<T, BY_ROW, R, PF, false>);
+    NEMO_ENS_BAND(1, 0, true)
+    NEMO_ENS_BAND(1, 0, false)
+    NEMO_ENS_BAND(2, 0, true)
+    NEMO_ENS_BAND(2, 0, false)
+    NEMO_ENS_BAND(4, 0, true)
+    NEMO_ENS_BAND(4, 0, false)
+    NEMO_ENS_BAND(4, 1, true)
+    NEMO_ENS_BAND(4, 1, false)
+    NEMO_ENS_BAND(4, 2, true)
+    NEMO_ENS_BAND(4, 2, false)
+    NEMO_ENS_BAND(8, 0, true)
+    NEMO_ENS_BAND(8, 1, true)
+    NEMO_ENS_BAND(8, 2, true)
+    if constexpr (sizeof(T) == 4) {
+        NEMO_ENS_BAND(8, 0, false)
+    }
 #undef NEMO_ENS_BAND
     NEMO_FATAL("ensemble launch: no band kernel for %d rows, prefetch %d", bt.rows, bt.prefetch);
 }

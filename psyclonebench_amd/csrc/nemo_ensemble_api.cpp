@@ -271,10 +271,15 @@ long tiles_of(const EnsContext &C, int rows)
     return n;
 }
 
+bool runs_band(const EnsContext &C, const EnsShape &sh)
+{
+    return ens_band(sh, C.prec, C.row_tab != nullptr, C.one_row_tiles);
+}
+
 // Rows and columns of the tile list of a shape.
 std::pair<int, int> list_key(const EnsContext &C, const EnsShape &sh)
 {
-    if (!ens_band(sh)) return {sh.rows, sh.cols};
+    if (!runs_band(C, sh)) return {sh.rows, sh.cols};
     const EnsBand bt =
         ens_band_tiles(sh, C.prec, C.row_tab != nullptr, C.one_row_tiles, C.two_row_tiles);
     return {bt.rows, bt.cols};
@@ -420,7 +425,7 @@ void launch_pair(EnsContext &C, int par, int row, hipStream_t s, hipEvent_t e0 =
     const auto &L = C.lists.at(list_key(C, sh));
     const double *tide = C.d_tide + (size_t)row * C.ndom;
     const int prev = C.paired ? par : q;  // the previous step's velocities
-    const bool band = ens_band(sh);
+    const bool band = runs_band(C, sh);
     const EnsBand bt =
         ens_band_tiles(sh, C.prec, C.row_tab != nullptr, C.one_row_tiles, C.two_row_tiles);
     if (e0) NEMO_HIP_CHECK(hipEventRecord(e0, s));

@@ -257,3 +257,31 @@ def test_ensemble_default_tiles_equal_the_persistent_kernel(sizes, metrics, prec
     for d in range(len(models)):
         for n in FIELDS:
             assert_bitwise(out[0][d][n], out[1][d][n], f"domain {d} {n}")
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("metrics, sizes", [
+    ("point", ((181, 300), (301, 590))), ("point", ((181, 300), (301, 640))),
+    ("row", ((601, 500), (301, 960))), ("row", ((601, 500), (301, 1010)))],
+    ids=["point 3866", "point 4116", "row 9830", "row 10080"])
+def test_ensemble_shapes_on_both_sides_of_their_lines(metrics, sizes, precision):
+    """Shapes of 4 and 8 rows, one wavefront a tile, run band tiles or
+    overlapped-wavefront tiles by the number of one-row tiles (the ids; lines at
+    4000 and 10000): the bits of the persistent kernel on either side."""
+    print("shapes", metrics, sizes, precision, flush=True)
+    models = [band_model(nx, ny, metrics, seed=40 + k) for k, (nx, ny) in enumerate(sizes)]
+    probe = EnsembleStepper(models[:1], precision=precision)
+    shapes = [k for k, s in enumerate(probe.shapes()) if s[2] == 0 and s[0] in (4, 8)]
+    probe.release()
+    assert len(shapes) == 18
+    ref = None
+    for k in [None] + shapes:
+        ens = EnsembleStepper(models, precision=precision)
+        ens.set_shape([s[2] > 0 for s in ens.shapes()].index(True) if k is None else k)
+        ens.run(3)
+        out = [{n: ens.fetch(d, n) for n in FIELDS} for d in range(len(models))]
+        ens.release()
+        ref = ref or out
+        for d in range(len(models)):
+            for n in FIELDS:
+                assert_bitwise(out[d][n], ref[d][n], f"shape {k} domain {d} {n}")
