@@ -299,11 +299,21 @@ void launch_band_f64(hipStream_t s, const StepIn<double> &f, const double *tab,
     }
 }
 
-bool band_f32_shape(int rows, int cols, int prefetch)
+// FP32 shapes asked for by rows and prefetch: time of 20 steps with the
+// overlapped-wavefront tile over that with the band tile. 4 rows: by row 1.06
+// .. 2.2, by point 0.98 .. 1.13 (100 x 3000 0.95). 8 rows by row: 1.07 .. 1.95
+// without prefetch; with it 0.93 .. 1.03 up to 640^2 (7062 tiles of one row),
+// 1.00 .. 1.9 from 768^2 (10010). 8 rows by point: without prefetch 1.00 .. 1.10
+// up to 300 x 250 (1260), 0.89 .. 1.03 above; with it 0.66 .. 0.98.
+constexpr long kBandByRowTilesF32 = 10000, kBandByPointTilesF32 = 1500;
+
+bool band_f32_shape(int rows, int cols, int prefetch, bool by_row, const Bounds &b)
 {
-    return band_f32_auto(rows, cols, prefetch) ||
-           ((rows == 4 || rows == 8) && (cols == 61 || cols == 56) && prefetch >= 0 &&
-            prefetch <= 2);
+    if (band_f32_auto(rows, cols, prefetch)) return true;
+    if ((rows != 4 && rows != 8) || (cols != 61 && cols != 56)) return false;
+    if (rows == 4) return true;
+    if (by_row) return prefetch == 0 || tiles(b, 1, 61) > kBandByRowTilesF32;
+    return prefetch == 0 && tiles(b, 1, 61) <= kBandByPointTilesF32;
 }
 
 void launch_band_f32(hipStream_t s, int rows, int cols, int prefetch, const MixedIn &f,
@@ -333,24 +343,31 @@ void launch_band_f32(hipStream_t s, int rows, int cols, int prefetch, const Mixe
         rows = 4;
         prefetch = tab ? 2 : 0;
     }
-#define NEMO_BAND_F32(R, OW, PF)                                                     \
-    if (rows == R && cols == OW && prefetch == PF) {                                 \
-        tab ? launch<float, true, R, OW, PF, true, false>(a)                         \
-            : launch<float, false, R, OW, PF, true, false>(a);                       \
+#define NEMO_BAND_F32(R, OW, PF, BY_ROW)                                             \
+    if (rows == R && cols == OW && prefetch == PF && (tab != nullptr) == BY_ROW) {   \
+        launch<float, BY_ROW, R, OW, PF, true, false>(a);                            \
         return;                                                                      \
     }
-    NEMO_BAND_F32(4, 61, 0)
-    NEMO_BAND_F32(4, 61, 1)
-    NEMO_BAND_F32(4, 61, 2)
-    NEMO_BAND_F32(4, 56, 0)
-    NEMO_BAND_F32(4, 56, 1)
-    NEMO_BAND_F32(4, 56, 2)
-    NEMO_BAND_F32(8, 61, 0)
-    NEMO_BAND_F32(8, 61, 1)
-    NEMO_BAND_F32(8, 61, 2)
-    NEMO_BAND_F32(8, 56, 0)
-    NEMO_BAND_F32(8, 56, 1)
-    NEMO_BAND_F32(8, 56, 2)
+    NEMO_BAND_F32(4, 61, 0, true)
+    NEMO_BAND_F32(4, 61, 0, false)
+    NEMO_BAND_F32(4, 61, 1, true)
+    NEMO_BAND_F32(4, 61, 1, false)
+    NEMO_BAND_F32(4, 61, 2, true)
+    NEMO_BAND_F32(4, 61, 2, false)
+    NEMO_BAND_F32(4, 56, 0, true)
+    NEMO_BAND_F32(4, 56, 0, false)
+    NEMO_BAND_F32(4, 56, 1, true)
+    NEMO_BAND_F32(4, 56, 1, false)
+    NEMO_BAND_F32(4, 56, 2, true)
+    NEMO_BAND_F32(4, 56, 2, false)
+    NEMO_BAND_F32(8, 61, 0, true)
+    NEMO_BAND_F32(8, 61, 0, false)
+    NEMO_BAND_F32(8, 61, 1, true)
+    NEMO_BAND_F32(8, 61, 2, true)
+    NEMO_BAND_F32(8, 56, 0, true)
+    NEMO_BAND_F32(8, 56, 0, false)
+    NEMO_BAND_F32(8, 56, 1, true)
+    NEMO_BAND_F32(8, 56, 2, true)
 #undef NEMO_BAND_F32
     NEMO_FATAL("mixed step: no band kernel for %d rows x %d columns, prefetch %d", rows, cols,
                prefetch);

@@ -43,16 +43,16 @@ struct MixedOut {
 void launch_mixed_step(hipStream_t s, int rows, int cols, int prefetch, const MixedIn &f,
                        const StepScalars<float> &p, const MixedOut &o, int W,
                        Bounds b, const double *tide_tab, int tide_k, double tide_val);
-// The band form (nemo_band.hip): the shapes it has (the others run
-// launch_mixed_step), and one step with its Flather faces. The default shape
-// of a handle (32 rows, 61 columns, no prefetch) stands for the library's
-// choice by grid size. tab: the row table (launch_row_metrics) or null; cu /
+// The band form (nemo_band.hip): whether a shape runs it on a grid with or
+// without metrics by row (the others run launch_mixed_step), and one step with
+// its Flather faces. The default shape of a handle (32 rows, 61 columns, no
+// prefetch) stands for the library's choice by grid size. tab: the row table (launch_row_metrics) or null; cu /
 // cv: sqrt(g / h) at the Flather faces, as arrays (null: no Flather face).
 constexpr bool band_f32_auto(int rows, int cols, int prefetch)
 {
     return rows == 32 && cols == 61 && prefetch == 0;
 }
-bool band_f32_shape(int rows, int cols, int prefetch);
+bool band_f32_shape(int rows, int cols, int prefetch, bool by_row, const Bounds &b);
 void launch_row_metrics(hipStream_t s, const MixedIn &f, int W, unsigned base, const Bounds &b,
                         float *tab, int *bad, int mark);
 void launch_band_f32(hipStream_t s, int rows, int cols, int prefetch, const MixedIn &f,

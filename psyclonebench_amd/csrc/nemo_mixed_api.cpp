@@ -116,7 +116,7 @@ void launch_pair(MixedContext &C, int par, hipStream_t s, const double *tide_tab
     const MixedOut o{C.t_hi[q], C.t_lo[q], C.u[q], C.v[q], C.su[q], C.sv[q]};
     const Bounds b{C.G.xs, C.G.xe, C.G.ys, C.G.ye};
     const int prev = C.paired ? par : q;  // the previous step's velocities
-    const bool band = band_f32_shape(C.rows, C.cols, C.prefetch);
+    const bool band = band_f32_shape(C.rows, C.cols, C.prefetch, C.row_tab != nullptr, b);
     if (e0) NEMO_HIP_CHECK(hipEventRecord(e0, s));
     if (band)
         launch_band_f32(s, C.rows, C.cols, C.prefetch, C.inputs(par), C.row_tab, C.scalars(), o,

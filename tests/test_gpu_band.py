@@ -194,3 +194,23 @@ def test_numerators_outside_the_quick_range_in_one_row_tiles():
     st = TimeStepper(m.copy(), mode=2)
     st.run(3)
     check(st, ref, "falling state")
+
+
+@pytest.mark.parametrize("metrics, nx, ny", [("point", 181, 496), ("point", 181, 502),
+                                             ("row", 605, 996), ("row", 605, 1000)])
+def test_mixed_shapes_on_both_sides_of_their_lines(metrics, nx, ny):
+    """FP32 shapes of 8 rows run band tiles or overlapped-wavefront tiles by the
+    number of one-row tiles (lines at 1500 by point, 10000 by row): the bits of
+    the 48-column kernel on either side."""
+    print("mixed lines", metrics, nx, ny, flush=True)
+    m = live_model(nx, ny, metrics, seed=13)
+    ref = None
+    for rows, cols, pf in ((16, 48, 0), (8, 61, 0), (8, 61, 1), (8, 61, 2), (8, 56, 0),
+                           (8, 56, 1), (8, 56, 2)):
+        st = MixedStepper(m, rows=rows, cols=cols, prefetch=pf)
+        st.run(4)
+        out = {n: st.fetch(n) for n in ("sshn_t", "un", "vn", "sshn_u", "sshn_v")}
+        st.release()
+        ref = ref or out
+        for n in out:
+            assert_bitwise(out[n], ref[n], f"{nx}x{ny} {metrics} {rows}x{cols} p{pf} {n}")
