@@ -110,6 +110,14 @@ __global__ void k_split_f64(const double *__restrict__ src, float *__restrict__ 
     lo[k] = (float)(s - (double)h);
 }
 
+// Shapes that band_f32_shape always sends to the band form: 4 rows of 61 or 56
+// columns, and the default one.
+[[noreturn]] void band_only(int rows, int cols, int prefetch)
+{
+    NEMO_FATAL("mixed step: %d rows x %d columns, prefetch %d, run band tiles only", rows, cols,
+               prefetch);
+}
+
 inline dim3 blocks_for(long n) { return dim3((unsigned)((n + 255) / 256)); }
 
 }  // namespace
@@ -127,15 +135,19 @@ void launch_mixed_step(hipStream_t s, int rows, int cols, int prefetch, const Mi
 #define NEMO_MIXED_PF_CASE(RR, PF)                                                   \
     case RR * 4 + PF: {                                                              \
         const dim3 grid((unsigned)(nstrip * ((nrow + RR - 1) / RR)));                \
-        if (cols == 48)                                                              \
+        if (cols == 48) {                                                            \
             k_mixed_wave_p<RR, 48, PF><<<grid, dim3(64), 0, s>>>(                    \
                 f, p, o, W, b, nstrip, tide_tab, tide_k, tide_val);                  \
-        else if (cols == 56)                                                         \
-            k_mixed_wave_p<RR, 56, PF><<<grid, dim3(64), 0, s>>>(                    \
-                f, p, o, W, b, nstrip, tide_tab, tide_k, tide_val);                  \
-        else                                                                         \
-            k_mixed_wave_p<RR, wave::OUT, PF><<<grid, dim3(64), 0, s>>>(             \
-                f, p, o, W, b, nstrip, tide_tab, tide_k, tide_val);                  \
+        } else if constexpr (RR == 8) { /* 4 rows: band tiles */                     \
+            if (cols == 56)                                                          \
+                k_mixed_wave_p<RR, 56, PF><<<grid, dim3(64), 0, s>>>(                \
+                    f, p, o, W, b, nstrip, tide_tab, tide_k, tide_val);              \
+            else                                                                     \
+                k_mixed_wave_p<RR, wave::OUT, PF><<<grid, dim3(64), 0, s>>>(         \
+                    f, p, o, W, b, nstrip, tide_tab, tide_k, tide_val);              \
+        } else {                                                                     \
+            band_only(rows, cols, prefetch);                                         \
+        }                                                                            \
         break;                                                                       \
     }
             NEMO_MIXED_PF_CASE(4, 1)
@@ -154,15 +166,21 @@ void launch_mixed_step(hipStream_t s, int rows, int cols, int prefetch, const Mi
 #define NEMO_MIXED_CASE(RR)                                                          \
     case RR: {                                                                       \
         const dim3 grid((unsigned)(nstrip * ((nrow + RR - 1) / RR)));                \
-        if (cols == 48)                                                              \
+        if (cols == 48) {                                                            \
             k_mixed_wave_a<RR, 48><<<grid, dim3(64), 0, s>>>(                        \
                 f, p, o, W, b, nstrip, tide_tab, tide_k, tide_val);                  \
-        else if (cols == 56)                                                         \
-            k_mixed_wave_a<RR, 56><<<grid, dim3(64), 0, s>>>(                        \
-                f, p, o, W, b, nstrip, tide_tab, tide_k, tide_val);                  \
-        else                                                                         \
+        } else if (cols == 56) {                                                     \
+            if constexpr (RR != 4)                                                   \
+                k_mixed_wave_a<RR, 56><<<grid, dim3(64), 0, s>>>(                    \
+                    f, p, o, W, b, nstrip, tide_tab, tide_k, tide_val);              \
+            else                                                                     \
+                band_only(rows, cols, prefetch);                                     \
+        } else if constexpr (RR != 4 && RR != 32) {                                  \
             k_mixed_wave<RR><<<grid, dim3(64), 0, s>>>(f, p, o, W, b, nstrip,        \
                                                        tide_tab, tide_k, tide_val);   \
+        } else {                                                                     \
+            band_only(rows, cols, prefetch);                                         \
+        }                                                                            \
         break;                                                                       \
     }
         NEMO_MIXED_CASE(4)
