@@ -331,7 +331,7 @@ def ensemble_leg(a) -> dict:
             "shape": {"rows": shape[0], "columns": shape[3], "prefetch": shape[4],
                       "launch": "persistent" if shape[2] else "one wavefront per tile",
                       "waves_per_workgroup": shape[1], "workgroups": shape[2] or None},
-            "autotune_kernel_ms": [round(x, 4) for x in tune_ms],
+            "autotune_step_ms": [round(x, 4) for x in tune_ms],
             "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS,
                          "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                          "traffic": (traffic_from_profile(

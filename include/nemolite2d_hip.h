@@ -266,8 +266,8 @@ NEMO_API int nemo_ens_shape_prefetch(void *handle, int shape);
 NEMO_API void nemo_ens_set_shape(void *handle, int shape);
 NEMO_API int nemo_ens_shape(void *handle);
 /* Times every shape on steps_per_shape steps of this ensemble (HIP events
- * around each step kernel; mean ms per shape into ms_out if not NULL),
- * restores the state, selects and returns the fastest shape. */
+ * around a graph replay of whole steps; mean ms per step into ms_out if not
+ * NULL), restores the state, selects and returns the fastest shape. */
 NEMO_API int nemo_ens_autotune(void *handle, int steps_per_shape, double *ms_out);
 /* nsteps steps istep, istep+1, ... (one hipGraph replay; asynchronous). */
 NEMO_API void nemo_ens_steps(void *handle, int nsteps, int istep);

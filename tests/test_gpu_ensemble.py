@@ -285,3 +285,21 @@ def test_ensemble_shapes_on_both_sides_of_their_lines(metrics, sizes, precision)
         for d in range(len(models)):
             for n in FIELDS:
                 assert_bitwise(out[d][n], ref[d][n], f"shape {k} domain {d} {n}")
+
+
+def test_autotune_times_whole_steps():
+    """A shape with a Flather launch of its own is compared with the band tiles,
+    which need none, by the whole step: its time is that of the step kernel and
+    of at least the shortest launch (over 1 us; the median of several tries)."""
+    models = [band_model(64, 64, "row", seed=50 + k) for k in range(3)]
+    ens = EnsembleStepper(models)
+    shapes = ens.shapes()
+    k = [s[:1] + s[2:] for s in shapes].index((16, 0, 61, 0))
+    extra = []
+    for _ in range(7):
+        _, ms = ens.autotune(50)
+        ens.set_shape(k)
+        extra.append((ms[k] - ens.timed_run(50)) * 1e3)
+    ens.release()
+    print("whole step less its kernel, us:", [round(x, 2) for x in extra], flush=True)
+    assert sorted(extra)[3] > 1.0
