@@ -5,7 +5,8 @@
 // new), a tenth of the link. The FP32 values come into pinned memory chunk by
 // chunk, half the bytes of the FP64 ones, and several threads widen a chunk
 // while the next ones arrive. The threads live for one call and touch memory
-// only; the stage belongs to the handle.
+// only; they poll for a chunk while it may come within the next microseconds
+// and sleep while steps before it still run. The stage belongs to the handle.
 //
 // us a field, pageable copy and one loop / staged, one thread / staged, team:
 // 82 k values 31 / 32 / 34; 0.3 M 125 / 100 / 83; 1.2 M 507 / 379 / 317: a
@@ -14,6 +15,8 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
+#include <condition_variable>
 #include <exception>
 #include <mutex>
 #include <thread>
@@ -60,10 +63,10 @@ public:
             NEMO_HIP_CHECK(hipEventRecord(ready_[c % kSlots], s));
         };
         // thread t of `threads` widens its part of every chunk
-        std::atomic<size_t> arrived{0};
-        std::atomic<int> threads{0};  // 0: not yet known
+        Arrivals arrived;
+        int nt = 1;  // known before the first arrival
         Done done[kMaxThreads];
-        auto part = [&](size_t c, int t, int nt) {
+        auto part = [&](size_t c, int t) {
             const size_t m = count(c), a = m * t / nt, b = m * (t + 1) / nt;
             const float *const d = stage_ + c % kSlots * 2 * kChunk;
             double *const o = out + c * kChunk;
@@ -74,11 +77,9 @@ public:
             done[t].chunks.store(c + 1, std::memory_order_release);
         };
         auto helper = [&](int t) {
-            int nt;
-            while ((nt = threads.load(std::memory_order_acquire)) == 0) std::this_thread::yield();
             for (size_t c = 0; c < chunks; c++) {
-                while (arrived.load(std::memory_order_acquire) <= c) std::this_thread::yield();
-                part(c, t, nt);
+                arrived.wait(c);
+                part(c, t);
             }
         };
         for (size_t c = 0; c < std::min(chunks, kSlots); c++) queue(c);
@@ -91,12 +92,11 @@ public:
             while (team.size() + 1 < want) team.emplace_back(helper, (int)team.size() + 1);
         } catch (const std::exception &) {  // no more threads: fewer will do
         }
-        const int nt = (int)team.size() + 1;
-        threads.store(nt, std::memory_order_release);
+        nt = (int)team.size() + 1;
         for (size_t c = 0; c < chunks; c++) {
             NEMO_HIP_CHECK(hipEventSynchronize(ready_[c % kSlots]));
-            arrived.store(c + 1, std::memory_order_release);
-            part(c, 0, nt);
+            arrived.add();
+            part(c, 0);
             if (c + kSlots >= chunks) continue;
             for (int t = 1; t < nt; t++)  // the slot is free when every part is out
                 while (done[t].chunks.load(std::memory_order_acquire) <= c)
@@ -110,8 +110,37 @@ private:
     static constexpr size_t kChunk = 1 << 18, kSlots = 3;  // 2 MB, with lo
     static constexpr size_t kPerThread = 1 << 17;
     static constexpr int kMaxThreads = 8;
+    static constexpr std::chrono::microseconds kPoll{200};  // ten chunks' time on the link
     struct alignas(64) Done {
         std::atomic<size_t> chunks{0};
+    };
+    // Chunks that have arrived.
+    class Arrivals {
+    public:
+        void add()
+        {
+            {
+                const std::lock_guard<std::mutex> hold(mutex_);
+                count_.store(count_.load(std::memory_order_relaxed) + 1,
+                             std::memory_order_release);
+            }
+            more_.notify_all();
+        }
+        void wait(size_t c)  // until chunk c is there
+        {
+            auto there = [&] { return count_.load(std::memory_order_acquire) > c; };
+            const auto until = std::chrono::steady_clock::now() + kPoll;
+            while (!there() && std::chrono::steady_clock::now() < until)
+                std::this_thread::yield();
+            if (there()) return;
+            std::unique_lock<std::mutex> hold(mutex_);
+            more_.wait(hold, there);
+        }
+
+    private:
+        std::mutex mutex_;
+        std::condition_variable more_;
+        std::atomic<size_t> count_{0};
     };
     std::mutex mutex_;
     float *stage_ = nullptr;

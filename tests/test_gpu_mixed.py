@@ -209,3 +209,23 @@ def test_threads_read_one_handle_at_the_same_time():
         for n, got in zip(names * 5, pool.map(st.fetch, names * 5)):
             assert_bitwise(got, ref[n], n)
     st.release()
+
+
+def test_a_read_behind_queued_steps_leaves_the_processors_alone():
+    """A record read right after steps were queued waits for them; its helper
+    threads sleep meanwhile. They used to turn idle loops, eight processors'
+    worth: the process may spend at most twice the waiting time (the waiting
+    thread itself may poll)."""
+    import time
+    st = MixedStepper(Model(replace(c1_config(4), jpiglo=2050, jpjglo=2050)))
+    ref = [st.run(1500), st.fetch("un")][1]   # the graph and the stage exist now
+    st.run(1500)
+    wall, cpu = time.perf_counter(), time.process_time()
+    got = st.fetch("un")
+    wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
+    st.release()
+    print(f"read behind queued steps: {wall * 1e3:.1f} ms, processor {cpu * 1e3:.1f} ms",
+          flush=True)
+    assert wall > 0.03, "the steps were over before the read"
+    assert got.shape == ref.shape
+    assert cpu < 2.0 * wall
