@@ -9,8 +9,13 @@
 // and sleep while steps before it still run. The stage belongs to the handle.
 //
 // us a field, pageable copy and one loop / staged, one thread / staged, team:
-// 82 k values 31 / 32 / 34; 0.3 M 125 / 100 / 83; 1.2 M 507 / 379 / 317: a
-// thread for every 128 k values.
+//   ssh         25 k values 32 / 30 / -;  81 k 62 / 52 / -;  0.18 M 118 / - / 84;
+//               1.2 M 790 / - / 370
+//   velocities  25 k 17 / 18 / -;  81 k 32 / 34 / -;  0.18 M 60 / - / 58;  1.2 M
+//               430 / - / 240
+// so a thread for every 128 k values, and below that the pageable copy for a
+// field of one word. A single chunk waits for the stream: an event costs 8 us
+// more (25 k values of ssh 40, of u 28).
 #pragma once
 
 #include <algorithm>
@@ -43,6 +48,13 @@ public:
     void read(hipStream_t s, const float *hi, const float *lo, size_t n, double *out)
     {
         if (n == 0) return;
+        if (!lo && n <= kOneThread) {
+            std::vector<float> a(n);
+            NEMO_HIP_CHECK(hipStreamSynchronize(s));
+            NEMO_HIP_CHECK(hipMemcpy(a.data(), hi, n * sizeof(float), hipMemcpyDeviceToHost));
+            for (size_t k = 0; k < n; k++) out[k] = (double)a[k];
+            return;
+        }
         // threads may read one handle at the same time; they share the stage
         const std::lock_guard<std::mutex> one(mutex_);
         if (!stage_) {
@@ -53,13 +65,16 @@ public:
         }
         const size_t chunks = (n + kChunk - 1) / kChunk;
         auto count = [&](size_t c) { return std::min(kChunk, n - c * kChunk); };
-        auto queue = [&](size_t c) {
+        auto copy = [&](size_t c) {
             float *const d = stage_ + c % kSlots * 2 * kChunk;
             const size_t bytes = count(c) * sizeof(float);
             NEMO_HIP_CHECK(hipMemcpyAsync(d, hi + c * kChunk, bytes, hipMemcpyDeviceToHost, s));
             if (lo)
                 NEMO_HIP_CHECK(hipMemcpyAsync(d + kChunk, lo + c * kChunk, bytes,
                                               hipMemcpyDeviceToHost, s));
+        };
+        auto queue = [&](size_t c) {
+            copy(c);
             NEMO_HIP_CHECK(hipEventRecord(ready_[c % kSlots], s));
         };
         // thread t of `threads` widens its part of every chunk
@@ -82,6 +97,12 @@ public:
                 part(c, t);
             }
         };
+        if (n <= kOneThread) {  // no event, no team
+            copy(0);
+            NEMO_HIP_CHECK(hipStreamSynchronize(s));
+            part(0, 0);
+            return;
+        }
         for (size_t c = 0; c < std::min(chunks, kSlots); c++) queue(c);
         // a thread for every kPerThread values, as far as there are processors
         const size_t want = std::min({(size_t)kMaxThreads, n / kPerThread + 1,
@@ -108,7 +129,8 @@ public:
 
 private:
     static constexpr size_t kChunk = 1 << 18, kSlots = 3;  // 2 MB, with lo
-    static constexpr size_t kPerThread = 1 << 17;
+    static constexpr size_t kPerThread = 1 << 17, kOneThread = kPerThread - 1;
+    static_assert(kOneThread <= kChunk, "one chunk");
     static constexpr int kMaxThreads = 8;
     static constexpr std::chrono::microseconds kPoll{200};  // ten chunks' time on the link
     struct alignas(64) Done {

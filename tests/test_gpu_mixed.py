@@ -229,3 +229,10 @@ def test_a_read_behind_queued_steps_leaves_the_processors_alone():
     assert wall > 0.03, "the steps were over before the read"
     assert got.shape == ref.shape
     assert cpu < 2.0 * wall
+
+
+@pytest.mark.parametrize("nx, ny", [(61, 40), (509, 252), (509, 253), (509, 254)])
+def test_read_back_around_the_smallest_team(nx, ny):
+    """Fields of 2^17 values (509 x 253), a row less and more: below, one thread
+    reads them, the velocities without the stage."""
+    test_read_back_of_the_uploaded_state(nx, ny)
