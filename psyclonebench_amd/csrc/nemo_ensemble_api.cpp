@@ -343,17 +343,10 @@ void build_flather_lists(EnsContext &C, void *const *arrays, hipStream_t s)
     C.fl_v.upload(V, s);
     if (C.prec == 64 || (U.idx.empty() && V.idx.empty())) return;
     // the factors as arenas, read at the Flather faces only
-    std::vector<float> c(C.total);
-    for (int dir = 0; dir < 2; dir++) {
-        const HostFlather &L = dir ? V : U;
-        std::fill(c.begin(), c.end(), 0.0f);
-        for (size_t k = 0; k < L.idx.size(); k++) c[(size_t)L.idx[k]] = (float)L.coef[k];
-        float *&dst = dir ? C.cv : C.cu;
-        dst = static_cast<float *>(arena(C, sizeof(float), s));
-        NEMO_HIP_CHECK(hipMemcpyAsync(dst, c.data(), C.total * sizeof(float),
-                                      hipMemcpyHostToDevice, s));
-        NEMO_HIP_CHECK(hipStreamSynchronize(s));  // c is reused
-    }
+    C.cu = static_cast<float *>(arena(C, 2 * sizeof(float), s));
+    C.cv = C.cu + C.total;
+    launch_flather_factors(s, C.fl_u.view(), (int)U.idx.size(), C.cu);
+    launch_flather_factors(s, C.fl_v.view(), (int)V.idx.size(), C.cv);
 }
 
 // The tables of metrics by row of every domain; dropped when one domain has
@@ -369,18 +362,18 @@ void build_row_tables(EnsContext &C, const In &in, hipStream_t s)
         values += row_table_values(Bounds{e.xs, e.xe, e.ys, e.ye});
     }
     if (sizeof(T) == 8 && !table_divisor(C.fric())) return;
-    T *const tab = dev_alloc<T>(values);
+    T *const tab = dev_alloc<T>(values + 1);  // and the mark of metrics that vary
     C.row_tab = tab;
-    int *bad = dev_alloc<int>(1), host_bad = 0;
-    NEMO_HIP_CHECK(hipMemcpy(bad, &host_bad, sizeof(int), hipMemcpyHostToDevice));
+    int *const bad = reinterpret_cast<int *>(tab + values);
+    int host_bad = 0;
+    launch_fill_int(s, bad, 1, 0);
     for (int d = 0; d < C.ndom; d++) {
         const EnsDomain &e = C.hdom[d];
         launch_row_metrics(s, in, e.W, e.off, Bounds{e.xs, e.xe, e.ys, e.ye},
                            tab + (size_t)C.rec[d] * kRowTableWidth, bad, 1);
     }
+    NEMO_HIP_CHECK(hipMemcpyAsync(&host_bad, bad, sizeof(int), hipMemcpyDeviceToHost, s));
     NEMO_HIP_CHECK(hipStreamSynchronize(s));
-    NEMO_HIP_CHECK(hipMemcpy(&host_bad, bad, sizeof(int), hipMemcpyDeviceToHost));
-    NEMO_HIP_CHECK(hipFree(bad));
     if (host_bad) {
         NEMO_HIP_CHECK(hipFree(C.row_tab));
         C.row_tab = nullptr;

@@ -64,6 +64,9 @@ void launch_band_f32(hipStream_t s, int rows, int cols, int prefetch, const Mixe
 void launch_flather_f32(hipStream_t s, const FlatherList &lu, const FlatherList &lv,
                         float *ua, float *va, const float *ua_prev, const float *va_prev,
                         const float *su, const float *sv);
+// factor[idx[k]] = coef[k] for the n faces of a list, the other elements as
+// they are
+void launch_flather_factors(hipStream_t s, const FlatherList &list, int n, float *factor);
 void launch_to_f32(hipStream_t s, const double *src, float *dst, long n);
 void launch_split_f64(hipStream_t s, const double *src, float *hi, float *lo, long n);
 

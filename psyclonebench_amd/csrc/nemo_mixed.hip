@@ -92,6 +92,13 @@ __global__ __launch_bounds__(64) void k_flather_f32(FlatherList lu, FlatherList 
     }
 }
 
+__global__ void k_flather_factors(const int *__restrict__ idx, const double *__restrict__ coef,
+                                  int n, float *__restrict__ factor)
+{
+    const int k = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (k < n) factor[idx[k]] = (float)coef[k];
+}
+
 __global__ void k_to_f32(const double *__restrict__ src, float *__restrict__ dst,
                          long n)
 {
@@ -206,6 +213,13 @@ void launch_flather_f32(hipStream_t s, const FlatherList &lu, const FlatherList 
     if (n == 0) return;
     k_flather_f32<<<dim3((unsigned)((n + 63) / 64)), dim3(64), 0, s>>>(
         lu, lv, ua, va, ua_prev, va_prev, su, sv);
+    NEMO_LAUNCH_CHECK();
+}
+
+void launch_flather_factors(hipStream_t s, const FlatherList &list, int n, float *factor)
+{
+    if (n == 0) return;
+    k_flather_factors<<<blocks_for(n), dim3(256), 0, s>>>(list.idx, list.coef, n, factor);
     NEMO_LAUNCH_CHECK();
 }
 

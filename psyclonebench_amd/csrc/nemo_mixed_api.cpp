@@ -29,7 +29,8 @@ struct MixedContext {
     signed char *tm = nullptr;       // T mask, one byte a point
     float *fcor_u = nullptr, *fcor_v = nullptr;
     // band form: the table of metrics by row (null: they vary along a row) and
-    // the Flather factors at their faces (null: no Flather face)
+    // the Flather factors at their faces (null: no Flather face; cv is the
+    // second half of cu)
     float *row_tab = nullptr, *cu = nullptr, *cv = nullptr;
     float *t_hi[2] = {}, *t_lo[2] = {}, *u[2] = {}, *v[2] = {}, *su[2] = {}, *sv[2] = {};
     DeviceFlather fl_u, fl_v;
@@ -87,7 +88,7 @@ struct MixedContext {
         for (hipEvent_t e : ev) (void)hipEventDestroy(e);
         for (float *p : cst)
             if (p) (void)hipFree(p);
-        float *more[] = {fcor_u, fcor_v, row_tab, cu, cv, t_hi[0], t_hi[1], t_lo[0], t_lo[1], u[0], u[1],
+        float *more[] = {fcor_u, fcor_v, row_tab, cu, t_hi[0], t_hi[1], t_lo[0], t_lo[1], u[0], u[1],
                          v[0], v[1], su[0], su[1], sv[0], sv[1]};
         for (float *p : more)
             if (p) (void)hipFree(p);
@@ -137,23 +138,21 @@ void prepare_band(MixedContext &C, const HostFlather &u, const HostFlather &v, h
 {
     const size_t n = (size_t)C.G.total;
     if (!u.idx.empty() || !v.idx.empty()) {
-        std::vector<float> c(n, 0.0f);
-        for (size_t k = 0; k < u.idx.size(); k++) c[u.idx[k]] = (float)u.coef[k];
-        C.cu = dev_alloc<float>(n);
-        NEMO_HIP_CHECK(hipMemcpy(C.cu, c.data(), n * sizeof(float), hipMemcpyHostToDevice));
-        std::fill(c.begin(), c.end(), 0.0f);
-        for (size_t k = 0; k < v.idx.size(); k++) c[v.idx[k]] = (float)v.coef[k];
-        C.cv = dev_alloc<float>(n);
-        NEMO_HIP_CHECK(hipMemcpy(C.cv, c.data(), n * sizeof(float), hipMemcpyHostToDevice));
+        C.cu = dev_alloc<float>(2 * n);
+        C.cv = C.cu + n;
+        NEMO_HIP_CHECK(hipMemsetAsync(C.cu, 0, 2 * n * sizeof(float), s));
+        launch_flather_factors(s, C.fl_u.view(), (int)u.idx.size(), C.cu);
+        launch_flather_factors(s, C.fl_v.view(), (int)v.idx.size(), C.cv);
     }
     const Bounds b{C.G.xs, C.G.xe, C.G.ys, C.G.ye};
-    C.row_tab = dev_alloc<float>(row_table_values(b));
-    int *bad = dev_alloc<int>(1), host_bad = 0;
-    NEMO_HIP_CHECK(hipMemcpy(bad, &host_bad, sizeof(int), hipMemcpyHostToDevice));
+    const size_t values = row_table_values(b);
+    C.row_tab = dev_alloc<float>(values + 1);  // and the mark of metrics that vary
+    int *const bad = reinterpret_cast<int *>(C.row_tab + values);
+    int host_bad = 0;
+    launch_fill_int(s, bad, 1, 0);
     launch_row_metrics(s, C.inputs(0), C.G.W, 0u, b, C.row_tab, bad, 1);
+    NEMO_HIP_CHECK(hipMemcpyAsync(&host_bad, bad, sizeof(int), hipMemcpyDeviceToHost, s));
     NEMO_HIP_CHECK(hipStreamSynchronize(s));
-    NEMO_HIP_CHECK(hipMemcpy(&host_bad, bad, sizeof(int), hipMemcpyDeviceToHost));
-    NEMO_HIP_CHECK(hipFree(bad));
     if (host_bad) {
         NEMO_HIP_CHECK(hipFree(C.row_tab));
         C.row_tab = nullptr;
