@@ -168,9 +168,10 @@ NEMO_API double nemo_hip_fused_kernel_ms(void);
  * width x rows per band). All shapes compute bitwise the same result;
  * default 31, the band form: it evaluates every face once, has the Flather
  * faces in the same launch, picks the band height by the size of the grid
- * and, in calls of two or more steps on a grid whose metrics do not vary
- * along a row, reads them as one record a row (checked on the device arrays
- * in every such call).
+ * and, on a grid whose metrics do not vary along a row, reads them as one
+ * record a row in calls of two or more steps and at least 2 million points in
+ * all (interior points times steps; checked on the device arrays in every
+ * such call).
  * Applies to the next launches of every context. */
 NEMO_API int nemo_hip_fused_variant_count(void);
 NEMO_API void nemo_hip_set_fused_variant(int variant);
@@ -212,7 +213,8 @@ NEMO_API void nemo_mp_steps(void *handle, int nsteps, int istep);
 NEMO_API double nemo_mp_kernel_ms(void *handle, int nsteps, int istep);
 /* Rows per band of the kernel: 4, 8, 16, 32 (default), 48, 64, 80, 96 or
  * 128. With the other settings at their defaults, 32 leaves the band height
- * to the library, which picks it by the size of the grid. */
+ * to the library, which picks it by the size of the grid. 4 and 8 rows of 61 or
+ * 56 columns run whichever of the library's two tiles is the faster. */
 NEMO_API void nemo_mp_set_rows(void *handle, int rows);
 /* Output columns per wavefront: 61 (default; strips overlap by 3 columns),
  * 56 (every strip's stores start on a 32-byte boundary) or 48 (on a 64-byte
@@ -230,8 +232,9 @@ NEMO_API void nemo_mp_destroy(void *handle);
 /* ---- batched ensemble (no reference counterpart) -----------------------
  * ndom independent domains, each in its own dl_esm_inf layout, advanced
  * together: one launch per step walks a tile -> domain work list (one
- * wavefront per tile, or a persistent grid), then one launch runs every
- * domain's Flather segments.
+ * wavefront per tile, or a persistent grid). The default shape writes the
+ * Flather faces in that launch; a shape whose tiles do not is followed by one
+ * launch over every domain's Flather segments.
  *   arrays      ndom x 25 host pointers, each row in the c_invoke_time_step
  *               argument order (tmask as int*); read during creation only
  *   geom        ndom x 6 ints: xs, xe, ys, ye (0-based internal bounds),

@@ -101,8 +101,8 @@ __device__ __forceinline__ float high(Ssh s) { return s.hi; }
 __device__ __forceinline__ const double *ssh_of(const StepIn<double> &f) { return f.sshn_t; }
 __device__ __forceinline__ const float *ssh_of(const MixedIn &f) { return f.ssh_hi; }
 
-// What the Flather part reads besides the step's inputs. on: 0 leaves the
-// Flather faces to a separate launch. u_prev / v_prev: the velocities at the
+// What the Flather part reads besides the step's inputs. on: 0 where the domain
+// has no Flather face. u_prev / v_prev: the velocities at the
 // end of the previous step. cu / cv (FP32): sqrt(g / h) at the faces, rounded
 // from FP64 (null in FP64, where the tile evaluates it).
 template <typename T>

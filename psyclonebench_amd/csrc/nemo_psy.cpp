@@ -361,7 +361,9 @@ void run_steps(Context &C, int nsteps, int istep, hipStream_t s,
     ensure_tide_table(C, nsteps);
     // The table costs a launch, a wait (some 18 us together) and one pass over 13
     // arrays, and saves about 15 us a step per million points: worth it from 2
-    // million points in all (4 steps at 400^2 95 us without, 102 with).
+    // million points in all (4 steps of 204 x 784 97 us without, 102 with; 2 of
+    // 1024^2 161 with, 181 by point). Where the metrics vary the call pays for
+    // the look alone: up to 2.5% of 2 steps of 4 million points.
     bool by_row = false;
     const long points = (long)(C.G.xe - C.G.xs + 1) * (C.G.ye - C.G.ys + 1);
     if (g_fused_variant == kDefaultVariant && nsteps > 1 && points * nsteps >= 2000000)
