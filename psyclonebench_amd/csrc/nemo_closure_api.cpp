@@ -467,11 +467,10 @@ void nemo_cl_last_stats(void *h, double *out)
     NEMO_HIP_CHECK(hipMemcpy(gp.data(), C.guard_partial, gp.size() * sizeof(double),
                              hipMemcpyDeviceToHost));
     const double npx = (double)C.nx * C.ny;
-    for (int c = 0; c < 3; c++) {
-        double s = 0.0;
-        for (int b = 0; b < loss_blocks(C.nx, C.ny); b++) s += p[(size_t)b * 3 + c];
-        out[c] = s / npx;
-    }
+    double sum[3] = {};
+    for (size_t b = 0; b < p.size(); b += 3)
+        for (int c = 0; c < 3; c++) sum[c] += p[b + c];
+    for (int c = 0; c < 3; c++) out[c] = sum[c] / npx;
     out[3] = ns[0];
     for (int r = 0; r < 3; r++) {
         double s = 0.0;
